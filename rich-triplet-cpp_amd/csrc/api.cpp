@@ -105,23 +105,12 @@ int gemv_args(const char* fn, const void* w, const float* x, const float* y, int
     return RT_HIP_OK;
 }
 
-// Runs a GEMV in batches of activation rows that fit the LDS budget.
-template <typename F>
-int gemv_batched(const char* fn, int fmt, const float* x, float* y, int64_t n, int64_t k,
-                 int32_t m, F&& launch) {
+// The longest K of the BF16 and Q4_0 GEMVs: `bytes` of one staged activation
+// row and 4 KB of row sums within one workgroup's LDS.
+int gemv_k_bound(const char* fn, size_t bytes) {
     hipError_t e;
-    DeviceState* st = state_for_current(&e);
-    if (!st) return hip_fail(e, fn);
-    const size_t cap = lds_cap();
-    int mb = m;
-    while (mb > 1 && gemv_lds_bytes(fmt, mb, k) > cap) --mb;
-    if (gemv_lds_bytes(fmt, mb, k) > cap)
-        return fail(RT_HIP_E_SHAPE, std::string(fn) + ": k too large for the LDS-staged GEMV");
-    for (int32_t m0 = 0; m0 < m; m0 += mb) {
-        const int32_t mm = (m - m0) < mb ? (m - m0) : mb;
-        e = launch(x + static_cast<size_t>(m0) * k, y + static_cast<size_t>(m0) * n, mm);
-        if (e != hipSuccess) return hip_fail(e, fn);
-    }
+    if (!state_for_current(&e)) return hip_fail(e, fn);
+    if (bytes + 4096 > lds_cap()) return fail(RT_HIP_E_SHAPE, std::string(fn) + ": k too large for the LDS-staged GEMV");
     return RT_HIP_OK;
 }
 
@@ -292,7 +281,6 @@ int64_t rt_hip_gemm_workspace_bytes(int32_t format, int32_t a_dtype, int64_t m, 
 
 int64_t rt_hip_gemv_workspace_bytes(int32_t format, int64_t n, int64_t k, int32_t m) {
     if (n <= 0 || k <= 0 || m < 1 || m > RT_HIP_GEMV_MAX_M) return -1;
-    if (m == 1 || (format != RT_HIP_Q4K && format != RT_HIP_BF16)) return 0;
     return static_cast<int64_t>(gemv_batch_workspace_bytes(format, n, k, m));
 }
 
@@ -313,24 +301,16 @@ int rt_hip_gemv_q4k(const void* blocks, const float* x, float* y, int64_t n, int
                     int32_t m, rt_hip_stream stream) {
     int rc = gemv_args("rt_hip_gemv_q4k", blocks, x, y, n, k, m, 256);
     if (rc) return rc;
-    if (m > 1 && tune_param("GEMV_BATCH_MFMA", 1))
-        return check_stream_launch(launch_gemv_batch(RT_HIP_Q4K, blocks, x, y, n, k, m, static_cast<hipStream_t>(stream)),
-                                   "rt_hip_gemv_q4k");
-    if (m == 1) {
-        // the int8-MFMA kernel stages 3.5 bytes per value (the VALU kernel's
-        // bound below is 4.25)
-        hipError_t e;
-        if (!state_for_current(&e)) return hip_fail(e, "rt_hip_gemv_q4k");
-        if (q4k_m1_lds_bytes(k) > lds_cap())
-            return fail(RT_HIP_E_SHAPE, "rt_hip_gemv_q4k: k too large for the LDS");
-        return check_stream_launch(launch_gemv_q4k_mfma(blocks, x, y, n, k, static_cast<hipStream_t>(stream)),
-                                   "rt_hip_gemv_q4k");
-    }
-    return gemv_batched("rt_hip_gemv_q4k", RT_HIP_Q4K, x, y, n, k, m,
-                        [&](const float* xx, float* yy, int mm) {
-                            return launch_gemv_q4k(blocks, xx, yy, n, k, mm,
-                                                   static_cast<hipStream_t>(stream));
-                        });
+    // the M = 1 kernel stages 3.5 bytes per value; the batched one stages K in
+    // chunks
+    hipError_t e;
+    if (!state_for_current(&e)) return hip_fail(e, "rt_hip_gemv_q4k");
+    if (m == 1 && q4k_m1_lds_bytes(k) > lds_cap())
+        return fail(RT_HIP_E_SHAPE, "rt_hip_gemv_q4k: k too large for the LDS");
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    return check_stream_launch(m == 1 ? launch_gemv_q4k_mfma(blocks, x, y, n, k, s)
+                                      : launch_gemv_batch(RT_HIP_Q4K, blocks, x, y, n, k, m, s),
+                               "rt_hip_gemv_q4k");
 }
 
 int rt_hip_gemv_q4k_multi(int32_t count, const void* const* blocks, float* const* y,
@@ -724,14 +704,11 @@ int rt_hip_gemv_bf16(const uint16_t* w, const float* x, float* y, int64_t n, int
                      int32_t m, rt_hip_stream stream) {
     int rc = gemv_args("rt_hip_gemv_bf16", w, x, y, n, k, m, 8);
     if (rc) return rc;
-    if (m > 1 && tune_param("GEMV_BATCH_MFMA", 1))
-        return check_stream_launch(launch_gemv_batch(RT_HIP_BF16, w, x, y, n, k, m, static_cast<hipStream_t>(stream)),
-                                   "rt_hip_gemv_bf16");
-    return gemv_batched("rt_hip_gemv_bf16", RT_HIP_BF16, x, y, n, k, m,
-                        [&](const float* xx, float* yy, int mm) {
-                            return launch_gemv_bf16(w, xx, yy, n, k, mm, nullptr,
-                                                    static_cast<hipStream_t>(stream));
-                        });
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (m == 1 && (rc = gemv_k_bound("rt_hip_gemv_bf16", static_cast<size_t>(k) * 4))) return rc;
+    return check_stream_launch(m == 1 ? launch_gemv_bf16_m1(w, x, y, n, k, nullptr, s)
+                                      : launch_gemv_batch(RT_HIP_BF16, w, x, y, n, k, m, s),
+                               "rt_hip_gemv_bf16");
 }
 
 int64_t rt_hip_q4mat_bytes(int64_t n, int64_t k) {
@@ -749,29 +726,24 @@ int rt_hip_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_
     const char* fn = "rt_hip_gemv_q4mat";
     int rc = gemv_args(fn, w, x, y, n, k, m, 32);
     if (rc) return rc;
-    if (q4mat_gemv_lds_bytes(1, k) > lds_cap()) return fail(RT_HIP_E_SHAPE, std::string(fn) + ": k too large for the LDS");
+    if (q4mat_gemv_lds_bytes(k) > lds_cap()) return fail(RT_HIP_E_SHAPE, std::string(fn) + ": k too large for the LDS");
     hipError_t e;
     if (!state_for_current(&e)) return hip_fail(e, fn);
-    int mb = m;
-    while (mb > 1 && q4mat_gemv_lds_bytes(mb, k) > lds_cap()) --mb;
-    for (int32_t m0 = 0; m0 < m; m0 += mb) {
-        const int32_t mm = (m - m0) < mb ? (m - m0) : mb;
-        e = launch_gemv_q4mat(w, x + static_cast<size_t>(m0) * k, y + static_cast<size_t>(m0) * n, n, k, mm,
-                              static_cast<hipStream_t>(stream));
-        if (e != hipSuccess) return hip_fail(e, fn);
-    }
-    return RT_HIP_OK;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    return check_stream_launch(m == 1 ? launch_gemv_q4mat(w, x, y, n, k, s)
+                                      : launch_gemv_batch(RT_HIP_Q4MAT, w, x, y, n, k, m, s),
+                               fn);
 }
 
 int rt_hip_gemv_q4_0(const void* blocks, const float* x, float* y, int64_t n, int64_t k,
                      int32_t m, rt_hip_stream stream) {
     int rc = gemv_args("rt_hip_gemv_q4_0", blocks, x, y, n, k, m, 256);
     if (rc) return rc;
-    return gemv_batched("rt_hip_gemv_q4_0", RT_HIP_Q4_0, x, y, n, k, m,
-                        [&](const float* xx, float* yy, int mm) {
-                            return launch_gemv_q4_0(blocks, xx, yy, n, k, mm,
-                                                    static_cast<hipStream_t>(stream));
-                        });
+    if ((rc = gemv_k_bound("rt_hip_gemv_q4_0", static_cast<size_t>(k) * 33 / 32 * 4))) return rc;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    return check_stream_launch(m == 1 ? launch_gemv_q4_0_m1(blocks, x, y, n, k, s)
+                                      : launch_gemv_batch(RT_HIP_Q4_0, blocks, x, y, n, k, m, s),
+                               "rt_hip_gemv_q4_0");
 }
 
 int rt_hip_dequant_q6k_bf16(const void* blocks, uint16_t* out, int64_t n, int64_t k, rt_hip_stream stream) {

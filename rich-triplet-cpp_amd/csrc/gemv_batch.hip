@@ -1,42 +1,55 @@
 // gemv_batch.hip -- batched GEMV, M = 2..8 activation rows (speculative
 // verify): Y[m][n] = sum_k X[m][k] * W[n][k] on MFMA, every weight byte read
-// once for all M rows (decode_gemma3.msl:416-518, MAX_BATCH 8).
+// once for all M rows (decode_gemma3.msl:416-518, MAX_BATCH 8).  Weights:
+// Q4_K blocks, GGUF Q4_0 blocks, Q4Mat storage, or BF16.
 //
 // One MFMA step covers 32 values of K for a 16-row weight tile and up to four
 // activation rows t of a group q (Q = ceil(M / 4) groups, one MFMA each):
-//  * B is the weight tile: lane l = (n = l%16, g = l/16) supplies the 8
-//    weights of row n at k-slots 8g..8g+7 of the step.
-//  * A row i = 4t + lambda (lambda < 3; row 4t + 3 is zero) is limb lambda of
-//    activation row 4q + t over the same k-slots.
+//  * B is the weight tile: lane l = (n = l%16, g = l/16) supplies 8 weights
+//    of row n; the same 8 positions of the activations stand in A, so each
+//    format picks the positions its bytes hold (Fmt::kX*).
+//  * A row i = 4t + lambda (lambda < 3) is limb lambda of activation row
+//    4q + t.  Rows i with lambda == 3 or past M hold whatever lies in LDS:
+//    a row of A reaches only its own row of the result, and theirs are unused.
 //  * The output lane (n, g) holds C[4g + r][n], r = 0..3: the three limb
 //    dots of activation row 4q + g for weight row n, combined in the lane.
 //
 // Exact activation limbs, so that the MFMA products are exact:
 //  * BF16 weights (v_mfma_f32_16x16x32_bf16): three bf16 limbs with
-//    h + m + l == x exactly -- h = bf16(x), m = bf16(x - h), l = x - h - m
-//    (each difference is exact in f32, the last has at most 8 significant
-//    bits).  Products of bf16 values are exact in f32, so only the f32
-//    accumulation rounds, as in an f32 dot product.
-//  * Q4_K weights (v_mfma_i32_16x16x32_i8): the step is one 32-value
-//    sub-block, and x carries the int8 limbs of the M = 1 kernel
-//    (q4k_mfma.hpp): per sub-block a power-of-two s and A0 + A1/256 + A2/65536
-//    == x / s to 2.5e-7 * absmax.  Each limb dot against the nibbles is an
-//    exact int32, and per sub-block j (quant_q4k.cpp:482-523)
-//        sum x * w = (d*sv_j) * (s*C0 + s/256*C1 + s/65536*C2) - (dmin*mv_j) * sum(x).
-//    Sub-block j's values k = 32j + t sit in byte 32*(j/2) + t of qs, low
-//    nibble for even j and high for odd (quant_q4k.cpp:280-317).
+//    h + m + l == x exactly.  Products of bf16 values are exact in f32, so
+//    only the f32 accumulation rounds, as in an f32 dot product.
+//  * 4-bit weights (v_mfma_i32_16x16x32_i8): the step is one 32-value block
+//    with one scale, and x carries the int8 limbs of the M = 1 kernel
+//    (q4k_mfma.hpp): per block a power-of-two s and A0 + A1/256 + A2/65536
+//    == x / s to 2.5e-7 * absmax.  Each limb dot is an exact int32.
+//    - Q4_K: nibbles 0..15, so R = C0 * 65536 + C1 * 256 + C2 stays below
+//      32 * 15 * 2^22 < 2^31 and is converted once; the minimum's term,
+//      -(dmin * mv_j) * sum(x), is a contraction over the super-block's eight
+//      sub-blocks and runs on v_mfma_f32_16x16x4_f32 (quant_q4k.cpp:482-523).
+//    - Q4_0, Q4Mat: signed values (nibble - 8, or the two's-complement
+//      nibble) as int8 multiples of 16, so no offset term is left.
 //
-// Work split.  A workgroup of kWaves waves stages one K-slice of all M rows
-// as limbs in LDS and each wave runs one 16-row tile over that slice, its
-// weights streamed through a ring of D slots.  LDS bounds the slice, and
-// short outputs need several slices to occupy the CUs.  With one slice the
-// workgroup writes Y.  With more, every workgroup writes its partial
-// products to a workspace and counts its arrival for its tile group; the
-// last to arrive adds the group's partials in slice order (so the result
-// does not depend on arrival order) and resets the counter.  A slice is
-// padded with zero activation steps to whole ring rounds, so the loop has
-// no tail: padded steps add exact zeros, and weight loads past the slice's
-// real slots get an empty buffer range (zeros, no memory traffic).
+// Work split: a workgroup of 8 waves stages all M rows as limbs in LDS, KS
+// waves share a 16-row tile's K (slots ks, ks + KS, ...) and their sums meet
+// in LDS; 8 / KS tiles run side by side, and the workgroup walks tile groups
+// blockIdx.x, + gridDim.x, ...  Where K is too long for LDS it is staged in
+// chunks, or, where that is quicker, the chunks run in workgroups of their
+// own and the last to arrive adds the partial sums (plan()).  Each wave keeps
+// kDepth slots of weights in flight in registers, over chunk and group ends.
+//
+// Bound: short outputs by the chain launch -> x -> limbs -> MFMA -> store.
+// The limbs cost about 90 VALU per 8 values in every workgroup (1024 x 3072,
+// M = 8: 1.6 us of 7.5, reading x 1.1); long outputs by the epilogue's VALU,
+// about 100 per slot at M <= 4 and 140 at M <= 8.  Keeping K inside the
+// workgroup saves the merge through memory that every K longer than one slice
+// used to pay (1.7 us).  Measured, before -> now, us per launch in a graph:
+//   Q4_K  3072 x 3072  M = 4: 7.8 -> 5.6   M = 8: 9.3 -> 7.8
+//   Q4_K  8192 x 3072  M = 4: 8.4 -> 7.7   M = 8: 10.0 -> 9.9
+//   Q4_K  3072 x 8192  M = 4: 11.8 -> 10.3 M = 8: 14.5 -> 13.6
+//   BF16  3072 x 3072  M = 4: 10.8 -> 8.1  M = 8: 11.7 -> 10.2
+//   Q4_0  4096 x 4096  M = 4: 19.3 -> 6.2  M = 8: 30.2 -> 8.4 (VALU before)
+//   Q4_0  4096 x 11008 M = 4: 248 -> 12.5  M = 8: 626 -> 15.7
+//   Q4Mat 4096 x 4096  M = 4: 16.4 -> 6.6  M = 8: 53.2 -> 9.4 (VALU before)
 #include "q4k_mfma.hpp"
 #include "rt_common.hpp"
 #include "rt_launch.hpp"
@@ -47,65 +60,261 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * kWave;
-constexpr int kZeroBytes = 16;
+constexpr int kWaves = 8;  // (16 for long outputs at M > 4, below)
+constexpr int kDepth = 2;  // weight slots in flight per wave
+constexpr uint32_t kNoRead = 0x7ffffff0u;
 
 // ---- formats -------------------------------------------------------------
-// A slot is the unit the ring loads: kSteps 32-value steps of one tile.
-// LDS per (step, group): kLimb bytes of A limbs ([g][t][lambda] x kFrag)
-// and kCst bytes of per-row constants.
+// A slot is the unit a wave loads: kSteps 32-value steps of one 16-row tile.
+// load(): row n's bytes of slot `sl`, lane (n, g); rows past the resource's
+// range and pieces past K read zeros.
 
 struct BBf16 {
+    static constexpr bool kInt = false, kMin = false;
     static constexpr int kSteps = 4;  // 128 values
-    static constexpr int kSlotCost = 1;  // one slot's time, in units of one slice's reduction
-    static constexpr int kFrag = 16;  // 8 bf16
-    static constexpr int kLimb = 48 * kFrag;
-    static constexpr int kCst = 0;
+    static constexpr int kX0 = 8, kX1 = 4;  // lane group g: values 8g.. and 8g + 4..
+    static constexpr bool kTail = true;     // K need not be whole slots
     struct Slot { u32x4 v[4]; };
-    // The tile's rows start at `tile` (row-major, rb bytes apart); the slot
-    // covers values [k, k + 128).  Lane (n, g) reads 16 bytes of row n per
-    // step; pieces past K (K % 8 == 0: all or nothing) read zeros.
-    __device__ static void load(const uint8_t* tile, int64_t left, int64_t rb, int k, int K, int lane,
-                                Slot& s) {
-        const BufRsrc rs = make_rsrc(tile + 2 * static_cast<int64_t>(k), left - 2 * static_cast<int64_t>(k));
-        const uint32_t roff = static_cast<uint32_t>((lane & 15) * rb);
+    struct Tile {
+        const uint8_t* base;
+        int64_t left;
+        uint32_t roff;
+    };
+    __device__ static Tile tile(const uint8_t* w, int64_t, int row0, int n_rows, int K, int lane) {
+        const int64_t rb = 2 * static_cast<int64_t>(K);
+        return Tile{w + row0 * rb, static_cast<int64_t>(n_rows - row0) * rb,
+                    static_cast<uint32_t>((lane & 15) * rb)};
+    }
+    __device__ static void load(const Tile& t, bool live, int sl, int K, int lane, Slot& s) {
+        const int64_t o = static_cast<int64_t>(sl) * 256;
+        const BufRsrc rs = make_rsrc(t.base + o, live ? t.left - o : 0);
         const int g = lane >> 4;
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
-            const bool in = k + 32 * st + 8 * g < K;
-            s.v[st] = ld16(rs, in ? roff + static_cast<uint32_t>(64 * st + 16 * g) : 0xfffffff0u);
+            const bool in = sl * 128 + 32 * st + 8 * g < K;
+            s.v[st] = ld16(rs, in ? t.roff + static_cast<uint32_t>(64 * st + 16 * g) : 0xfffffff0u);
         }
     }
 };
 
+// 4-bit formats: a decoded slot is eight blocks' B operands and scales.
+struct Dec4 {
+    long b[8];
+    float ds[8];
+    float mn[2];  // Q4_K: -(dmin * mv) of sub-blocks g and 4 + g
+};
+
+__device__ __forceinline__ long pair64(uint32_t lo, uint32_t hi) {
+    return static_cast<long>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 struct BQ4k {
+    static constexpr bool kInt = true, kMin = true;
     static constexpr int kSteps = 8;  // one super-block
-    static constexpr int kSlotCost = 2;  // one slot's time, in units of one slice's reduction
-    static constexpr int kFrag = 8;   // 8 int8
-    static constexpr int kLimb = 48 * kFrag;
-    static constexpr int kCst = 64;   // 4 rows x {s, s/256, s/65536, sum}
+    static constexpr int kX0 = 8, kX1 = 4;
+    static constexpr bool kTail = false;
+    static constexpr bool kInterleave = false;
     struct Slot {
         u32x4 h;      // d | dmin << 16, scales[12]
         u32x2 p[4];   // qs[32c + 8g, +8), c = 0..3
     };
-    __device__ static void load(const uint8_t* tile, int64_t left, int64_t rb, int k, int, int lane, Slot& s) {
-        const int64_t o = static_cast<int64_t>(k >> 8) * kQ4kBlockBytes;
-        const BufRsrc rs = make_rsrc(tile + o, left - o);
-        const uint32_t roff = static_cast<uint32_t>((lane & 15) * rb);
+    struct Tile {
+        const uint8_t* base;
+        int64_t left;
+        uint32_t roff;
+    };
+    __device__ static Tile tile(const uint8_t* w, int64_t, int row0, int n_rows, int K, int lane) {
+        const int64_t rb = static_cast<int64_t>(K >> 8) * kQ4kBlockBytes;
+        return Tile{w + row0 * rb, static_cast<int64_t>(n_rows - row0) * rb,
+                    static_cast<uint32_t>((lane & 15) * rb)};
+    }
+    __device__ static void load(const Tile& t, bool live, int sl, int, int lane, Slot& s) {
+        const int64_t o = static_cast<int64_t>(sl) * kQ4kBlockBytes;
+        const BufRsrc rs = make_rsrc(t.base + o, live ? t.left - o : 0);
         const uint32_t g8 = static_cast<uint32_t>(lane >> 4) * 8u;
-        s.h = ld16(rs, roff);
+        s.h = ld16(rs, t.roff);
 #pragma unroll
         for (int c = 0; c < 4; ++c)
             s.p[c] = __builtin_bit_cast(
-                u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, static_cast<int>(roff + 16u + 32u * c + g8), 0, 0));
+                u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, static_cast<int>(t.roff + 16u + 32u * c + g8), 0, 0));
+    }
+    // Sub-block j's values k = 32j + t sit in byte 32*(j/2) + t of qs, low
+    // nibble for even j and high for odd (quant_q4k.cpp:280-317); the 6-bit
+    // scales four at a time (Q4KMat::scale_min, quant_q4k.cpp:58-69).
+    __device__ static void decode(const Slot& s, int lane, Dec4& o) {
+        const uint32_t h1 = s.h[1], h2 = s.h[2], h3 = s.h[3];
+        const uint32_t sl = h1 & 0x3f3f3f3fu, sh = (h3 & 0x0f0f0f0fu) | ((h1 >> 2) & 0x30303030u);
+        const uint32_t ml = h2 & 0x3f3f3f3fu, mh = ((h3 >> 4) & 0x0f0f0f0fu) | ((h2 >> 2) & 0x30303030u);
+        const float d = f16_bits_to_f32(s.h[0] & 0xffffu), nd = -f16_bits_to_f32(s.h[0] >> 16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            o.ds[j] = d * ubyte_f32(sl, j);
+            o.ds[4 + j] = d * ubyte_f32(sh, j);
+        }
+        const uint32_t g8 = static_cast<uint32_t>(lane >> 4) * 8u;
+        o.mn[0] = nd * static_cast<float>(__builtin_amdgcn_ubfe(ml, g8, 8));
+        o.mn[1] = nd * static_cast<float>(__builtin_amdgcn_ubfe(mh, g8, 8));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            o.b[2 * c] = pair64(s.p[c][0] & 0x0f0f0f0fu, s.p[c][1] & 0x0f0f0f0fu);
+            o.b[2 * c + 1] = pair64((s.p[c][0] >> 4) & 0x0f0f0f0fu, (s.p[c][1] >> 4) & 0x0f0f0f0fu);
+        }
     }
 };
 
-template <class F>
-__host__ __device__ inline size_t batch_lds_bytes(int steps, int q) {
-    return static_cast<size_t>(steps) * q * (F::kLimb + F::kCst) + kZeroBytes;
+// 4 x 4 transpose over (lane group, register): out[j] of lane group g is
+// in[g] of lane group j.  Four gfx950 permlane swaps.
+__device__ __forceinline__ void transpose4(uint32_t (&a)[4]) {
+    auto s0 = __builtin_amdgcn_permlane32_swap(a[0], a[2], false, false);
+    auto s1 = __builtin_amdgcn_permlane32_swap(a[1], a[3], false, false);
+    auto t0 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
+    auto t1 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
+    a[0] = t0[0];
+    a[1] = t0[1];
+    a[2] = t1[0];
+    a[3] = t1[1];
 }
+// out[j] = lane group j's value, in every lane.
+__device__ __forceinline__ void gather4(uint32_t v, uint32_t (&o)[4]) {
+    auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    auto e = __builtin_amdgcn_permlane32_swap(r[0], r[0], false, false);
+    auto d = __builtin_amdgcn_permlane32_swap(r[1], r[1], false, false);
+    o[0] = e[0];
+    o[1] = d[0];
+    o[2] = e[1];
+    o[3] = d[1];
+}
+// Signed nibbles of v (two's complement) as int8 multiples of 16.
+__device__ __forceinline__ long signed16(uint32_t v) { return pair64((v << 4) & 0xf0f0f0f0u, v & 0xf0f0f0f0u); }
+
+// GGUF Q4_0: 18-byte blocks (d f16, qs[16]; value j < 16 the low nibble of
+// qs[j] minus 8, value 16 + j the high one; gguf.cpp:495-529).  A row's slot
+// is 144 contiguous bytes: lane group g loads bytes [36g, 36g + 36), blocks
+// 2g and 2g + 1 whole, and the transpose hands every lane dword g of each
+// block: values 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3.
+struct BQ40 {
+    static constexpr bool kInt = true, kMin = false;
+    static constexpr int kSteps = 8;
+    static constexpr int kX0 = 4, kX1 = 16;  // values 4g.. and 4g + 16..
+    static constexpr bool kTail = false;
+    static constexpr bool kInterleave = false;
+    struct Slot {
+        u32x4 a, b;
+        uint32_t c;
+    };
+    struct Tile {
+        const uint8_t* base;
+        int64_t left;
+        uint32_t roff;
+    };
+    __device__ static Tile tile(const uint8_t* w, int64_t, int row0, int n_rows, int K, int lane) {
+        const int64_t rb = static_cast<int64_t>(K >> 5) * kQ40BlockBytes;
+        return Tile{w + row0 * rb, static_cast<int64_t>(n_rows - row0) * rb,
+                    static_cast<uint32_t>((lane & 15) * rb + 36 * (lane >> 4))};
+    }
+    __device__ static void load(const Tile& t, bool live, int sl, int, int, Slot& s) {
+        const int64_t o = static_cast<int64_t>(sl) * 144;
+        const BufRsrc rs = make_rsrc(t.base + o, live ? t.left - o : 0);
+        s.a = ld16(rs, t.roff);  // dword-aligned 16-byte loads
+        s.b = ld16(rs, t.roff + 16);
+        s.c = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(t.roff + 32), 0, 0);
+    }
+    __device__ static void decode(const Slot& s, int, Dec4& o) {
+        uint32_t x[4], y[4], dd[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = __builtin_amdgcn_alignbyte(j < 3 ? s.a[j + 1] : s.b[0], s.a[j], 2);
+        y[0] = s.b[1];
+        y[1] = s.b[2];
+        y[2] = s.b[3];
+        y[3] = s.c;
+        // both d's: the low half of dword 0, the high half of dword 4
+        gather4((s.a[0] & 0xffffu) | (s.b[0] & 0xffff0000u), dd);
+        transpose4(x);
+        transpose4(y);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            o.ds[2 * j] = 0.0625f * f16_bits_to_f32(dd[j] & 0xffffu);
+            o.ds[2 * j + 1] = 0.0625f * f16_bits_to_f32(dd[j] >> 16);
+            o.b[2 * j] = signed16(x[j] ^ 0x88888888u);
+            o.b[2 * j + 1] = signed16(y[j] ^ 0x88888888u);
+        }
+    }
+};
+
+// Q4Mat (rt_hip.h): packed nibbles, element 2i the low nibble of byte i, and
+// f32 scales.  Lane group g loads groups 2g and 2g + 1 of the slot (32 bytes
+// and two scales); after the transpose dword g of a group holds values 8g ..
+// 8g + 7, the even ones in its low nibbles.
+struct BQ4m {
+    static constexpr bool kInt = true, kMin = false;
+    static constexpr int kSteps = 8;
+    static constexpr int kX0 = 8, kX1 = 4;
+    static constexpr bool kTail = true;
+    static constexpr bool kInterleave = true;
+    struct Slot {
+        u32x4 a, b;
+        uint32_t s0, s1;
+    };
+    struct Tile {
+        const uint8_t* base;
+        const uint8_t* sc;
+        int64_t left, sleft;
+        uint32_t roff, soff;
+    };
+    __device__ static Tile tile(const uint8_t* w, int64_t sc_off, int row0, int n_rows, int K, int lane) {
+        const int64_t rb = K >> 1, sb = static_cast<int64_t>(K >> 5) * 4;
+        return Tile{w + row0 * rb, w + sc_off + row0 * sb, static_cast<int64_t>(n_rows - row0) * rb,
+                    static_cast<int64_t>(n_rows - row0) * sb,
+                    static_cast<uint32_t>((lane & 15) * rb + 32 * (lane >> 4)),
+                    static_cast<uint32_t>((lane & 15) * sb + 8 * (lane >> 4))};
+    }
+    __device__ static void load(const Tile& t, bool live, int sl, int K, int lane, Slot& s) {
+        const int64_t o = static_cast<int64_t>(sl) * 128, os = static_cast<int64_t>(sl) * 32;
+        const BufRsrc rs = make_rsrc(t.base + o, live ? t.left - o : 0);
+        const BufRsrc rc = make_rsrc(t.sc + os, live ? t.sleft - os : 0);
+        const int grp = sl * 8 + 2 * (lane >> 4), ng = K >> 5;
+        const bool i0 = grp < ng, i1 = grp + 1 < ng;
+        s.a = ld16(rs, i0 ? t.roff : kNoRead);
+        s.b = ld16(rs, i1 ? t.roff + 16 : kNoRead);
+        s.s0 = __builtin_amdgcn_raw_buffer_load_b32(rc, static_cast<int>(i0 ? t.soff : kNoRead), 0, 0);
+        s.s1 = __builtin_amdgcn_raw_buffer_load_b32(rc, static_cast<int>(i1 ? t.soff + 4 : kNoRead), 0, 0);
+    }
+    __device__ static void decode(const Slot& s, int, Dec4& o) {
+        uint32_t x[4] = {s.a[0], s.a[1], s.a[2], s.a[3]}, y[4] = {s.b[0], s.b[1], s.b[2], s.b[3]}, d0[4], d1[4];
+        gather4(s.s0, d0);
+        gather4(s.s1, d1);
+        transpose4(x);
+        transpose4(y);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            o.ds[2 * j] = 0.0625f * __uint_as_float(d0[j]);
+            o.ds[2 * j + 1] = 0.0625f * __uint_as_float(d1[j]);
+            o.b[2 * j] = signed16(x[j]);
+            o.b[2 * j + 1] = signed16(y[j]);
+        }
+    }
+};
+
+// LDS of one staged slot for Q row groups:
+//   4-bit: limbs [4 step pairs][4Q rows][4 g][3 lambda][2 steps][8 bytes], then
+//          scales s / 65536 [4Q rows][8 steps] and (Q4_K) sums of x, the same shape;
+//   BF16:  limbs [4 steps][4Q rows][4 g][3 lambda][16 bytes].
+// Step (pair) records are 16 bytes longer than their limbs, which spreads the
+// lanes of a staging write, one step after another, over the banks.
+__host__ __device__ constexpr int step_bytes(int q) { return q * 768 + 16; }
+template <class F>
+__host__ __device__ constexpr int limb_bytes(int q) {
+    return 4 * step_bytes(q);
+}
+template <class F>
+__host__ __device__ constexpr int cst_bytes(int q) {
+    return F::kInt ? q * 4 * 8 * 4 : 0;
+}
+template <class F>
+__host__ __device__ constexpr int slot_lds(int q) {
+    return limb_bytes<F>(q) + cst_bytes<F>(q) * (F::kMin ? 2 : 1);
+}
+constexpr int red_bytes(int waves, int q) { return waves * q * kWave * 4; }
 
 // Sum and max over the aligned quad of lanes (every lane gets the same bits).
 __device__ __forceinline__ float quad_sum(float v) {
@@ -119,6 +328,16 @@ __device__ __forceinline__ float quad_max(float v) {
     return v;
 }
 
+// One launch's shape: tile groups of waves / KS tiles (KS = 1 << ks_log); K
+// in `nslots` slots, staged `cslots` at a time.
+// With slices > 1 (grid y) a workgroup takes one chunk alone and the chunks'
+// partial sums meet in memory.
+struct BatchShape {
+    int n, k, m, ks_log, groups, nslots, cslots, nchunks, per;  // per: slots per wave and chunk, whole rings
+    int slices, waves;
+    int64_t sc_off;  // Q4Mat: byte offset of the scales
+};
+
 // Partials are stored and reloaded with agent-scope (device-coherent)
 // accesses: they bypass the per-XCD L2, so the workgroup that reduces them
 // sees every other XCD's stores once those have completed.
@@ -130,120 +349,145 @@ __device__ __forceinline__ float ld_dev(const float* p) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Workgroup (blockIdx.x, blockIdx.y) = (group of kWaves tiles, K-slice).
-// The slice is `slots` ring slots from slot slice * slots (the last slice may
-// hold fewer real ones); `psteps` = slots padded to whole rounds of D, in
-// steps, is what LDS holds.  Y is [M][N]; with gridDim.y > 1 slices, P holds
-// the partials ([slice][M][N]) and counters[blockIdx.x] the arrivals.
-template <class F, int Q, int D, int XP>
-__global__ __launch_bounds__(kThreads) void k_gemv_batch(const uint8_t* __restrict__ W, const float* __restrict__ X,
-                                                         float* __restrict__ Y, float* __restrict__ P,
-                                                         uint32_t* __restrict__ counters, int N, int K, int M,
-                                                         int slots, int psteps) {
-    constexpr bool kQ4 = F::kSteps == 8;
+// XP: units of 8 activations a thread holds while staging one chunk.  Up to 4
+// the kernel fits 128 registers, so two workgroups may share a CU.
+template <class F, int Q, int XP, int NW>
+__global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __restrict__ W, const float* __restrict__ X,
+                                                         int k, int m, int n, int ks_log, int cslots, int nslots,
+                                                         int groups, int per, float* __restrict__ Y, int nchunks,
+                                                         int64_t sc_off, float* __restrict__ P,
+                                                         uint32_t* __restrict__ counters) {
+    // (the arguments before Y are preloaded into SGPRs at wave launch)
+    const BatchShape S{n, k, m, ks_log, groups, nslots, cslots, nchunks, per, static_cast<int>(gridDim.y), NW, sc_off};
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int kLimb = limb_bytes<F>(Q), kCst = cst_bytes<F>(Q), kThreads = NW * kWave;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int slice = blockIdx.y;
-    const int k0 = slice * slots * F::kSteps * 32;          // first value of the slice
-    const int kend = min(K, k0 + slots * F::kSteps * 32);  // end of its real values
-    const int tile = blockIdx.x * kWaves + wave;
-    const int row0 = 16 * tile;
-    const int64_t rb = kQ4 ? static_cast<int64_t>(K >> 8) * kQ4kBlockBytes : 2 * static_cast<int64_t>(K);
-    const uint8_t* const tbase = W + static_cast<int64_t>(row0) * rb;
-    const int64_t tleft = static_cast<int64_t>(N - row0) * rb;  // <= 0 past the last tile: zeros
-    // Real slots of this slice; loads of later ones (the padding and the
-    // ring's last refills) get an empty range, so no wave reads a byte of
-    // the next slice.
-    const int nreal = min(slots, (K + F::kSteps * 32 - 1) / (F::kSteps * 32) - slice * slots);
-    auto load = [&](int sl, typename F::Slot& dst) {
-        F::load(tbase, sl < nreal ? tleft : 0, rb, k0 + sl * F::kSteps * 32, K, lane, dst);
+    const int KS = 1 << S.ks_log, ks = wave & (KS - 1), tw = wave >> S.ks_log, TW = NW >> S.ks_log;
+    const int g = lane >> 4;
+    uint8_t* const cst = lds + S.cslots * kLimb;    // scales, then sums
+    uint8_t* const sums = cst + S.cslots * kCst;
+    float* const red = reinterpret_cast<float*>(lds + S.cslots * slot_lds<F>(Q));
+
+    // x of a chunk into registers: unit u = tid + kThreads * i of the chunk's
+    // row-major sequence is 8 values of row m's step r / 4, lane group r % 4.
+    // Rows past M fall outside the buffer's range and read zeros.
+    f32x4 xa[XP], xb[XP];
+    const BufRsrc xr = make_rsrc(X, static_cast<int64_t>(S.m) * S.k * 4);
+    auto chunk_slots = [&](int c) { return min(S.cslots, S.nslots - c * S.cslots); };
+    struct Units {  // (m, r) of this thread's units, one after another
+        uint32_t upr, dm, dr, m, r;
+        __device__ void next() {
+            m += dm;
+            r += dr;
+            const uint32_t over = r >= upr ? 1u : 0u;
+            m += over;
+            r -= over ? upr : 0u;
+        }
+    };
+    auto units_of = [&](int c) {
+        Units u;
+        u.upr = static_cast<uint32_t>(chunk_slots(c) * F::kSteps * 4);
+        // upr is at least 16 and below 2^14: a reciprocal rounded up by 2^-17 of
+        // itself gives exact quotients of values up to 1024
+        const float inv = __builtin_amdgcn_rcpf(static_cast<float>(u.upr)) * 1.0000076f;
+        u.dm = static_cast<uint32_t>(static_cast<float>(kThreads) * inv);
+        u.dr = kThreads - u.dm * u.upr;
+        u.m = static_cast<uint32_t>(static_cast<float>(tid) * inv);
+        u.r = static_cast<uint32_t>(tid) - u.m * u.upr;
+        return u;
+    };
+    auto load_x = [&](int c) {
+        Units u = units_of(c);
+        const uint32_t k0 = static_cast<uint32_t>(c * S.cslots * F::kSteps * 32);
+#pragma unroll
+        for (int i = 0; i < XP; ++i) {
+            const uint32_t e = k0 + (F::kX0 == 8 ? 8 * u.r : 32 * (u.r >> 2) + 4 * (u.r & 3));
+            uint32_t off = u.m * static_cast<uint32_t>(4 * S.k) + 4 * e;
+            if constexpr (F::kTail) off = e < static_cast<uint32_t>(S.k) ? off : kNoRead;
+            xa[i] = __builtin_bit_cast(f32x4, ld16(xr, off));
+            xb[i] = __builtin_bit_cast(f32x4, ld16(xr, off + 4 * F::kX1));
+            u.next();
+        }
+    };
+    // Limbs (and, for the 4-bit formats, the per-row block constants) into LDS.
+    auto stage = [&](int c) {
+        Units u = units_of(c);
+#pragma unroll
+        for (int i = 0; i < XP; ++i) {
+            const bool in = u.m < static_cast<uint32_t>(S.m);
+            f32x4 a = xa[i], b = xb[i];
+            if constexpr (F::kInt) {
+                if constexpr (F::kInterleave) {
+                    a = f32x4{xa[i][0], xa[i][2], xb[i][0], xb[i][2]};
+                    b = f32x4{xa[i][1], xa[i][3], xb[i][1], xb[i][3]};
+                }
+                // Block (step, m) is the quad of units g = 0..3.
+                float amax = fmaxf(fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))),
+                                   fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3]))));
+                amax = quad_max(amax);
+                float sc, inv;
+                q4k_mfma::sub_block_scale(amax, sc, inv);
+                uint32_t a0, a1, a2, b0, b1, b2;
+                q4k_mfma::limb_words(a, inv, a0, a1, a2);
+                q4k_mfma::limb_words(b, inv, b0, b1, b2);
+                float sum = 0.0f;
+                if constexpr (F::kMin)
+                    sum = quad_sum(((a[0] + a[1]) + (a[2] + a[3])) + ((b[0] + b[1]) + (b[2] + b[3])));
+                if (in) {
+                    uint8_t* const dst =
+                        lds + (u.r >> 3) * step_bytes(Q) + u.m * 192 + (u.r & 3) * 48 + ((u.r & 4) << 1);
+                    *reinterpret_cast<u32x2*>(dst) = u32x2{a0, b0};
+                    *reinterpret_cast<u32x2*>(dst + 16) = u32x2{a1, b1};
+                    *reinterpret_cast<u32x2*>(dst + 32) = u32x2{a2, b2};
+                    if ((u.r & 3) == 0) {
+                        const uint32_t o = (u.r >> 5) * kCst + u.m * 32 + (u.r & 28);
+                        *reinterpret_cast<float*>(cst + o) = sc * (1.0f / 65536.0f);
+                        if constexpr (F::kMin) *reinterpret_cast<float*>(sums + o) = sum;
+                    }
+                }
+            } else {
+                u32x2 ha, ma, la, hb, mb, lb;
+                bf16_limbs4(a, ha, ma, la);
+                bf16_limbs4(b, hb, mb, lb);
+                if (in) {
+                    u32x4* d4 = reinterpret_cast<u32x4*>(lds + (u.r >> 2) * step_bytes(Q) + u.m * 192 + (u.r & 3) * 48);
+                    d4[0] = u32x4{ha[0], ha[1], hb[0], hb[1]};
+                    d4[1] = u32x4{ma[0], ma[1], mb[0], mb[1]};
+                    d4[2] = u32x4{la[0], la[1], lb[0], lb[1]};
+                }
+            }
+            u.next();
+        }
     };
 
-    // x of the slice first, into registers: unit u = (step s, row m, g) is
-    // the 8 values k0 + 32 s + 8 g .. + 8 of row m (zero past the slice).
-    const int units = psteps * M * 4;
-    f32x4 xa[XP], xb[XP];
-#pragma unroll
-    for (int i = 0; i < XP; ++i) {
-        const int u = tid + kThreads * i;
-        const int g = u & 3, sm = u >> 2;
-        const int s = sm / M, m = sm - s * M;
-        const int kk = k0 + 32 * s + 8 * g;
-        const bool in = u < units && kk < kend;
-        const f32x4* src = reinterpret_cast<const f32x4*>(X + static_cast<int64_t>(in ? m : 0) * K + (in ? kk : 0));
-        const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
-        xa[i] = in ? src[0] : z;
-        xb[i] = in ? src[1] : z;
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    int group = blockIdx.x, chunk = blockIdx.y;
+    auto tile_of = [&](int grp) { return F::tile(W, S.sc_off, 16 * (grp * TW + tw), S.n, S.k, lane); };
+    typename F::Tile cur = tile_of(group);
+    typename F::Slot ring[kDepth];
+    // Slot i of this wave in chunk c (none past the chunk's end: an empty
+    // range reads zeros and no memory).
+    auto issue = [&](const typename F::Tile& t, int grp, int c, int i, typename F::Slot& dst) {
+        const int sl = ks + (i << S.ks_log);
+        const bool live = grp < S.groups && sl < chunk_slots(c);
+        F::load(t, live, c * S.cslots + (live ? sl : 0), S.k, lane, dst);
+    };
 
-    typename F::Slot ring[D];
+    load_x(chunk);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-        load(j, ring[j]);
+    for (int j = 0; j < kDepth; ++j) {
+        issue(cur, group, chunk, j, ring[j]);
         __builtin_amdgcn_sched_barrier(0);
     }
-
-    // Limbs (and, for Q4_K, the per-row sub-block constants) into LDS.
-    const uint32_t zoff = static_cast<uint32_t>(psteps * Q * F::kLimb);
-    uint8_t* const cst = lds + zoff + kZeroBytes;
-    if (tid == 0) *reinterpret_cast<u32x4*>(lds + zoff) = u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < XP; ++i) {
-        const int u = tid + kThreads * i;
-        const int g = u & 3, sm = u >> 2;
-        const int s = sm / M, m = sm - s * M;
-        const int q = m >> 2, t = m & 3;
-        uint8_t* const dst = lds + (static_cast<size_t>(s) * Q + q) * F::kLimb + ((g * 4 + t) * 3) * F::kFrag;
-        if constexpr (kQ4) {
-            // Sub-block (s, m) is the quad of units g = 0..3.
-            float amax = fmaxf(fmaxf(fmaxf(fabsf(xa[i][0]), fabsf(xa[i][1])), fmaxf(fabsf(xa[i][2]), fabsf(xa[i][3]))),
-                               fmaxf(fmaxf(fabsf(xb[i][0]), fabsf(xb[i][1])), fmaxf(fabsf(xb[i][2]), fabsf(xb[i][3]))));
-            float sum = ((xa[i][0] + xa[i][1]) + (xa[i][2] + xa[i][3])) + ((xb[i][0] + xb[i][1]) + (xb[i][2] + xb[i][3]));
-            amax = quad_max(amax);
-            sum = quad_sum(sum);
-            float sc, inv;
-            q4k_mfma::sub_block_scale(amax, sc, inv);
-            uint32_t a0, a1, a2, b0, b1, b2;
-            q4k_mfma::limb_words(xa[i], inv, a0, a1, a2);
-            q4k_mfma::limb_words(xb[i], inv, b0, b1, b2);
-            if (u < units) {
-                *reinterpret_cast<u32x2*>(dst) = u32x2{a0, b0};
-                *reinterpret_cast<u32x2*>(dst + 8) = u32x2{a1, b1};
-                *reinterpret_cast<u32x2*>(dst + 16) = u32x2{a2, b2};
-                if (g == 0)
-                    *reinterpret_cast<f32x4*>(cst + ((static_cast<size_t>(s) * Q + q) * 4 + t) * 16) =
-                        f32x4{sc, sc * (1.0f / 256.0f), sc * (1.0f / 65536.0f), sum};
-            }
-        } else {
-            u32x2 ha, ma, la, hb, mb, lb;
-            bf16_limbs4(xa[i], ha, ma, la);
-            bf16_limbs4(xb[i], hb, mb, lb);
-            if (u < units) {
-                u32x4* d4 = reinterpret_cast<u32x4*>(dst);
-                d4[0] = u32x4{ha[0], ha[1], hb[0], hb[1]};
-                d4[1] = u32x4{ma[0], ma[1], mb[0], mb[1]};
-                d4[2] = u32x4{la[0], la[1], lb[0], lb[1]};
-            }
-        }
-    }
+    stage(chunk);
     lds_barrier();
 
-    // This lane's A rows: (t, lambda) = ((l % 16) / 4, l % 4) of group q; a
-    // zero row (lambda == 3, or a row past M) reads the zero line.
-    const int ai = lane & 15, g = lane >> 4;
-    const int at = ai >> 2, al = ai & 3;
-    uint32_t abase[Q], amask[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const bool live = al < 3 && 4 * q + at < M;
-        abase[q] = live ? static_cast<uint32_t>(q * F::kLimb + ((g * 4 + at) * 3 + al) * F::kFrag) : zoff;
-        amask[q] = live ? 0xffffffffu : 0u;
-    }
-    auto a_off = [&](int s, int q) {
-        return abase[q] + ((static_cast<uint32_t>(s) * (Q * F::kLimb)) & amask[q]);
-    };
+    // This lane's A rows: (t, lambda) = ((l % 16) / 4, l % 4) of each group q.
+    const int ai = lane & 15;
+    const uint32_t a_base = static_cast<uint32_t>((ai >> 2) * 192 + g * 48 + min(ai & 3, 2) * 16);
+    // Sums as an f32 A operand: row i = 4t + q of it is activation row 4q + t.
+    const uint32_t s_base = static_cast<uint32_t>((min(ai & 3, Q - 1) * 4 + (ai >> 2)) * 32 + 4 * g);
 
     f32x4 C[Q];
     float acc[Q];
@@ -252,221 +496,312 @@ __global__ __launch_bounds__(kThreads) void k_gemv_batch(const uint8_t* __restri
         C[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         acc[q] = 0.0f;
     }
-
-    // Steady rounds (straight-line; slots past the slice load zeros and
-    // compute against zero limbs).
-    const int rounds = psteps / (F::kSteps * D);
-    for (int r = 0; r < rounds; ++r) {
+    auto consume = [&](const typename F::Slot& slot, int sl) {
+        const uint8_t* const lb = lds + sl * kLimb + a_base;
+        if constexpr (!F::kInt) {
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            const int slot = r * D + j;
-            const int s0 = slot * F::kSteps;
-            if constexpr (!kQ4) {
-                bf16x8 B[4];
+            for (int st = 0; st < 4; ++st)
 #pragma unroll
-                for (int st = 0; st < 4; ++st) B[st] = __builtin_bit_cast(bf16x8, ring[j].v[st]);
-                __builtin_amdgcn_sched_barrier(0);
-                load(slot + D, ring[j]);
+                for (int q = 0; q < Q; ++q) {
+                    const bf16x8 A = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lb + st * step_bytes(Q) + q * 768));
+                    C[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, slot.v[st]), C[q], 0,
+                                                                   0, 0);
+                }
+        } else {
+            Dec4 w;
+            F::decode(slot, lane, w);
+            // The minimum's term of this super-block, added to the row sums
+            // below: kept apart to the end, the two halves of each sum would
+            // grow several times larger than the sum and round accordingly.
+            f32x4 mins = {0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (F::kMin) {
+                const uint8_t* const sb = sums + sl * kCst + s_base;
+                mins = __builtin_amdgcn_mfma_f32_16x16x4f32(*reinterpret_cast<const float*>(sb), w.mn[0], mins, 0, 0, 0);
+                mins = __builtin_amdgcn_mfma_f32_16x16x4f32(*reinterpret_cast<const float*>(sb + 16), w.mn[1], mins, 0,
+                                                            0, 0);
+            }
 #pragma unroll
-                for (int st = 0; st < 4; ++st)
+            for (int q = 0; q < Q; ++q) {
+                const f32x4* kp = reinterpret_cast<const f32x4*>(cst + sl * kCst + (q * 4 + g) * 32);
+                const f32x4 k0 = kp[0], k1 = kp[1];
 #pragma unroll
-                    for (int q = 0; q < Q; ++q) {
-                        const bf16x8 A = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lds + a_off(s0 + st, q)));
-                        C[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[st], C[q], 0, 0, 0);
-                    }
-            } else {
-                const u32x4 h = ring[j].h;
-                u32x2 p[4];
+                for (int p = 0; p < 4; ++p) {
+                    const u32x4 a2 = *reinterpret_cast<const u32x4*>(lb + p * step_bytes(Q) + q * 768);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) p[c] = ring[j].p[c];
-                __builtin_amdgcn_sched_barrier(0);
-                load(slot + D, ring[j]);
-                const float d = f16_bits_to_f32(h[0] & 0xffffu);
-                const float dmin = f16_bits_to_f32(h[0] >> 16);
-#pragma unroll
-                for (int jj = 0; jj < 8; ++jj) {
-                    uint32_t sv, mv;
-                    decode_scale_min(make_scale_sel(jj), h[1], h[2], h[3], sv, mv);
-                    const float a = d * static_cast<float>(sv);
-                    const float dm = dmin * static_cast<float>(mv);
-                    const u32x2 pc = p[jj >> 1];
-                    const uint32_t n0 = (jj & 1) ? (pc[0] >> 4) & 0x0f0f0f0fu : pc[0] & 0x0f0f0f0fu;
-                    const uint32_t n1 = (jj & 1) ? (pc[1] >> 4) & 0x0f0f0f0fu : pc[1] & 0x0f0f0f0fu;
-                    const long B = static_cast<long>((static_cast<uint64_t>(n1) << 32) | n0);
-                    const int s = s0 + jj;
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) {
-                        const long A = *reinterpret_cast<const long*>(lds + a_off(s, q));
+                    for (int e = 0; e < 2; ++e) {
+                        const int j = 2 * p + e;
                         const i32x4 z = {0, 0, 0, 0};
-                        const i32x4 c = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, z, 0, 0, 0);
-                        const f32x4 k4 = *reinterpret_cast<const f32x4*>(
-                            cst + ((static_cast<uint32_t>(s) * Q + q) * 4 + g) * 16);
-                        float dot = static_cast<float>(c[0]) * k4[0];
-                        dot = __builtin_fmaf(static_cast<float>(c[1]), k4[1], dot);
-                        dot = __builtin_fmaf(static_cast<float>(c[2]), k4[2], dot);
-                        acc[q] = __builtin_fmaf(a, dot, acc[q]);
-                        acc[q] = __builtin_fmaf(-dm, k4[3], acc[q]);
+                        const i32x4 c =
+                            __builtin_amdgcn_mfma_i32_16x16x32_i8(pair64(a2[2 * e], a2[2 * e + 1]), w.b[j], z, 0, 0, 0);
+                        const float kj = j < 4 ? k0[j & 3] : k1[j & 3];
+                        if constexpr (F::kMin) {
+                            // |R * nibble| sums below 2^31 (see above); the shifts wrap, the total does not
+                            const uint32_t tot = (((static_cast<uint32_t>(c[0]) << 8) + static_cast<uint32_t>(c[1]))
+                                                  << 8) + static_cast<uint32_t>(c[2]);
+                            acc[q] = __builtin_fmaf(w.ds[j], static_cast<float>(static_cast<int>(tot)) * kj, acc[q]);
+                        } else {
+                            const int hi = c[0] * 256 + c[1];
+                            const float dot = __builtin_fmaf(static_cast<float>(hi), 256.0f, static_cast<float>(c[2]));
+                            acc[q] = __builtin_fmaf(w.ds[j], dot * kj, acc[q]);
+                        }
                     }
                 }
+                if constexpr (F::kMin) acc[q] += mins[q];
             }
         }
-    }
+    };
 
-    // Row n of the tile, activation row 4q + g.
-    const int row = row0 + (lane & 15);
-    const int nslices = gridDim.y;
-    const int64_t total = static_cast<int64_t>(M) * N;
-    bool keep[Q];
-    int64_t idx[Q];
+    for (;;) {
+        // The next unit of work: this group's next chunk, or the next group.
+        const bool last_chunk = S.slices > 1 || chunk + 1 == S.nchunks;
+        const int ngroup = last_chunk ? group + static_cast<int>(gridDim.x) : group, nchunk = last_chunk ? 0 : chunk + 1;
+        const typename F::Tile next = tile_of(min(ngroup, S.groups - 1));
+        const int cs = chunk_slots(chunk);
+        for (int i = 0; i < S.per; i += kDepth) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int m = 4 * q + g;
-        keep[q] = m < M && row < N;
-        idx[q] = static_cast<int64_t>(m) * N + row;
-        const float v = kQ4 ? acc[q] : (C[q][0] + C[q][1]) + C[q][2];
-        if (nslices == 1) {
-            if (keep[q]) Y[idx[q]] = v;
-        } else if (keep[q]) {
-            st_dev(P + slice * total + idx[q], v);
+            for (int j = 0; j < kDepth; ++j) {
+                const int sl = ks + ((i + j) << S.ks_log);
+                if (sl < cs) consume(ring[j], sl);
+                __builtin_amdgcn_sched_barrier(0);
+                const int ii = i + j + kDepth;
+                if (ii < S.per)
+                    issue(cur, group, chunk, ii, ring[j]);
+                else if (ngroup < S.groups)
+                    issue(next, ngroup, nchunk, ii - S.per, ring[j]);
+            }
+        }
+        if (last_chunk) {
+            // Row n of the tile, activation row 4q + g.
+            const int row = 16 * (group * TW + tw) + (lane & 15);
+            float v[Q];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                v[q] = F::kInt ? acc[q] : (C[q][0] + C[q][1]) + C[q][2];
+                C[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                acc[q] = 0.0f;
+            }
+            if (S.ks_log) {
+                // The KS waves' sums in wave order.
+#pragma unroll
+                for (int q = 0; q < Q; ++q) red[(wave * Q + q) * kWave + lane] = v[q];
+                lds_barrier();
+                if (ks == 0) {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+                        for (int j = 1; j < KS; ++j) v[q] += red[((wave + j) * Q + q) * kWave + lane];
+                }
+                if (ngroup < S.groups) lds_barrier();  // before the next group's sums
+            }
+            const int64_t total = static_cast<int64_t>(S.m) * S.n;
+            const bool mine = ks == 0 && row < S.n;
+            if (S.slices > 1) {
+                // Every wave's partials have completed, then one arrival per
+                // workgroup; the last to arrive adds them in slice order (the
+                // result does not depend on which) and resets the counter.
+                // The ordering rests on the accesses themselves: the partials
+                // are agent-scope stores (written through past the XCD's L2)
+                // whose completion every wave has waited for (vmcnt(0))
+                // before the barrier and the arrival, and the merging
+                // workgroup reads them with agent-scope loads, issued once
+                // the arrival's result is known.  A release/acquire on the
+                // arrival would write back and invalidate the XCD's whole L2
+                // in every workgroup: measured 15.8 against 10.2 us for Q4_K
+                // 8192 x 3072 at M = 8.
+                if (mine)
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+                        if (4 * q + g < S.m)
+                            st_dev(P + blockIdx.y * total + static_cast<int64_t>(4 * q + g) * S.n + row, v[q]);
+                wait_vmcnt<0>();
+                lds_barrier();
+                uint32_t* const flag = reinterpret_cast<uint32_t*>(lds);  // the limbs are dead
+                if (tid == 0)
+                    *flag = __hip_atomic_fetch_add(counters + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                lds_barrier();
+                if (*flag != static_cast<uint32_t>(S.slices - 1)) return;
+                if (mine)
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+                        if (4 * q + g < S.m) {
+                            const float* const src = P + static_cast<int64_t>(4 * q + g) * S.n + row;
+                            v[q] = ld_dev(src);
+                            for (int j = 1; j < S.slices; ++j) v[q] += ld_dev(src + j * total);
+                        }
+                if (tid == 0) __hip_atomic_store(counters + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (mine) {
+#pragma unroll
+                for (int q = 0; q < Q; ++q)
+                    if (4 * q + g < S.m) Y[static_cast<int64_t>(4 * q + g) * S.n + row] = v[q];
+            }
+        }
+        if (ngroup >= S.groups) break;
+        group = ngroup;
+        chunk = nchunk;
+        cur = next;
+        if (S.nchunks > 1) {
+            load_x(chunk);
+            lds_barrier();  // every wave is done with the limbs in LDS
+            stage(chunk);
+            lds_barrier();
         }
     }
-    if (nslices == 1) return;
+}
 
-    // Every wave's partials have completed, then one arrival per workgroup.
-    // The limbs are dead: LDS dword 0 carries the arrival number.
-    // The ordering rests on the accesses themselves rather than on fences:
-    // the partials are agent-scope atomic stores (written through past the
-    // XCD's L2) whose completion every wave has waited for (vmcnt(0)) before
-    // the barrier and the arrival, and the merging workgroup reads them with
-    // agent-scope atomic loads (not served from its L2), issued only once
-    // the arrival's result is known.  A release/acquire on the arrival would
-    // also write back and invalidate the whole L2 of the XCD in every
-    // workgroup (buffer_wbl2 / buffer_inv): measured 15.8 against 10.2 us
-    // for Q4_K 8192 x 3072 at M = 8.
-    wait_vmcnt<0>();
-    lds_barrier();
-    uint32_t* const flag = reinterpret_cast<uint32_t*>(lds);
-    if (tid == 0)
-        *flag = __hip_atomic_fetch_add(counters + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    lds_barrier();
-    if (*flag != static_cast<uint32_t>(nslices - 1)) return;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        if (!keep[q]) continue;
-        float sum = ld_dev(P + idx[q]);
-        for (int j = 1; j < nslices; ++j) sum += ld_dev(P + j * total + idx[q]);
-        Y[idx[q]] = sum;
+// Two workgroups of `cs`-slot chunks fit one CU: LDS, and registers (XP <= 4).
+template <class F>
+bool two_fit(int64_t cs, int m, int q) {
+    return 2 * (cs * slot_lds<F>(q) + red_bytes(kWaves, q)) <= static_cast<int64_t>(lds_cap()) &&
+           cs * F::kSteps * 4 * m <= 4 * kWaves * kWave;
+}
+
+// The launch shape: the least estimated time over the splits of K between
+// the waves of a workgroup (KS) and, with `sliced`, between workgroups.  In
+// units of 0.1 us above the launch, fitted to Q4_K times at N x K = 1024 ..
+// 10240 x 3072, 3072 x 8192 and 2560 x 10240 and BF16 ones at 3072 and 8192
+// x 3072 and 3072 x 8192, M = 2, 4 and 8:
+//   staging   1.3 per 1024 activations (every workgroup, each chunk it takes;
+//             once when one chunk holds all of K), 12 (BF16 20) more per
+//             further chunk;
+//   slots     7 (M <= 4) or 9 per 4-bit slot of each wave, 6 per BF16 slot;
+//   3 for the waves' reduction, 14 + 5 slices for a merge through memory
+//             (6 at M > 4; BF16 15 + 5);
+//   two workgroups of one CU overlap: each then takes 1.2 times as long (1.5
+//             at M > 4, BF16 1.7).
+// The best of the shapes swept is within 5% of the one taken at those sizes
+// (Q4_K 3072 x 8192, M = 4: 10.3 us in 4 slices, 11.5 in one; M = 8: 13.5,
+// 16.9).
+template <class F, int Q>
+bool plan(int64_t n, int64_t k, int m, bool sliced, BatchShape* out) {
+    const int64_t cus = device_info().cus;
+    const int64_t tiles = (n + 15) / 16, nslots = (k + F::kSteps * 32 - 1) / (F::kSteps * 32);
+    const int64_t lds = static_cast<int64_t>(lds_cap());
+    // Chunks: what LDS holds, and 8 units of x per thread.
+    const int64_t fit = (lds - red_bytes(kWaves, Q)) / slot_lds<F>(Q);
+    const int64_t by_x = 8 * kWaves * kWave / (static_cast<int64_t>(F::kSteps) * 4 * m);
+    const int64_t cmax = fit < by_x ? fit : by_x;
+    if (cmax < 1) return false;
+    const int64_t cmin = (nslots + cmax - 1) / cmax;
+    // Long outputs at M > 4 whose limbs leave room for one workgroup per CU:
+    // 16 waves, each with tiles of its own (8 waves leave the matrix cores
+    // waiting: Q4_K 128256 x 3072, M = 8: 75.0 us with 8, 63 with 16).
+    if (F::kInt && Q == 2 && cmin == 1 && tiles >= 16 * cus &&
+        nslots * slot_lds<F>(Q) + red_bytes(16, Q) <= lds &&
+        2 * (nslots * slot_lds<F>(Q) + red_bytes(kWaves, Q)) > lds) {
+        const int64_t p = (nslots + kDepth - 1) / kDepth * kDepth;
+        *out = BatchShape{static_cast<int>(n), static_cast<int>(k), m, 0, static_cast<int>((tiles + 15) / 16),
+                          static_cast<int>(nslots), static_cast<int>(nslots), 1, static_cast<int>(p), 1, 16, 0};
+        return true;
     }
-    if (tid == 0) __hip_atomic_store(counters + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <class F, int Q, int D, int XP>
-hipError_t run(const void* w, const float* x, float* y, float* p, uint32_t* counters, int64_t n, int64_t k, int m,
-               int slots, int slices, int psteps, hipStream_t s) {
-    const int64_t tiles = (n + 15) / 16;
-    const dim3 grid(static_cast<unsigned>((tiles + kWaves - 1) / kWaves), static_cast<unsigned>(slices));
-    hipLaunchKernelGGL((k_gemv_batch<F, Q, D, XP>), grid, dim3(kThreads), batch_lds_bytes<F>(psteps, Q), s,
-                       static_cast<const uint8_t*>(w), x, y, p, counters, static_cast<int>(n), static_cast<int>(k), m,
-                       slots, psteps);
-    return hipGetLastError();
-}
-
-template <class F, int Q, int D>
-hipError_t run_d(const void* w, const float* x, float* y, float* p, uint32_t* counters, int64_t n, int64_t k, int m,
-                 int per, int slices, hipStream_t s) {
-    const int psteps = per * F::kSteps;
-    const int xp = static_cast<int>((static_cast<int64_t>(psteps) * m * 4 + kThreads - 1) / kThreads);
-    if (xp <= 1) return run<F, Q, D, 1>(w, x, y, p, counters, n, k, m, per, slices, psteps, s);
-    if (xp <= 2) return run<F, Q, D, 2>(w, x, y, p, counters, n, k, m, per, slices, psteps, s);
-    return run<F, Q, D, 4>(w, x, y, p, counters, n, k, m, per, slices, psteps, s);
+    double cost = -1.0;
+    const int fs = tune_param("BATCH_SLICES", 0), fk = tune_param("BATCH_KS", -1);
+    for (int64_t slices = 1; slices <= (sliced ? 8 : 1); ++slices) {
+        if (slices > 1 && (slices < cmin || slices > nslots)) continue;
+        if (fs && slices != fs) continue;
+        const int64_t nchunks = slices > 1 ? slices : cmin;
+        const int64_t cs = (nslots + nchunks - 1) / nchunks;
+        if (cs * (nchunks - 1) >= nslots) continue;  // an empty last chunk
+        const int64_t occ = two_fit<F>(cs, m, Q) ? 2 : 1;
+        for (int lg = 0; lg <= 3; ++lg) {
+            if (fk >= 0 && lg != fk) continue;
+            const int64_t groups = (tiles + (kWaves >> lg) - 1) / (kWaves >> lg);
+            if (slices > 1 && (groups > static_cast<int64_t>(kArrivalCounters) || groups * slices > occ * cus)) continue;
+            const double share = slices > 1 && groups * slices > cus ? (F::kInt ? (Q == 1 ? 1.2 : 1.5) : 1.7) : 1.0;
+            const double rounds = slices > 1 ? 1.0 : static_cast<double>((groups + cus - 1) / cus);
+            const double stage = 1.3 * static_cast<double>(cs * F::kSteps * 32 * m) / 1024.0;
+            const double slot = F::kInt ? (Q == 1 ? 7.0 : 9.0) : 6.0, again = F::kInt ? 12.0 : 20.0;
+            const double merge = (F::kInt ? 14.0 : 15.0) + (F::kInt && Q == 2 ? 6.0 : 5.0) * static_cast<double>(slices);
+            const double per = static_cast<double>((cs + (1 << lg) - 1) >> lg);
+            const double restage = nchunks > 1 ? rounds * static_cast<double>(nchunks) : 1.0;
+            double t = slices > 1 ? share * (stage + per * slot) + merge
+                                  : restage * (stage + again) - again + rounds * static_cast<double>(nchunks) * per * slot;
+            if (lg) t += 3.0 * rounds;
+            if (cost >= 0.0 && t >= cost) continue;
+            cost = t;
+            int64_t p = (cs + (1 << lg) - 1) >> lg;
+            p = (p + kDepth - 1) / kDepth * kDepth;
+            *out = BatchShape{static_cast<int>(n),      static_cast<int>(k),  m, lg, static_cast<int>(groups),
+                              static_cast<int>(nslots), static_cast<int>(cs), static_cast<int>(nchunks),
+                              static_cast<int>(p),      static_cast<int>(slices), kWaves, 0};
+        }
+    }
+    return cost >= 0.0;
 }
 
 template <class F, int Q>
-hipError_t run_q(const void* w, const float* x, float* y, float* p, uint32_t* counters, int64_t n, int64_t k, int m,
-                 int per, int slices, hipStream_t s) {
-    const int dmax = tune_param("BATCH_DMAX", 1);
-    if (per % 4 == 0 && dmax >= 4) return run_d<F, Q, 4>(w, x, y, p, counters, n, k, m, per, slices, s);
-    if (per % 2 == 0 && dmax >= 2) return run_d<F, Q, 2>(w, x, y, p, counters, n, k, m, per, slices, s);
-    return run_d<F, Q, 1>(w, x, y, p, counters, n, k, m, per, slices, s);
-}
-
-// Slots per slice: what the LDS budget holds and XP <= 4 registers of x per
-// thread cover; among those, the least estimated time
-//     rounds of workgroups over the CUs * kSlotCost * slots per slice
-//     + slices (the last workgroup's reduction reads one partial per slice),
-// ties to the longer slice.  Candidates are the shortest slice for each
-// slice count.  (Fitted to times measured at N x K = 3072x3072, 8192x3072,
-// 3072x8192 (Q4_K), 3072x8192 and 1024x3072 (BF16), M = 2 and 8.)
-// The ring depth: one slot.  Deeper rings (2, 4 slots, selectable for
-// measurement) measured slower at those shapes -- their registers cost
-// resident workgroups, and other waves hide a slot's load better.
-template <class F>
-bool plan(int64_t n, int64_t k, int m, int64_t* per_out, int64_t* slices_out) {
-    const int q = (m + 3) / 4;
-    const int64_t total_slots = (k + F::kSteps * 32 - 1) / (F::kSteps * 32);
-    const int64_t groups = ((n + 15) / 16 + kWaves - 1) / kWaves;
-    const int64_t cus = device_info().cus;
-    const size_t budget = static_cast<size_t>(tune_param("BATCH_LDS", 65536));
-    auto fits = [&](int64_t per) {
-        const int64_t ps = per * F::kSteps;
-        return batch_lds_bytes<F>(static_cast<int>(ps), q) <= budget && ps * m * 4 <= 4 * static_cast<int64_t>(kThreads);
-    };
-    if (!fits(1)) return false;
-    int64_t per = 1, best = -1, prev = 0;
-    for (int64_t sl = 1; sl <= total_slots; ++sl) {
-        const int64_t c = (total_slots + sl - 1) / sl;
-        if (c == prev || !fits(c)) continue;
-        prev = c;
-        const int64_t cost = (groups * sl + cus - 1) / cus * F::kSlotCost * c + sl;
-        if (best < 0 || cost < best) {
-            best = cost;
-            per = c;
-        }
-    }
-    const int forced = tune_param("BATCH_SLOTS", 0);
-    if (forced > 0 && fits(forced)) per = forced;
-    *per_out = per;
-    *slices_out = (total_slots + per - 1) / per;
-    return true;
-}
-
-template <class F>
-hipError_t dispatch(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, hipStream_t s) {
-    const int q = (m + 3) / 4;
-    const int64_t groups = ((n + 15) / 16 + kWaves - 1) / kWaves;
-    int64_t per = 0, slices = 0;
-    if (!plan<F>(n, k, m, &per, &slices)) return hipErrorInvalidValue;
-
+hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, int64_t sc_off, hipStream_t s) {
+    BatchShape S;
+    if (!plan<F, Q>(n, k, m, true, &S)) return hipErrorInvalidValue;
     float* part = nullptr;
     uint32_t* counters = nullptr;
-    if (slices > 1) {
-        if (groups > static_cast<int64_t>(kArrivalCounters)) return hipErrorInvalidValue;
+    if (S.slices > 1) {
+        // Without scratch (it may not grow under a stream capture) K stays
+        // inside the workgroups.
         hipError_t e;
         counters = arrival_counters(s, &e);
-        if (!counters) return e;
-        part = static_cast<float*>(workspace(static_cast<size_t>(slices) * m * n * sizeof(float), s, &e));
-        if (!part) return e;
+        if (counters)
+            part = static_cast<float*>(workspace(static_cast<size_t>(S.slices) * m * n * sizeof(float), s, &e));
+        if (!part && !plan<F, Q>(n, k, m, false, &S)) return hipErrorInvalidValue;
     }
-    const int sl = static_cast<int>(per), nsl = static_cast<int>(slices);
-    if (q == 1) return run_q<F, 1>(w, x, y, part, counters, n, k, m, sl, nsl, s);
-    return run_q<F, 2>(w, x, y, part, counters, n, k, m, sl, nsl, s);
+    S.sc_off = sc_off;
+    const size_t lds = static_cast<size_t>(S.cslots) * slot_lds<F>(Q) + red_bytes(S.waves, Q);
+    // Two workgroups per CU where they fit; BF16 streams as fast from one
+    // (65536 x 2560, M = 4: 62.6 us against 66.1).
+    const int64_t slots =
+        (F::kInt && S.waves == kWaves && two_fit<F>(S.cslots, m, Q) ? 2 : 1) * static_cast<int64_t>(device_info().cus);
+    const dim3 grid(static_cast<unsigned>(S.slices > 1 || S.groups < slots ? S.groups : slots),
+                    static_cast<unsigned>(S.slices));
+    const int threads = S.waves * kWave;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(static_cast<unsigned>(threads)), lds, s, static_cast<const uint8_t*>(w), x, S.k, S.m, S.n,
+                           S.ks_log, S.cslots, S.nslots, S.groups, S.per, y, S.nchunks, S.sc_off, part, counters);
+        return hipGetLastError();
+    };
+    const int xp = static_cast<int>((static_cast<int64_t>(S.cslots) * F::kSteps * 4 * m + threads - 1) / threads);
+    if constexpr (F::kInt && Q == 2) {
+        if (S.waves == 16) return go(k_gemv_batch<F, Q, 4, 16>);
+    }
+    if (xp <= 2) return go(k_gemv_batch<F, Q, 2, kWaves>);
+    if (xp <= 4) return go(k_gemv_batch<F, Q, 4, kWaves>);
+    return go(k_gemv_batch<F, Q, 8, kWaves>);
+}
+
+template <class F>
+hipError_t dispatch(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, int64_t sc_off,
+                    hipStream_t s) {
+    return m <= 4 ? run<F, 1>(w, x, y, n, k, m, sc_off, s) : run<F, 2>(w, x, y, n, k, m, sc_off, s);
+}
+
+template <class F>
+size_t workspace_of(int64_t n, int64_t k, int m) {
+    BatchShape S;
+    const bool ok = m <= 4 ? plan<F, 1>(n, k, m, true, &S) : plan<F, 2>(n, k, m, true, &S);
+    return ok && S.slices > 1 ? static_cast<size_t>(S.slices) * m * n * sizeof(float) : 0;
 }
 
 }  // namespace
 
 size_t gemv_batch_workspace_bytes(int fmt, int64_t n, int64_t k, int m) {
     if (m < 2 || m > 8) return 0;
-    int64_t per = 0, slices = 0;
-    const bool ok = fmt == RT_HIP_Q4K ? plan<BQ4k>(n, k, m, &per, &slices)
-                                      : (fmt == RT_HIP_BF16 ? plan<BBf16>(n, k, m, &per, &slices) : false);
-    return ok && slices > 1 ? static_cast<size_t>(slices) * m * n * sizeof(float) : 0;
+    switch (fmt) {
+        case RT_HIP_Q4K: return workspace_of<BQ4k>(n, k, m);
+        case RT_HIP_BF16: return workspace_of<BBf16>(n, k, m);
+        case RT_HIP_Q4_0: return workspace_of<BQ40>(n, k, m);
+        case RT_HIP_Q4MAT: return workspace_of<BQ4m>(n, k, m);
+    }
+    return 0;
 }
 
 hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, int64_t n, int64_t k, int m,
                              hipStream_t s) {
-    if (m < 2 || m > 8) return hipErrorInvalidValue;
-    if (fmt == RT_HIP_Q4K) return dispatch<BQ4k>(w, x, y, n, k, m, s);
-    if (fmt == RT_HIP_BF16) return dispatch<BBf16>(w, x, y, n, k, m, s);
+    if (m < 1 || m > 8) return hipErrorInvalidValue;
+    switch (fmt) {
+        case RT_HIP_Q4K: return dispatch<BQ4k>(w, x, y, n, k, m, 0, s);
+        case RT_HIP_BF16: return dispatch<BBf16>(w, x, y, n, k, m, 0, s);
+        case RT_HIP_Q4_0: return dispatch<BQ40>(w, x, y, n, k, m, 0, s);
+        case RT_HIP_Q4MAT:
+            return dispatch<BQ4m>(w, x, y, n, k, m, static_cast<int64_t>(q4mat_scales_offset(n, k)), s);
+    }
     return hipErrorInvalidValue;
 }
 

@@ -81,31 +81,26 @@ __device__ __forceinline__ void sub_block_scale(float amax, float& s, float& inv
 
 // The three limb words (planes A0, A1, A2; value e in byte e) of four
 // activations of one sub-block, inv = 1/s.  |v * inv| < 64 and the scaling
-// is exact, so b = v * inv * 2^16 + 1.5 * 2^23 is rounded once, to the
-// nearest integer, and its bits are 0x4B400000 + R with R = rint(v/s * 2^16),
-// |R| < 2^22.  The signed base-256 digits of R are then bytes of b:
-//     A2 = R mod 256 (as int8)          = byte 0 of b
-//     A1 = ((R + 128) >> 8) mod 256     = byte 1 of b + 128
-//     A0 = (R + 32896) >> 16            = byte 2 of b + 0x8080 - 0x400000
-// (the last subtracts the magic's own 0x40 in bits 16..23), so that
-// R = 65536 A0 + 256 A1 + A2 with |A0| <= 64.  v_perm gathers each plane.
+// is exact, so v * inv * 2^16 + 1.5 * 2^23 is rounded once, to the nearest
+// integer, and its bits are 0x4B400000 + R with R = rint(v/s * 2^16),
+// |R| <= 2^22.  With 0x8080 added, as an integer, the bytes are the digits of
+// R in base 256 with each low digit biased by 128:
+//     A2 = byte 0 - 128, A1 = byte 1 - 128 (as int8: the byte with bit 7 flipped),
+//     A0 = byte 2 - 64 (bytes 0..128: + 64 carries into no neighbour, then the flip),
+// so that R = 65536 A0 + 256 A1 + A2 with |A0| <= 64.  v_perm gathers each plane.
 __device__ __forceinline__ void limb_words(const f32x4 v, float inv, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
-    uint32_t b[4], m[4], h[4];
+    uint32_t b[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        b[e] = __float_as_uint(__builtin_fmaf(v[e] * inv, 65536.0f, 12582912.0f));
-        m[e] = b[e] + 128u;
-        h[e] = b[e] - 4161408u;  // + 0x8080 - 0x400000
-    }
+    for (int e = 0; e < 4; ++e)
+        b[e] = __float_as_uint(__builtin_fmaf(v[e] * inv, 65536.0f, 12582912.0f)) + 0x8080u;
     // perm(hi, lo, sel): byte j of the result is byte sel_j of {hi:lo}
-    auto gather = [](const uint32_t (&x)[4], uint32_t byte) {
-        const uint32_t pair = 0x0c0c0400u | (byte * 0x0101u);
-        return __builtin_amdgcn_perm(__builtin_amdgcn_perm(x[3], x[2], pair),
-                                     __builtin_amdgcn_perm(x[1], x[0], pair), 0x05040100u);
-    };
-    w0 = gather(h, 2);
-    w1 = gather(m, 1);
-    w2 = gather(b, 0);
+    const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);  // bytes 0 of both, then bytes 1
+    const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
+    const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0602u);  // bytes 2
+    const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0602u);
+    w2 = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
+    w1 = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
+    w0 = (__builtin_amdgcn_perm(h23, h01, 0x05040100u) + 0x40404040u) ^ 0x80808080u;
 }
 
 // Limbs of 4 activations (one f32x4) of a sub-block whose 8 holders are the

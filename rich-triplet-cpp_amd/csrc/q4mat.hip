@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kT) void k_gemv_q4mat(const uint8_t* __restrict__ P
 
 template <int M>
 hipError_t run_gemv(const uint8_t* p, const float* sc, const float* x, float* y, int64_t n, int64_t k, hipStream_t s) {
-    const size_t lds = q4mat_gemv_lds_bytes(M, k);
+    const size_t lds = q4mat_gemv_lds_bytes(k);
     const int64_t waves = kT / kWave;
     const int64_t cus = device_info().cus;
     int64_t wgs = (n + waves - 1) / waves;
@@ -223,24 +223,11 @@ size_t q4mat_bytes(int64_t n, int64_t k) {
     return q4mat_scales_offset(n, k) + static_cast<size_t>((n * k + 31) / 32) * 4;
 }
 
-size_t q4mat_gemv_lds_bytes(int m, int64_t k) {
-    return static_cast<size_t>(m) * (static_cast<size_t>(k) * 4 + static_cast<size_t>(k / 32) * 4);
-}
+size_t q4mat_gemv_lds_bytes(int64_t k) { return static_cast<size_t>(k) * 4 + static_cast<size_t>(k / 32) * 4; }
 
-hipError_t launch_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, hipStream_t s) {
+hipError_t launch_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_t k, hipStream_t s) {
     const auto* p = static_cast<const uint8_t*>(w);
-    const auto* sc = reinterpret_cast<const float*>(p + q4mat_scales_offset(n, k));
-    switch (m) {
-        case 1: return run_gemv<1>(p, sc, x, y, n, k, s);
-        case 2: return run_gemv<2>(p, sc, x, y, n, k, s);
-        case 3: return run_gemv<3>(p, sc, x, y, n, k, s);
-        case 4: return run_gemv<4>(p, sc, x, y, n, k, s);
-        case 5: return run_gemv<5>(p, sc, x, y, n, k, s);
-        case 6: return run_gemv<6>(p, sc, x, y, n, k, s);
-        case 7: return run_gemv<7>(p, sc, x, y, n, k, s);
-        case 8: return run_gemv<8>(p, sc, x, y, n, k, s);
-        default: return hipErrorInvalidValue;
-    }
+    return run_gemv<1>(p, reinterpret_cast<const float*>(p + q4mat_scales_offset(n, k)), x, y, n, k, s);
 }
 
 hipError_t launch_dequant_4bit(int fmt, const void* w, void* out, bool bf16, int64_t n, int64_t k, hipStream_t s) {

@@ -40,11 +40,6 @@ void* workspace(size_t bytes, hipStream_t s, hipError_t* err);
 constexpr size_t kArrivalCounters = 16384;
 uint32_t* arrival_counters(hipStream_t s, hipError_t* err);
 
-// Largest M*K the GEMV kernels stage in LDS (f32 activations + 16-value sums).
-size_t gemv_lds_bytes(int fmt, int m, int64_t k);
-
-hipError_t launch_gemv_q4k(const void* w, const float* x, float* y, int64_t n, int64_t k,
-                           int m, hipStream_t s);
 hipError_t launch_gemv_q4k_mfma(const void* w, const float* x, float* y, int64_t n, int64_t k,
                                 hipStream_t s);
 // Up to four M = 1 Q4_K GEMVs sharing x, K; `tiled`: the weights are in the
@@ -132,21 +127,19 @@ hipError_t launch_gemv_q4k_bf16_fused(int count, const void* const* w, float* co
                                       float eps = 0.0f, const float* inv_freq = nullptr, int pos = 0,
                                       int head_dim = 0, int rope_jobs = 0, const RopeCache& cache = {});
 
-hipError_t launch_gemv_bf16(const uint16_t* w, const float* x, float* y, int64_t n, int64_t k,
-                            int m, uint64_t* argmax_key, hipStream_t s);
 // M = 1 BF16 GEMV (gemv_bf16.hip); `key` (may be null) receives the fused
 // argmax.  LDS: bf16_m1_lds_bytes(k).
 size_t bf16_m1_lds_bytes(int64_t k);
 hipError_t launch_gemv_bf16_m1(const uint16_t* w, const float* x, float* y, int64_t n, int64_t k,
                                uint64_t* key, hipStream_t s);
-hipError_t launch_gemv_q4_0(const void* w, const float* x, float* y, int64_t n, int64_t k,
-                            int m, hipStream_t s);
-// Batched GEMV, 2 <= m <= 8, Q4_K (K % 256 == 0) or BF16 (K % 8 == 0) on
-// bf16 MFMA (gemv_batch.hip): every weight byte is read once for all m rows;
-// K-slices beyond the LDS budget are summed through the library workspace.
+// Batched GEMV, m <= 8, Q4_K or Q4_0 (K % 256 == 0), Q4Mat (K % 32 == 0) or
+// BF16 (K % 8 == 0) on the matrix cores (gemv_batch.hip): every weight byte
+// is read once for all m rows.  Long K at several rows is split over
+// workgroups through the library workspace where that has (or may grow to)
+// the room.
 hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, int64_t n, int64_t k, int m,
                              hipStream_t s);
-// Workspace bytes one launch_gemv_batch call needs (0 when K fits one slice).
+// Workspace bytes one launch_gemv_batch call takes when they are there.
 size_t gemv_batch_workspace_bytes(int fmt, int64_t n, int64_t k, int m);
 // M = 1 GGUF Q4_0 GEMV (gemv_q40.hip); LDS q40_m1_lds_bytes(k).
 size_t q40_m1_lds_bytes(int64_t k);
@@ -196,13 +189,13 @@ hipError_t launch_gemv_q4k_q8(const void* w, bool tiled, const float* x, float* 
                               hipStream_t s);
 
 // Q4Mat (q4mat.hip): one buffer of packed nibbles then f32 scales at
-// q4mat_scales_offset; K % 32 == 0.  The M <= 8 GEMV stages x [M][K] in LDS
+// q4mat_scales_offset; K % 32 == 0.  The M = 1 GEMV stages x in LDS
 // (q4mat_gemv_lds_bytes).  launch_dequant_4bit: Q4Mat or GGUF Q4_0 -> bf16
 // or f32 [N, K].
 size_t q4mat_scales_offset(int64_t n, int64_t k);
 size_t q4mat_bytes(int64_t n, int64_t k);
-size_t q4mat_gemv_lds_bytes(int m, int64_t k);
-hipError_t launch_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, hipStream_t s);
+size_t q4mat_gemv_lds_bytes(int64_t k);
+hipError_t launch_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_t k, hipStream_t s);
 hipError_t launch_dequant_4bit(int fmt, const void* w, void* out, bool bf16, int64_t n, int64_t k, hipStream_t s);
 
 // ---- decode-step operations (decoder_ops.hip) ----------------------------------

@@ -1,0 +1,122 @@
+"""Batched GEMV (M = 2..8) of every weight format at the edges of its launch
+shapes: row tiles of 16 and their remainders, K of one slot, of odd slot
+counts, and of partial slots where a format allows them (BF16 K % 8, Q4Mat
+K % 32), K staged in one chunk, in several, and split over workgroups, and
+outputs long enough for workgroups that walk several tile groups.
+
+Reference: float64 products of the dequantized weights (the oracle's
+decoders).  Bound, per row of y: the activation limbs of the 4-bit formats
+are within 2.5e-7 of a block's absmax (q4k_mfma.hpp) and f32 sums round by
+2^-24 a step, so each output is within 4e-7 * sum|w x|-like terms; taken
+normwise over the output that is below 1e-5 at every size here, the bound
+the single-row GEMVs are held to.
+"""
+import numpy as np
+import pytest
+
+from helpers import GEMV_TOL, f32_to_bf16_rne, bf16_bits_to_f32, from_dev, normwise_err, say, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def weights(rt, orc, fmt, rng, n, k):
+    """(device bytes, float64 values) of a random weight in `fmt`."""
+    if fmt == "q4mat":
+        packed = rng.integers(0, 256, n * k // 2, dtype=np.uint8)
+        scales = (0.002 + 0.004 * rng.random(n * k // 32)).astype(np.float32)
+        nib = np.stack([packed & 15, packed >> 4], -1).reshape(-1).astype(np.int64)
+        v = np.where(nib > 7, nib - 16, nib) * np.repeat(scales.astype(np.float64), 32)
+        return rt.q4mat_upload(packed, scales, n, k), v.reshape(n, k)
+    if fmt == "q4_0":
+        b = rng.integers(0, 256, (n * k // 32, 18), dtype=np.uint8)
+        b[:, :2] = (0.002 + 0.004 * rng.random(b.shape[0])).astype(np.float16)[:, None].view(np.uint8)
+        d = b[:, :2].copy().view(np.float16).astype(np.float64)
+        q = np.concatenate([b[:, 2:] & 15, b[:, 2:] >> 4], 1).astype(np.float64) - 8
+        return to_dev(b.reshape(-1)), (d * q).reshape(n, k)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    if fmt == "bf16":
+        bits = f32_to_bf16_rne(w)
+        return to_dev(bits), bf16_bits_to_f32(bits).astype(np.float64).reshape(n, k)
+    blocks = orc.q4k_quantize(w)
+    return to_dev(blocks), orc.q4k_dequant(blocks, n, k).astype(np.float64)
+
+
+def run(rt, fmt, w, x, n, k):
+    code = {"q4k": rt.Q4K, "bf16": rt.BF16, "q4_0": rt.Q4_0, "q4mat": rt.Q4MAT}[fmt]
+    return from_dev(rt.gemv(code, w, to_dev(x), n, k))
+
+
+SHAPES = [(1, 256, 2), (15, 512, 3), (17, 768, 4), (129, 1280, 5), (300, 2816, 8), (48, 12032, 4), (40, 8448, 7),
+          (4112, 256, 8)]
+TAILS = {"bf16": [(33, 8, 2), (70, 1160, 5)], "q4mat": [(33, 32, 2), (70, 1184, 5)]}
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "bf16", "q4_0", "q4mat"])
+def test_batched_gemv_edges(rt, orc, fmt):
+    for n, k, m in SHAPES + TAILS.get(fmt, []):
+        say(f"[gemv batch {fmt}] {n} x {k}, M = {m}")
+        rng = np.random.default_rng(n + k + m)
+        w, v = weights(rt, orc, fmt, rng, n, k)
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        x[-1] *= np.float32(1e-20)  # rows keep scales of their own
+        y = run(rt, fmt, w, x, n, k)
+        for r in range(m):
+            want = v @ x[r].astype(np.float64)
+            scale = np.abs(v) @ np.abs(x[r].astype(np.float64))
+            assert np.max(np.abs(y[r] - want)) <= GEMV_TOL * np.max(scale), (fmt, n, k, m, r)
+        assert np.array_equal(y, run(rt, fmt, w, x, n, k))  # the order of sums is fixed
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q4_0", "q4mat"])
+def test_batched_gemv_long_output(rt, orc, fmt):
+    """Outputs of several rounds of workgroups: M = 8 (16-wave workgroups) and M = 3, rows checked throughout."""
+    import torch
+    n, k = 70001, 2560
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rng = np.random.default_rng(3)
+    base, v = weights(rt, orc, fmt, rng, 512, k)
+    if fmt == "q4mat":  # the same 512 rows over and over: packed bytes, then scales
+        off = rt.library().lib.rt_hip_q4mat_scales_offset(512, k)
+        reps = -(-n // 512)
+        pk, sc = base[:512 * k // 2].reshape(512, -1), base[off:off + 512 * k // 8].reshape(512, -1)
+        buf = torch.zeros(rt.q4mat_bytes(n, k), dtype=torch.uint8, device="cuda")
+        buf[:n * k // 2] = pk.repeat(reps, 1)[:n].reshape(-1)
+        o = rt.library().lib.rt_hip_q4mat_scales_offset(n, k)
+        buf[o:o + n * k // 8] = sc.repeat(reps, 1)[:n].reshape(-1)
+        w = buf
+    else:
+        w = base.reshape(512, -1).repeat(-(-n // 512), 1)[:n].reshape(-1).contiguous()
+    x = torch.randn((8, k), device="cuda", generator=g).cpu().numpy()
+    for m in (3, 8):
+        say(f"[gemv batch {fmt}] {n} x {k}, M = {m}")
+        y = run(rt, fmt, w, x[:m], n, k)
+        want = (x[:m].astype(np.float64) @ v.T)
+        assert normwise_err(y[:, :512], want) <= GEMV_TOL
+        for r0 in range(512, n, 512):  # every other copy of the rows gives the same sums
+            r1 = min(n, r0 + 512)
+            assert np.array_equal(y[:, r0:r1], y[:, :r1 - r0]), r0
+
+
+def test_batched_gemv_without_workspace_room(rt, orc):
+    """A shape that is split over workgroups, captured without room to grow the
+    workspace, keeps K inside its workgroups: accepted, and right."""
+    import torch
+    lib = rt.library().lib
+    m, k = 8, 12288
+    n = 64
+    while lib.rt_hip_gemv_workspace_bytes(rt.Q4_0, n, k, m) <= rt.workspace_bytes() and n < 4096:
+        n *= 2
+    rng = np.random.default_rng(5)
+    w, v = weights(rt, orc, "q4_0", rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    dx, y = to_dev(x), torch.zeros((m, n), device="cuda")
+    say(f"[gemv batch] Q4_0 {n} x {k} captured, workspace {rt.workspace_bytes()} bytes")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rt.gemv(rt.Q4_0, w, dx, n, k, y=y)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert normwise_err(from_dev(y), x.astype(np.float64) @ v.T) <= GEMV_TOL
