@@ -925,14 +925,21 @@ int rt_hip_gemm(int32_t format, const void* a, int32_t a_dtype, const void* w, c
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (gemm_dequant_in_kernel(format, a_dtype == RT_HIP_BF16, m, n, k))  // decoded inside the GEMM
         return check_stream_launch(launch_gemm(format, a, a_dtype == RT_HIP_BF16, w, bias, c, m, n, k, s), fn);
-    const size_t own = (gemm_workspace_bytes(RT_HIP_BF16, a_dtype == RT_HIP_BF16, m, n, k) + 255) / 256 * 256;
+    size_t own = (gemm_workspace_bytes(RT_HIP_BF16, a_dtype == RT_HIP_BF16, m, n, k) + 255) / 256 * 256;
     hipError_t e;
     auto* ws = static_cast<uint8_t*>(workspace(own + static_cast<size_t>(n * k) * 2, s, &e));
+    bool scratch = true;
+    if (!ws && k % 256 != 0) {  // room for the widened weight alone will do
+        own = 0;
+        scratch = false;
+        ws = static_cast<uint8_t*>(workspace(static_cast<size_t>(n * k) * 2, s, &e));
+    }
     if (!ws) return check_stream_launch(e, fn);
     uint16_t* wb = reinterpret_cast<uint16_t*>(ws + own);
     e = launch_dequant_4bit(format, w, wb, true, n, k, s);
     if (e != hipSuccess) return hip_fail(e, fn);
-    return check_stream_launch(launch_gemm(RT_HIP_BF16, a, a_dtype == RT_HIP_BF16, wb, bias, c, m, n, k, s), fn);
+    return check_stream_launch(launch_gemm(RT_HIP_BF16, a, a_dtype == RT_HIP_BF16, wb, bias, c, m, n, k, s, scratch),
+                               fn);
 }
 
 int rt_hip_dequant(int32_t format, const void* w, void* out, int32_t out_dtype, int64_t n, int64_t k,

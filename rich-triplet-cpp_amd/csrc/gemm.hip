@@ -1,16 +1,8 @@
 // gemm.hip -- prefill / FLUX GEMM on bf16 MFMA (gfx950), C = A * W^T (+ bias).
 //
-// W is Q4_K blocks or bf16 [N, K]; A is f32 or bf16 [M, K]; C is f32 [M, N].
-// Operands are rounded to bf16 (RNE) where they enter LDS and contracted
-// with v_mfma_f32_16x16x32_bf16, f32 accumulation.  A Q4_K weight is
-// dequantized tile by tile straight into LDS (each K step of 64 values is
-// one 32-byte qs chunk of every row's super-block), so no dequantized copy
-// of the weight is ever written to HBM -- unlike the reference's FLUX path,
-// which dequantizes the whole weight into a scratch buffer before its GEMM
-// (src/metal_flux.mm:155-185).
-//
-// Block tile 128 x 128 x 64, 256 threads = 4 waves in 2 x 2, each wave a
-// 64 x 64 sub-tile of 4 x 4 MFMA 16x16 tiles.
+// W is Q4_K blocks, Q4Mat or GGUF Q4_0 storage, or bf16 [N, K]; A is f32 or
+// bf16 [M, K]; C is f32 [M, N].  Operands are rounded to bf16 (RNE) and
+// contracted with v_mfma_f32_16x16x32_bf16, f32 accumulation.
 //
 // MFMA operand layout: lane l supplies row (l % 16) of its A fragment and
 // column (l % 16) of its B fragment, 8 bf16 K-values each, the K slot being
@@ -33,9 +25,11 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
            (static_cast<uint32_t>(f32_to_bf16_rne(b)) << 16);
 }
 
-template <int WFMT, bool A_BF16>
-__global__ __launch_bounds__(256) void k_gemm(const void* __restrict__ Ap,
-                                              const void* __restrict__ Wp,
+// BF16 W without scratch: A converted as it enters LDS, no K split.  Runs
+// where the pipelined kernels' workspace cannot be had (a stream capture with
+// too little of it reserved) and K is not whole super-blocks.
+template <bool A_BF16>
+__global__ __launch_bounds__(256) void k_gemm(const void* __restrict__ Ap, const uint16_t* __restrict__ Wp,
                                               const float* __restrict__ bias,
                                               float* __restrict__ C, int M, int N, int K) {
     __shared__ __attribute__((aligned(16))) uint16_t sA[BM * LDS_STRIDE];
@@ -53,7 +47,6 @@ __global__ __launch_bounds__(256) void k_gemm(const void* __restrict__ Ap,
     // Staging roles: thread -> (row, 32-value half) of the 128 x 64 tiles.
     const int sr = tid >> 1, shalf = tid & 1;
     const int gm = m0 + sr, gn = n0 + sr;
-    const int nb = K >> 8;
 
     for (int k0 = 0; k0 < K; k0 += BK) {
         // ---- A tile: 32 values of row gm at k0 + 32*shalf -> bf16 in LDS.
@@ -85,52 +78,10 @@ __global__ __launch_bounds__(256) void k_gemm(const void* __restrict__ Ap,
             for (int j = 0; j < 4; ++j) dst[j] = out[j];
         }
         // ---- W tile.
-        if constexpr (WFMT == RT_HIP_Q4K) {
-            // Row gn, qs chunk c of super-block b, half shalf: 16 low-nibble
-            // values at k0 + 16*shalf and 16 high-nibble values 32 later.
-            u32x4 lo2[2], hi2[2];
-            if (gn < N) {
-                const int b = k0 >> 8, c = (k0 >> 6) & 3;
-                const uint8_t* bp = static_cast<const uint8_t*>(Wp) +
-                                    (static_cast<size_t>(gn) * nb + b) * kQ4kBlockBytes;
-                const u32x4 hd = ld16(bp);
-                const u32x4 q = ld16(bp + 16 + 32 * c + 16 * shalf);
-                const float d = f16_bits_to_f32(hd[0] & 0xffffu);
-                const float dm = f16_bits_to_f32(hd[0] >> 16);
-                uint32_t sv1, mv1, sv2, mv2;
-                decode_scale_min(make_scale_sel(2 * c), hd[1], hd[2], hd[3], sv1, mv1);
-                decode_scale_min(make_scale_sel(2 * c + 1), hd[1], hd[2], hd[3], sv2, mv2);
-                const float s1 = d * static_cast<float>(sv1), n1 = dm * static_cast<float>(mv1);
-                const float s2 = d * static_cast<float>(sv2), n2 = dm * static_cast<float>(mv2);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t w = q[j];
-                    float l[4], h[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const uint32_t byte = (w >> (8 * e)) & 0xffu;
-                        l[e] = s1 * static_cast<float>(byte & 0x0fu) - n1;
-                        h[e] = s2 * static_cast<float>(byte >> 4) - n2;
-                    }
-                    lo2[j >> 1][2 * (j & 1)] = pack_bf16x2(l[0], l[1]);
-                    lo2[j >> 1][2 * (j & 1) + 1] = pack_bf16x2(l[2], l[3]);
-                    hi2[j >> 1][2 * (j & 1)] = pack_bf16x2(h[0], h[1]);
-                    hi2[j >> 1][2 * (j & 1) + 1] = pack_bf16x2(h[2], h[3]);
-                }
-            } else {
-                lo2[0] = lo2[1] = hi2[0] = hi2[1] = u32x4{0u, 0u, 0u, 0u};
-            }
-            u32x4* dlo = reinterpret_cast<u32x4*>(sB + sr * LDS_STRIDE + 16 * shalf);
-            u32x4* dhi = reinterpret_cast<u32x4*>(sB + sr * LDS_STRIDE + 32 + 16 * shalf);
-            dlo[0] = lo2[0];
-            dlo[1] = lo2[1];
-            dhi[0] = hi2[0];
-            dhi[1] = hi2[1];
-        } else {
+        {
             u32x4 out[4];
             if (gn < N) {
-                const uint16_t* src = static_cast<const uint16_t*>(Wp) +
-                                      static_cast<size_t>(gn) * K + k0 + 32 * shalf;
+                const uint16_t* src = Wp + static_cast<size_t>(gn) * K + k0 + 32 * shalf;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) out[j] = ld16(src + 8 * j);
             } else {
@@ -182,7 +133,7 @@ __global__ __launch_bounds__(256) void k_gemm(const void* __restrict__ Ap,
 }
 
 // ---------------------------------------------------------------------------
-// Pipelined kernel (K % 256 == 0): bf16 A and W.
+// Pipelined kernel (K % 64 == 0): bf16 A and W.
 //
 // LDS tiles are 128 rows x 64 bf16 (128 B per row, unpadded) with the 16-byte
 // chunk c of row r stored at chunk slot c ^ (r & 7), so the MFMA fragment
@@ -371,8 +322,9 @@ __global__ __launch_bounds__(kPThreads) void k_gemm_pipe(const uint16_t* __restr
     // Step s: copy step t = s+kStages-1 (A, then W); MFMAs of step s; wait
     // for this wave's copies that step s+1 needs, then the barrier.  Copies
     // are ordered and counted by vmcnt: after W of step s+1 this wave has
-    // issued 16 more (A, W of s+2 and s+3).  kStages == 4 and S % 4 == 0:
-    // the unrolled round keeps every ring index a compile-time constant.
+    // issued 16 more (A, W of s+2 and s+3).  kStages == 4: the unrolled round
+    // keeps every ring index a compile-time constant, and steps past S copy
+    // zeros (empty ranges), which add nothing.
     static_assert(kStages == 4, "the unrolled round assumes a 4-stage ring");
     for (int s0 = 0; s0 < S; s0 += 4) {
 #pragma unroll
@@ -858,7 +810,7 @@ namespace {
 
 // How one GEMM call runs (shared by the launcher and the workspace query).
 struct GemmPlan {
-    bool pipe = false;  // pipelined MFMA kernels (k % 256 == 0, Q4_K or BF16 W)
+    bool pipe = false;  // pipelined MFMA kernels (BF16 W; 4-bit W with k % 256 == 0)
     bool big = false;   // 256 x 256 bf16 kernel
     bool ws = false;    // Q4_K W dequantized inside the GEMM by producer waves (k_gemm_ws)
     int splits = 1;     // split-K slices of the 128 x 128 kernels
@@ -869,7 +821,9 @@ struct GemmPlan {
 GemmPlan plan_gemm(int w_fmt, bool a_bf16, int64_t m, int64_t n, int64_t k) {
     GemmPlan p;
     const bool four_bit = w_fmt == RT_HIP_Q4MAT || w_fmt == RT_HIP_Q4_0;
-    p.pipe = k % 256 == 0 && (w_fmt == RT_HIP_Q4K || w_fmt == RT_HIP_BF16 || four_bit);
+    // Every BF16 K % 64 == 0 is whole 64-wide steps (a step count that is not a
+    // multiple of four runs up to three steps of zeros: 2 of 20 at K = 1152).
+    p.pipe = w_fmt == RT_HIP_BF16 || (k % 256 == 0 && (w_fmt == RT_HIP_Q4K || four_bit));
     if (!p.pipe) return p;
     // A Q4_K weight is dequantized (bf16, round-to-nearest-even of the exact
     // f32 value, as the reference's flux_dequant_q4k) either inside the GEMM
@@ -932,20 +886,24 @@ size_t gemm_workspace_bytes(int w_fmt, bool a_bf16, int64_t m, int64_t n, int64_
 }
 
 hipError_t launch_gemm(int w_fmt, const void* a, bool a_bf16, const void* w, const float* bias,
-                       float* c, int64_t m, int64_t n, int64_t k, hipStream_t s) {
+                       float* c, int64_t m, int64_t n, int64_t k, hipStream_t s, bool scratch) {
     if (k % BK) return hipErrorInvalidValue;
     const GemmPlan P = plan_gemm(w_fmt, a_bf16, m, n, k);
-    if (P.pipe) {
+    uint8_t* ws = nullptr;
+    bool pipe = P.pipe;
+    if (pipe && P.a_bytes + P.w_bytes + P.p_bytes) {
+        hipError_t e = hipErrorOutOfMemory;
+        if (scratch) ws = static_cast<uint8_t*>(workspace(P.a_bytes + P.w_bytes + P.p_bytes, s, &e));
+        if (!ws) {
+            if (k % 256 == 0) return e;
+            pipe = false;  // BF16 W, K not whole super-blocks: k_gemm needs no scratch
+        }
+    }
+    if (pipe) {
         const int64_t mt = P.mt, nt = P.nt, mt2 = P.mt2, nt2 = P.nt2;
         const bool big = P.big;
         const int splits = P.splits;
-        const size_t a_bytes = P.a_bytes, w_bytes = P.w_bytes, p_bytes = P.p_bytes;
-        uint8_t* ws = nullptr;
-        if (a_bytes + w_bytes + p_bytes) {
-            hipError_t e;
-            ws = static_cast<uint8_t*>(workspace(a_bytes + w_bytes + p_bytes, s, &e));
-            if (!ws) return e;
-        }
+        const size_t a_bytes = P.a_bytes, w_bytes = P.w_bytes;
         if (P.ws) {
             // Both roles of k_gemm_ws run the same number of barriers only if
             // each slice is whole super-blocks (S % 4 == 0).
@@ -1032,24 +990,14 @@ hipError_t launch_gemm(int w_fmt, const void* a, bool a_bf16, const void* w, con
         }
         return hipGetLastError();
     }
+    if (w_fmt != RT_HIP_BF16) return hipErrorInvalidValue;
     const dim3 grid(static_cast<unsigned>((n + BN - 1) / BN), static_cast<unsigned>((m + BM - 1) / BM));
-    if (w_fmt == RT_HIP_Q4K) {
-        if (a_bf16)
-            hipLaunchKernelGGL((k_gemm<RT_HIP_Q4K, true>), grid, dim3(256), 0, s, a, w, bias, c,
-                               static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
-        else
-            hipLaunchKernelGGL((k_gemm<RT_HIP_Q4K, false>), grid, dim3(256), 0, s, a, w, bias, c,
-                               static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
-    } else if (w_fmt == RT_HIP_BF16) {
-        if (a_bf16)
-            hipLaunchKernelGGL((k_gemm<RT_HIP_BF16, true>), grid, dim3(256), 0, s, a, w, bias, c,
-                               static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
-        else
-            hipLaunchKernelGGL((k_gemm<RT_HIP_BF16, false>), grid, dim3(256), 0, s, a, w, bias, c,
-                               static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
-    } else {
-        return hipErrorInvalidValue;
-    }
+    const auto* w16 = static_cast<const uint16_t*>(w);
+    const int im = static_cast<int>(m), in = static_cast<int>(n), ik = static_cast<int>(k);
+    if (a_bf16)
+        hipLaunchKernelGGL(k_gemm<true>, grid, dim3(256), 0, s, a, w16, bias, c, im, in, ik);
+    else
+        hipLaunchKernelGGL(k_gemm<false>, grid, dim3(256), 0, s, a, w16, bias, c, im, in, ik);
     return hipGetLastError();
 }
 

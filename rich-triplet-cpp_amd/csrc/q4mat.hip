@@ -1,5 +1,6 @@
 // q4mat.hip -- the reference's own 4-bit format, Q4Mat (include/rt/quant.hpp:
-// 23-75, src/quant_q4.cpp:17-156), on the GPU: the M <= 8 GEMV, and the
+// 23-75, src/quant_q4.cpp:17-156), on the GPU: the M = 1 GEMV (batches:
+// gemv_batch.hip), and the
 // dequantization to bf16 / f32 that the any-M GEMM and the parity tests use;
 // plus the GGUF Q4_0 dequantization for the same GEMM path.
 //

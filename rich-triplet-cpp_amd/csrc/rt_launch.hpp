@@ -256,8 +256,9 @@ hipError_t launch_gelu_mul(const float* gate, const float* up, float* out, int64
 hipError_t launch_swiglu(const float* gate, const float* up, float* out, int64_t n, hipStream_t s);
 hipError_t launch_add(const float* a, const float* b, float* out, int64_t n, hipStream_t s);
 
+// scratch false (BF16 W, k % 256 != 0): no library workspace.
 hipError_t launch_gemm(int w_fmt, const void* a, bool a_bf16, const void* w, const float* bias,
-                       float* c, int64_t m, int64_t n, int64_t k, hipStream_t s);
+                       float* c, int64_t m, int64_t n, int64_t k, hipStream_t s, bool scratch = true);
 // Whether launch_gemm dequantizes this 4-bit weight inside the GEMM (small
 // M, or wide N); otherwise a Q4Mat / Q4_0 caller dequantizes into the
 // workspace first.
