@@ -299,14 +299,16 @@ int rt_hip_attention_decode_noalloc(const float* q, const float* k_cache, const 
  * out_i = sum_j softmax(s)_j v_j.  head_dim must be a multiple of 8 in
  * [8, 128] (the Metal path's limits, metal_flux.mm:443-452; else
  * RT_HIP_E_SHAPE); t = 0 is a no-op.  Buffers 16-byte aligned; out must not
- * overlap q, k or v.  Products and sums in f32 (matrix cores, online softmax
+ * overlap q, k or v.  Products and sums to f32 accuracy (each f32 factor as
+ * three bf16 values that add up to it, on the matrix cores; online softmax
  * over tiles of 32 keys): results match the reference to f32 rounding and
- * are deterministic.  With more 128-query blocks (n_heads * ceil(t / 128))
- * than two per CU, the work is divided evenly over two workgroups per CU and
- * the blocks cut between two of them keep their partial states in the
- * library workspace (see above): rt_hip_flux_attention_workspace_bytes gives
- * the need for a shape (0 when none, -1 for invalid sizes), to reserve before
- * a graph capture. */
+ * are deterministic.  With more 256-query blocks (n_heads * ceil(t / 256))
+ * than CUs, the work is divided evenly over one workgroup per CU and the
+ * blocks cut between two of them keep their partial states in the library
+ * workspace (see above): rt_hip_flux_attention_workspace_bytes gives the need
+ * for a shape (0 when none, -1 for invalid sizes), to reserve before a graph
+ * capture; where it cannot be had the blocks stay whole, at the cost of a
+ * partly empty last round. */
 int rt_hip_flux_attention(const float* q, const float* k, const float* v, float* out, int64_t t, int32_t n_heads,
                           int32_t head_dim, rt_hip_stream stream);
 int64_t rt_hip_flux_attention_workspace_bytes(int64_t t, int32_t n_heads, int32_t head_dim);

@@ -537,10 +537,11 @@ int rt_hip_flux_attention(const float* q, const float* k, const float* v, float*
     float* part = nullptr;
     uint32_t* counters = nullptr;
     if (const size_t need = flux_attention_workspace(t, n_heads, head_dim)) {
+        // without scratch (it may not grow under a stream capture) the blocks
+        // stay whole
         part = static_cast<float*>(workspace(need, s, &e));
-        if (!part) return hip_fail(e, fn);
-        counters = arrival_counters(s, &e);
-        if (!counters) return hip_fail(e, fn);
+        counters = part ? arrival_counters(s, &e) : nullptr;
+        if (!counters) part = nullptr;
     }
     return check_stream_launch(launch_flux_attention(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s),
                                fn);

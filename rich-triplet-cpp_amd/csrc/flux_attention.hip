@@ -7,80 +7,142 @@
 // to 128 (the reference's limits, metal_flux.mm:443-452).
 // out[i][h] = sum_j softmax_j(scale * q_i . k_j) v_j for head h.
 //
-// A workgroup owns a block of 128 queries of one head (8 waves x 16) and
-// streams K and V once for all of them in tiles of 32 keys through a
-// two-stage LDS ring (2 x 32 KB at D = 128: two workgroups per CU): the
-// tiles are copied straight from memory into LDS by buffer loads (no
-// registers), the next tile's copy in flight while the current one is
-// used.  The products run in f32 on the matrix cores
-// (v_mfma_f32_16x16x4_f32), so every product and partial sum is an f32
-// operation, as in the reference:
-//  * S^T = K Q^T per 16-key x 16-query tile: lane (g = l/16, n = l%16)
-//    supplies K[key n][dim] and Q[query n][dim] for the same dim, so any
-//    assignment of dims to (k-step, lane group) is a valid contraction; dims
-//    16a + 4g + b over steps 4a + b let each lane read 4 consecutive dims
-//    with one 16-byte LDS read.  The result leaves lane (g, n) holding the
-//    scores of query n against keys 16t + 4g + r (t over the tile's two
-//    16-key halves).
-//  * Online softmax per query: the running maximum and denominator; the
-//    accumulator is rescaled by exp(m_old - m_new) before the tile is folded
-//    in (flux.msl:232-271).
-//  * O^T += V^T P^T: lane (g, n) supplies P[query n][key 16t + 4g + r] --
-//    exactly the score it holds -- and V[key 16t + 4g + r][dim 16c + n], so
-//    V stays key-major in LDS (as the copy writes it) and the result leaves
-//    lane (g, n) holding O[query n][dims 16c + 4g .. + 3]: its own query,
-//    rescaled by its own factor and stored as one 16-byte write.
+// A workgroup owns a block of 32 queries per wave (8 waves, 4 where the blocks
+// would leave CUs idle) of one head and streams K and V once for all of them
+// in tiles of 32 keys through LDS rings.
+//
+// f32 products on the bf16 matrix cores.  Every f32 factor is split into three
+// bf16 limbs with h + m + l == x exactly (24 bits of significand), and a
+// product is the six limb products hh, hm, mh, mm, hl, lh on
+// v_mfma_f32_32x32x16_bf16: products of bf16 values are exact in f32 and the
+// three left out (ml, lm, ll) are below 2^-25 of the product, under the
+// rounding of one f32 multiplication.  The matrix cores do a bf16 product at
+// 16 times the f32 rate, so six cost 3/8 of one f32 product.  Q's limbs live
+// in registers (split once per block), K's and V's are split as each tile is
+// staged, P's in the registers its scores were computed in:
+//  * S^T = K Q^T per 32-key x 32-query tile: lane (h = l/32, n = l%32) supplies
+//    K[key n] and Q[query n], dims 16a + 8h .. + 7 of step a; the result
+//    leaves lane (h, n) holding query n's scores against keys 8i + 4h + r
+//    (register 4i + r).  hh and the five corrections have accumulators of
+//    their own, added at the end.
+//  * Online softmax per query: the running maximum; each half of a query's
+//    keys keeps its own denominator (added at the end); the accumulator is
+//    rescaled by exp(m_old - m_new) where a maximum of the wave moved
+//    (flux.msl:232-271).
+//  * O^T += V^T P^T: lane (h, n) supplies P[query n] of the eight keys it
+//    holds in registers 8s .. 8s + 7 and V[those keys][dim 32c + n], which V's
+//    LDS rows (one per dim, keys in that order) hold as 16 bytes; the result
+//    leaves lane (h, n) holding O[query n][dims 32c + 8i + 4h + r].
+// From a tile of K or V that holds a value of 2^64 or more, an infinity or a
+// NaN, or throughout a block with a query of 2^55 or more, the block takes f32
+// MFMA steps on the values in memory: products that overflow and infinities
+// then behave as in f32 arithmetic (a limb's product could overflow to the
+// other sign).  A loop of its own: the limb loop has no registers to spare.
+//
 // The head is padded to DP in {32, 64, 128} dims with zeros (they add
 // nothing to a score and are never stored).  Keys past T are masked to -inf
-// (weight 0), their tile rows zero-filled by the copy's range check; query
-// rows past T are computed and not stored.  LDS rows are XOR-swizzled
-// (K by 16-byte granule, V by 16-dim block) so that the reads above hit
-// distinct banks; the copies apply the swizzle on the memory side.
+// (weight 0), their tile rows zero-filled by the loads' range check; query
+// rows past T are computed and not stored.
+//
+// Bound: the matrix cores.  A 32-key tile of a CU's 256 queries is 96 MFMAs a
+// wave, 6144 cycles a SIMD; between them come the softmax and the limb splits,
+// about 440 VALU instructions a wave and tile.  Measured at t = 4352, 24 heads
+// of 128: 2070 us with f32 MFMA (71% of that unit's peak, where 1480 us is the
+// least), 1250-1320 us with limbs: MFMA busy 57% at the 1.76 GHz the power limit
+// leaves (2.2 GHz when half idle).  Without the limb staging it would be 1075.
+// t = 1280: 230 -> 154 us; t = 2622, 18 x 88: 753 -> 355; t = 477, 13 x 128:
+// 88 -> 61; t = 466, 9 x 64: 38 -> 33; t = 100, 12 x 64: 12.6 -> 12.1.  The
+// normwise error against float64 at t = 4352 fell from 1.6e-6 to 8.7e-7.
+//  * Of the two waves of a SIMD one is in its products (priority 1) while the
+//    other does its softmax and staging, a barrier between phases: 1250 us;
+//    free-running waves 1410.
+//  * Tiles go through LDS copies of the raw f32 (no registers), are split once
+//    and read by all 8 waves: blocks of 128 queries halve the reuse of the
+//    splits and are taken only where 256 leave CUs idle.
 #include "rt_common.hpp"
 #include "rt_launch.hpp"
 
 namespace rt_hip {
 namespace {
 
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * kWave;
-constexpr int kBQ = 16 * kWaves;  // queries per workgroup
-constexpr int kBK = 32;           // keys per tile
-constexpr int kNT = kBK / 16;     // 16-key MFMA tiles per key tile
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kBK = 32;  // keys per tile
 constexpr float kLog2e = 1.44269504088896341f;
-constexpr uint32_t kNoRead = 0x7ffffff0u;  // past every tile's range: the copy writes zeros
+constexpr uint32_t kNoRead = 0x7ffffff0u;  // past every tile's range: reads zeros
 
 __device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
+// LDS: a ring of two tiles of K limbs [3][32 keys][DP] bf16, then one of three
+// tiles of V limbs [3][DP dims][32 keys], then each wave's share of a tile's
+// K and V as they are in memory, then the first tile without limbs.
 template <int DP>
-constexpr int stage_floats() {
-    return 2 * kBK * DP;  // K tile, then V tile
+constexpr int limb_plane() {
+    return 64 * DP;
 }
-template <int DP>
+// K units (key, 8 dims) and V units (4 keys, 1 dim) a thread stages: 4 DP and
+// 8 DP of them in all.
+constexpr int k_units(int dp, int nt) { return (4 * dp + nt - 1) / nt; }
+constexpr int v_units(int dp, int nt) { return (8 * dp + nt - 1) / nt; }
+template <int DP, int NW>
+constexpr int raw_wave_bytes() {  // per wave: 2 x 16 bytes a lane and K unit, 4 x 4 a lane and V unit
+    return 64 * (32 * k_units(DP, NW * 64) + 16 * v_units(DP, NW * 64));
+}
+template <int DP, int NW>
+constexpr int raw_bytes() {
+    return NW * raw_wave_bytes<DP, NW>();
+}
+template <int DP, int NW>
 constexpr size_t flux_lds_bytes() {
-    return static_cast<size_t>(2) * stage_floats<DP>() * 4;
+    return static_cast<size_t>(15) * limb_plane<DP>() + raw_bytes<DP, NW>() + 16;
 }
-
-// float offset of K[key][granule gr] (4 dims): granule slot gr ^ (key & mask)
+// 16-byte granule gr (8 dims) of a key's row: rows are exchanged granule-wise
+// so that the 16 lanes an LDS read serves together hit distinct banks.
 template <int DP>
 __device__ __forceinline__ int k_off(int key, int gr) {
-    constexpr int kMask = (DP / 4 < 16 ? DP / 4 : 16) - 1;
-    return key * DP + ((gr ^ (key & kMask)) << 2);
+    constexpr int kMask = DP / 8 - 1, kShift = DP == 128 ? 0 : (DP == 64 ? 1 : 2);
+    return key * (2 * DP) + ((gr ^ ((key >> kShift) & kMask & 15)) << 4);
 }
-// V[key][dim] sits at dim ^ v_sw(key): the 16-dim blocks of keys 4j .. 4j + 3
-// are exchanged by j (mod DP / 16, at most 4), so the four keys 4g + r
-// (g = 0..3) that one PV read touches fall in four different bank groups.
-template <int DP>
-__device__ __forceinline__ int v_sw(int key) {
-    constexpr int kMask = (DP / 16 < 4 ? DP / 16 : 4) - 1;
-    return ((key >> 2) & kMask) << 4;
+// 16-byte unit u = 2s + h of a dim's row: keys 16s + 4h + {0..3, 8..11}.
+__device__ __forceinline__ int v_off(int dim, int u) { return dim * 64 + ((u ^ ((dim >> 2) & 3)) << 4); }
+
+// Three bf16 limbs of a pair, packed: h + m + l == x for finite x that bf16
+// can hold (each residual is exact in f32).
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = bf16_pair(a, b);
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xffff0000u);
+    m = bf16_pair(ra, rb);
+    l = bf16_pair(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+}
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, u32x4& l) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t hh, mm, ll;
+        split2(v[2 * i], v[2 * i + 1], hh, mm, ll);
+        h[i] = hh;
+        m[i] = mm;
+        l[i] = ll;
+    }
+}
+// Adds the squares of a pair's high limbs to acc: NaN or infinite once one of
+// them is NaN or 2^64 or more in magnitude.  A sum that stays finite bounds
+// every value of K and V, and with |q| < 2^55 a score (128 products below
+// 2^119) and each of its limb products stays finite too.
+constexpr float kQLimit = 0x1p55f;
+__device__ __forceinline__ float limb_check(uint32_t h, float acc) {
+    const bf16x2 v = __builtin_bit_cast(bf16x2, h);
+    return __builtin_amdgcn_fdot2_f32_bf16(v, v, acc, false);
+}
+__device__ __forceinline__ bool not_finite(float x) { return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f800000u; }
+
+__device__ __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                   0);
 }
 
-// Partial states of a split query block: O [kBQ][DP], then m [kBQ], l [kBQ].
-template <int DP>
-constexpr int piece_floats() {
-    return kBQ * DP + 2 * kBQ;
-}
+// Partial states of a split query block: O [BQ][DP], then m [BQ], l [BQ].
+constexpr int piece_floats(int bq, int dp) { return bq * dp + 2 * bq; }
 
 // Stored and reloaded with agent-scope (device-coherent) accesses: they
 // bypass the per-XCD L2, so the workgroup that merges sees the other
@@ -93,6 +155,17 @@ __device__ __forceinline__ float ld_dev(const float* p) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// This wave's LDS reads and writes, or its copies into LDS, are done (and no
+// access moves across).
+__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void copies_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// The value of lane l ^ 32.
+__device__ __forceinline__ float other_half(float x, int h) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(h ? r[0] : r[1]);
+}
+
 // Work: item i = (head i / nqb, query block i % nqb) over key tiles
 // [0, ntile).  Without `part` workgroup (head, block) = (blockIdx.x,
 // blockIdx.y) does one whole item.  With it (more items than workgroup
@@ -102,29 +175,31 @@ __device__ __forceinline__ float ld_dev(const float* p) {
 // the boundary between workgroups w and w + 1 has two pieces: each stores
 // its state (o, m, l) in part[w][piece] and counts its arrival in cnt[w];
 // the second to arrive merges the two states and stores the output.
-// Two workgroups per CU (4 waves per SIMD): at most 128 VGPRs.
-template <int DP>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_flux_attn(
-    const float* __restrict__ Q, const float* __restrict__ K,
-                                                        const float* __restrict__ V, float* __restrict__ O, int T,
-                                                        int n_heads, int D, float scale, float* __restrict__ part,
-                                                        uint32_t* __restrict__ cnt, int per) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
+template <int DP, int NW>
+__global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux_attn(const float* __restrict__ Q, const float* __restrict__ K,
+                                                          const float* __restrict__ V, float* __restrict__ O, int T,
+                                                          int n_heads, int D, float scale, float* __restrict__ part,
+                                                          uint32_t* __restrict__ cnt, int per) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t arrival;
-    constexpr int NA = DP / 16;
-    constexpr int SF = stage_floats<DP>();
-    // Copy roles: a tile of one operand is DP / 8 instructions of 1 KB (64
-    // lanes x 16 bytes); wave w issues instructions w and w + 8.  Lane l of
-    // instruction j fills LDS granule 64 j + l = (key, slot) of the tile with
-    // the memory granule the swizzle puts there (offsets relative to the
-    // tile's first row, below 2^31 (key * stride * 4 < 32 * 2^26); dims past
-    // D read nothing).
-    constexpr int NI = DP / 8, CPW = (NI + kWaves - 1) / kWaves;
+    constexpr int NT = NW * kWave, BQ = 32 * NW;
+    constexpr int KS = DP / 16, NC = DP / 32;      // MFMA steps over the dims, 32-dim output blocks
+    constexpr int kPlane = limb_plane<DP>();
+    constexpr int KU = k_units(DP, NT), VU = v_units(DP, NT);
+    uint8_t* const ldsV = lds + 6 * kPlane;
+    int* const first_bad = reinterpret_cast<int*>(lds + 15 * kPlane + raw_bytes<DP, NW>());
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, g = lane >> 4;
+    const int n = lane & 31, h = lane >> 5;
+    uint8_t* const raw = lds + 15 * kPlane + wave * raw_wave_bytes<DP, NW>();
     const int64_t stride = static_cast<int64_t>(n_heads) * D;
-    const int ntile = (T + kBK - 1) / kBK, nqb = (T + kBQ - 1) / kBQ;
+    const int ntile = (T + kBK - 1) / kBK, nqb = (T + BQ - 1) / BQ;
+    // Two phases alternate: products (priority 1) and softmax + staging.  With
+    // 8 waves, w and w + 4 share a SIMD and the second group of four runs one
+    // phase behind the first, so that one wave of a SIMD has the matrix cores
+    // while the other has the VALU.
+    constexpr bool kTwo = NW == 8;
+    const bool second = kTwo && wave >= 4;
 
     // the units of this workgroup
     int64_t u, u_end;
@@ -141,134 +216,306 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const int t0 = static_cast<int>(u % ntile);
         const int t1 = static_cast<int>(min(static_cast<int64_t>(ntile), t0 + (u_end - u)));
         u += t1 - t0;
-        const int head = static_cast<int>(item / nqb), q0 = static_cast<int>(item % nqb) * kBQ;
+        const int head = static_cast<int>(item / nqb), q0 = static_cast<int>(item % nqb) * BQ;
         const float* kb = K + static_cast<int64_t>(head) * D;
         const float* vb = V + static_cast<int64_t>(head) * D;
-        auto copy_tile = [&](int tile, float* st) {
-            const int base = tile * kBK, rows = min(kBK, T - base);
+
+        // A tile's K and V, copied into the wave's own LDS (no registers) in a
+        // product phase; the limbs enter the rings in the phase after it.
+        const int vdim = tid % DP, vquad = tid / DP;
+        const uint32_t s4 = static_cast<uint32_t>(stride * 4);
+        auto load_tile = [&](int i0) {
+            const int base = (t0 + i0) * kBK, rows = min(kBK, T - base);
             const uint32_t bytes = static_cast<uint32_t>(((rows - 1) * stride + D) * 4);
             const BufRsrc rk = make_rsrc_n(kb + base * stride, bytes);
             const BufRsrc rv = make_rsrc_n(vb + base * stride, bytes);
 #pragma unroll
-            for (int i = 0; i < CPW; ++i) {
-                const int j = wave + kWaves * i;
-                if (j >= NI) break;  // wave-uniform
-                const int G = 64 * j + lane;
-                const int key = G / (DP / 4), slot = G % (DP / 4);
-                const int kd = 4 * (slot ^ (key & ((DP / 4 < 16 ? DP / 4 : 16) - 1)));
-                const int vd = (4 * slot) ^ v_sw<DP>(key);
-                const int row = key * static_cast<int>(stride);
-                const uint32_t koff = kd < D ? static_cast<uint32_t>((row + kd) * 4) : kNoRead;
-                const uint32_t voff = vd < D ? static_cast<uint32_t>((row + vd) * 4) : kNoRead;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rk, (__attribute__((address_space(3))) void*)(st + j * 256), 16, static_cast<int>(koff), 0, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rv, (__attribute__((address_space(3))) void*)(st + kBK * DP + j * 256), 16,
-                    static_cast<int>(voff), 0, 0, 0);
+            for (int i = 0; i < KU; ++i) {
+                const int id = tid + NT * i, key = id / (DP / 8), dim = 8 * (id % (DP / 8));
+                const uint32_t off = dim < D && key < kBK ? static_cast<uint32_t>(key) * s4 + 4 * dim : kNoRead;
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        rk, (__attribute__((address_space(3))) void*)(raw + (2 * i + j) * 1024), 16,
+                        static_cast<int>(off + 16u * j), 0, 0, 0);
             }
+            // (kNoRead plus up to 31 rows stays past the range and below 2^32)
+            const uint32_t off = vdim < D && vquad < 8 ? static_cast<uint32_t>(4 * vquad) * s4 + 4 * vdim : kNoRead;
+#pragma unroll
+            for (int i = 0; i < VU; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        rv, (__attribute__((address_space(3))) void*)(raw + KU * 2048 + (4 * i + j) * 256), 4,
+                        static_cast<int>(off + static_cast<uint32_t>(4 * i * (NT / DP) + j) * s4), 0, 0, 0);
+        };
+        auto stage_tile = [&](int i0) {
+            uint8_t* const sk = lds + (i0 & 1) * 3 * kPlane;
+            uint8_t* const sv = ldsV + (i0 % 3) * 3 * kPlane;
+            float bad = 0.0f;
+#pragma unroll
+            for (int i = 0; i < KU; ++i) {
+                const int id = tid + NT * i, key = id / (DP / 8), gr = id % (DP / 8);
+                if (KU * NT > 4 * DP && id >= 4 * DP) break;
+                const f32x4 x0 = *reinterpret_cast<const f32x4*>(raw + 2 * i * 1024 + lane * 16);
+                const f32x4 x1 = *reinterpret_cast<const f32x4*>(raw + (2 * i + 1) * 1024 + lane * 16);
+                const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+                u32x4 a, b, c;
+                split8(x, a, b, c);
+                uint8_t* const d = sk + k_off<DP>(key, gr);
+                *reinterpret_cast<u32x4*>(d) = a;
+                *reinterpret_cast<u32x4*>(d + kPlane) = b;
+                *reinterpret_cast<u32x4*>(d + 2 * kPlane) = c;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bad = limb_check(a[e], bad);
+            }
+#pragma unroll
+            for (int i = 0; i < VU; ++i) {
+                const int dim = vdim, quad = vquad + i * (NT / DP);
+                if (VU * NT > 8 * DP && quad >= 8) break;
+                // keys 4 quad .. + 3 = 16s + 8a + 4h' ..: unit 2s + h', half a
+                const int s = quad >> 2, a8 = (quad >> 1) & 1, hh = quad & 1;
+                u32x2 a, b, c;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    uint32_t x, y, z;
+                    const uint8_t* const src = raw + KU * 2048 + (4 * i + 2 * e) * 256 + lane * 4;
+                    split2(*reinterpret_cast<const float*>(src), *reinterpret_cast<const float*>(src + 256), x, y, z);
+                    a[e] = x;
+                    b[e] = y;
+                    c[e] = z;
+                }
+                uint8_t* const d = sv + v_off(dim, 2 * s + hh) + 8 * a8;
+                *reinterpret_cast<u32x2*>(d) = a;
+                *reinterpret_cast<u32x2*>(d + kPlane) = b;
+                *reinterpret_cast<u32x2*>(d + 2 * kPlane) = c;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) bad = limb_check(a[e], bad);
+            }
+            if (not_finite(bad)) atomicMin(first_bad, i0);
         };
 
-        // this lane's query row (n of the wave's 16): dims 16a + 4g .. + 3
-        const int qrow = q0 + wave * 16 + n;
+        lds_wait();  // (of the item before: the copies overwrite it)
+        load_tile(0);
+        // this lane's query row (n of the wave's 32): dims 16a + 8h .. + 7
+        const int qrow = q0 + wave * 32 + n;
         const float* qb = Q + static_cast<int64_t>(head) * D;
-        float qf[4 * NA];
+        u32x4 qh[KS], qm[KS], ql[KS];
+        bool qbad = false;
+        f32x4 qx[KS][2];  // all loads in flight at once; rows past T read row T - 1 (not stored)
 #pragma unroll
-        for (int a = 0; a < NA; ++a) {
-            f32x4 v4 = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (qrow < T && 16 * a + 4 * g < D)
-                v4 = *reinterpret_cast<const f32x4*>(qb + qrow * stride + 16 * a + 4 * g);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) qf[4 * a + b] = v4[b];
+        for (int a = 0; a < KS; ++a) {
+            const int dim = min(16 * a + 8 * h, D - 8);
+            const f32x4* p = reinterpret_cast<const f32x4*>(qb + min(qrow, T - 1) * stride + dim);
+            qx[a][0] = p[0];
+            qx[a][1] = p[1];
         }
-        f32x4 o[NA];  // o[c][r]: O[query n][dim 16c + 4g + r]
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int c = 0; c < NA; ++c) o[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        float m_run = -__builtin_inff(), l_run = 0.0f;  // of query n
+        for (int a = 0; a < KS; ++a) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = 16 * a + 8 * h < D ? qx[a][e >> 2][e & 3] : 0.0f;
+            split8(x, qh[a], qm[a], ql[a]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qbad |= !(fabsf(x[e]) < kQLimit);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x16 o[NC];  // o[c][4i + r]: O[query n][dim 32c + 8i + 4h + r]
+#pragma unroll
+        for (int c = 0; c < NC; ++c) o[c] = f32x16{};
+        float m_run = -__builtin_inff(), l_run = 0.0f;  // of query n; l of this half's keys
 
-        // The previous item's last barrier ended every read of the ring.
-        copy_tile(t0, lds);
-        wait_vmcnt<0>();
-        __syncthreads();
-        for (int tile = t0; tile < t1; ++tile) {
-            const float* ks = lds + ((tile - t0) & 1) * SF;
-            const float* vs = ks + kBK * DP;
-            // the next tile into the other stage (last read before the previous barrier)
-            if (tile + 1 < t1) copy_tile(tile + 1, lds + ((tile + 1 - t0) & 1) * SF);
-            const int base = tile * kBK;
-
-            // S^T: the tile's 16-key halves against the wave's 16 queries
-            f32x4 st[kNT];
-#pragma unroll
-            for (int t = 0; t < kNT; ++t) {
-                f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int a = 0; a < NA; ++a) {
-                    const f32x4 k4 = *reinterpret_cast<const f32x4*>(ks + k_off<DP>(16 * t + n, 4 * a + g));
-#pragma unroll
-                    for (int b = 0; b < 4; ++b)
-                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[b], qf[4 * a + b], c, 0, 0, 0);
-                }
-                st[t] = c;
-            }
-            // scale, mask, the tile's maximum for query n (8 in lane, 4 lanes)
+        // Scores of query n scaled, masked and turned into weights; the
+        // running state and the accumulator moved to the new maximum.
+        auto softmax = [&](f32x16& s, int base) {
             float mx = -__builtin_inff();
 #pragma unroll
-            for (int t = 0; t < kNT; ++t)
+            for (int e = 0; e < 16; ++e) s[e] *= scale;
+            if (base + kBK > T) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const bool valid = base + 16 * t + 4 * g + r < T;
-                    st[t][r] = valid ? st[t][r] * scale : -__builtin_inff();
-                    mx = fmaxf(mx, st[t][r]);
-                }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-            const float m_new = fmaxf(m_run, mx);  // finite: key `base` is valid
+                for (int e = 0; e < 16; ++e)
+                    if (base + 8 * (e >> 2) + 4 * h + (e & 3) >= T) s[e] = -__builtin_inff();
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+            mx = fmaxf(mx, other_half(mx, h));
+            const float m_new = fmaxf(m_run, mx);  // finite for finite scores: key `base` is valid
             const float alpha = exp_fast(m_run - m_new);  // 0 on the first tile
             float sum = 0.0f;
 #pragma unroll
-            for (int t = 0; t < kNT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    st[t][r] = exp_fast(st[t][r] - m_new);  // -inf -> 0
-                    sum += st[t][r];
-                }
-            sum += __shfl_xor(sum, 16, kWave);
-            sum += __shfl_xor(sum, 32, kWave);
+            for (int e = 0; e < 16; ++e) {
+                s[e] = exp_fast(s[e] - m_new);  // -inf -> 0
+                sum += s[e];
+            }
             l_run = l_run * alpha + sum;
             m_run = m_new;
+            if (__builtin_amdgcn_ballot_w64(!(alpha == 1.0f)) != 0) {
 #pragma unroll
-            for (int c = 0; c < NA; ++c) o[c] *= alpha;
-            // O^T += V^T P^T
+                for (int c = 0; c < NC; ++c) o[c] *= alpha;
+            }
+        };
+
+        constexpr int kMask = (DP / 8 - 1) & 15, kShift = DP == 128 ? 0 : (DP == 64 ? 1 : 2);
+        const int kbase = n * (2 * DP) + ((h ^ ((n >> kShift) & 1)) << 4);
+        f32x16 s;
+        u32x4 ph[2], pm[2], pl[2];  // limbs of P: keys of registers 8t .. 8t + 7
+        f32x16 sc;
+        // The fragments of one step: limbs of 16 dims of K, or of 16 keys of V
+        // for a 32-dim block.  Steps run one behind the next step's reads (the
+        // products of a step cover their latency; the scheduling barriers keep
+        // the reads ahead).
+        u32x4 fr[2][3];
+        auto read3 = [&](u32x4 (&f)[3], const uint8_t* p) {
 #pragma unroll
-            for (int t = 0; t < kNT; ++t)
+            for (int l = 0; l < 3; ++l) f[l] = *reinterpret_cast<const u32x4*>(p + l * kPlane);
+        };
+        // k_off(n, 2a + h) in two parts, recomputed each tile (opaque to the
+        // compiler, which would keep all KS of them in registers)
+        int kx = 0;
+        auto k_frag = [&](int i0, int a) -> const uint8_t* {
+            return lds + (i0 & 1) * 3 * kPlane + kbase + ((2 * a) << 4 ^ kx);
+        };
+        auto v_frag = [&](const uint8_t* st, int j) -> const uint8_t* {  // j = t * NC + c
+            return st + v_off(32 * (j % NC) + n, 2 * (j / NC) + h);
+        };
+        // S^T of tile i0; fr[buf] holds step 0.
+        auto scores = [&](int i0, int buf) {
+            sc = f32x16{};
+            s = f32x16{};
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int key = 16 * t + 4 * g + r;
-                    const float* vrow = vs + key * DP;
-                    const int sw = v_sw<DP>(key);
+            for (int a = 0; a < KS; ++a) {
+                u32x4(&f)[3] = fr[(a + buf) & 1];
+                if (a + 1 < KS) read3(fr[(a + 1 + buf) & 1], k_frag(i0, a + 1));
+                __builtin_amdgcn_sched_barrier(0);
+                s = mma(f[0], qh[a], s);
+                sc = mma(f[0], qm[a], sc);
+                sc = mma(f[1], qh[a], sc);
+                sc = mma(f[1], qm[a], sc);
+                sc = mma(f[0], ql[a], sc);
+                sc = mma(f[2], qh[a], sc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int nt = t1 - t0;  // tiles the limb loop takes
+        // O^T += V^T P^T of tile i0, then the scores of tile i0 + 1.
+        auto products = [&](int i0) {
+            kx = ((n >> kShift) & kMask & ~1) << 4;
+            asm volatile("" : "+v"(kx));
+            const uint8_t* const st = ldsV + (i0 % 3) * 3 * kPlane;
+            read3(fr[0], v_frag(st, 0));
 #pragma unroll
-                    for (int c = 0; c < NA; ++c)
-                        o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[(16 * c + n) ^ sw], st[t][r], o[c], 0, 0, 0);
-                }
-            // this wave's copy of the next tile has landed; after the barrier
-            // every wave's has, and every wave is done with this stage
-            wait_vmcnt<0>();
-            __syncthreads();
+            for (int j = 0; j < 2 * NC; ++j) {
+                u32x4(&f)[3] = fr[j & 1];
+                read3(fr[(j + 1) & 1], j + 1 < 2 * NC ? v_frag(st, j + 1) : k_frag(i0 + 1, 0));
+                __builtin_amdgcn_sched_barrier(0);
+                const int t = j / NC, c = j % NC;
+                o[c] = mma(f[2], ph[t], o[c]);
+                o[c] = mma(f[0], pl[t], o[c]);
+                o[c] = mma(f[1], pm[t], o[c]);
+                o[c] = mma(f[1], ph[t], o[c]);
+                o[c] = mma(f[0], pm[t], o[c]);
+                o[c] = mma(f[0], ph[t], o[c]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (kTwo || i0 + 1 < nt) scores(i0 + 1, 0);
+        };
+
+        __syncthreads();  // every wave is done with the previous item's LDS
+        if (tid == 0) *first_bad = nt;
+        __syncthreads();
+        copies_wait();
+        stage_tile(0);
+        // The second group, a phase behind, stages its share of a tile one
+        // phase ahead of the first group's.
+        const int ahead = second ? 2 : 1;
+        if (second && nt > 1) {
+            lds_wait();  // the copies overwrite what stage_tile(0) read
+            load_tile(1);
+            copies_wait();
+            stage_tile(1);
         }
+        if (qbad) atomicMin(first_bad, 0);
+        __syncthreads();
+        // Product phase i: O += P V of tile i - 1, then the scores of tile i.
+        // Softmax phase i: the weights of tile i, and this thread's share of
+        // tile i + ahead into LDS.  Tile i + 1 is whole before the first
+        // group's product phase i + 1 (the second group wrote its share two
+        // phases before, the first group one).  A tile's K was last read in
+        // the second group's phase i, two phases before the slot is written
+        // again; its V one product phase later, hence three slots.
+        if (second) lds_barrier();
+        nt = min(nt, __builtin_amdgcn_readfirstlane(*first_bad));
+        if (t0 + ahead < t1) load_tile(ahead);
+        kx = ((n >> kShift) & kMask & ~1) << 4;
+        read3(fr[0], k_frag(0, 0));
+        scores(0, 0);
+        for (int i = 0; i < nt; ++i) {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(0);
+            if (kTwo) lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            s += sc;
+            softmax(s, (t0 + i) * kBK);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float p[8] = {s[8 * t], s[8 * t + 1], s[8 * t + 2], s[8 * t + 3],
+                                    s[8 * t + 4], s[8 * t + 5], s[8 * t + 6], s[8 * t + 7]};
+                split8(p, ph[t], pm[t], pl[t]);
+            }
+            // (opaque: the compiler would compute them in the next phase)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) asm volatile("" : "+v"(ph[t]), "+v"(pm[t]), "+v"(pl[t]));
+            copies_wait();
+            if (t0 + i + ahead < t1) stage_tile(i + ahead);
+            __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+            nt = min(nt, __builtin_amdgcn_readfirstlane(*first_bad));
+            if (t0 + i + 1 + ahead < t1) load_tile(i + 1 + ahead);
+            products(i);  // (past the last tile: scores of whatever the slot holds, unused)
+        }
+        __builtin_amdgcn_s_setprio(0);
+        if (kTwo && !second) lds_barrier();
+        // The rest of a block that met a value without limbs, in f32 from memory.
+        for (int tile = t0 + nt; tile < t1; ++tile) {
+            const int base = tile * kBK;
+            s = f32x16{};
+#pragma unroll 1
+            for (int a = 0; a < DP / 2; ++a) {
+                const int dim = 2 * a + h;
+                const float ka = base + n < T && dim < D ? kb[(base + n) * stride + dim] : 0.0f;
+                const float qa = qrow < T && dim < D ? qb[qrow * stride + dim] : 0.0f;
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(ka, qa, s, 0, 0, 0);
+            }
+            softmax(s, base);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int key = base + 8 * (e >> 2) + 4 * h + (e & 3);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const float va = key < T && 32 * c + n < D ? vb[key * stride + 32 * c + n] : 0.0f;
+                    o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, s[e], o[c], 0, 0, 0);
+                }
+            }
+        }
+        l_run += other_half(l_run, h);
 
         if (t0 > 0 || t1 < ntile) {
             // One of two pieces of the item: its state, then the arrival.
             const int piece = t0 == 0 ? 0 : 1;
             const int bnd = static_cast<int>(blockIdx.x) - piece;  // the boundary that cut the item
-            float* mine = part + (static_cast<int64_t>(bnd) * 2 + piece) * piece_floats<DP>();
-            const int ql = wave * 16 + n;
+            constexpr int kPiece = piece_floats(BQ, DP);
+            float* mine = part + (static_cast<int64_t>(bnd) * 2 + piece) * kPiece;
+            const int qi = wave * 32 + n;
 #pragma unroll
-            for (int c = 0; c < NA; ++c)
+            for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) st_dev(mine + ql * DP + 16 * c + 4 * g + r, o[c][r]);
-            if (g == 0) {
-                st_dev(mine + kBQ * DP + ql, m_run);
-                st_dev(mine + kBQ * DP + kBQ + ql, l_run);
+                for (int e = 0; e < 16; ++e) st_dev(mine + qi * DP + 32 * c + 8 * (e >> 2) + 4 * h + (e & 3), o[c][e]);
+            if (h == 0) {
+                st_dev(mine + BQ * DP + qi, m_run);
+                st_dev(mine + BQ * DP + BQ + qi, l_run);
             }
             wait_vmcnt<0>();
             __syncthreads();
@@ -281,67 +528,96 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             // Merge: m = max, each side scaled by exp(m_side - m).  Two terms,
             // so the result does not depend on which piece merges.
-            const float* other = part + (static_cast<int64_t>(bnd) * 2 + (1 - piece)) * piece_floats<DP>();
-            const float mo = ld_dev(other + kBQ * DP + ql), lo = ld_dev(other + kBQ * DP + kBQ + ql);
+            const float* other = part + (static_cast<int64_t>(bnd) * 2 + (1 - piece)) * kPiece;
+            const float mo = ld_dev(other + BQ * DP + qi), lo = ld_dev(other + BQ * DP + BQ + qi);
             const float m = fmaxf(m_run, mo);
             const float am = exp_fast(m_run - m), ao = exp_fast(mo - m);
             l_run = l_run * am + lo * ao;
 #pragma unroll
-            for (int c = 0; c < NA; ++c)
+            for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) o[c][r] = o[c][r] * am + ld_dev(other + ql * DP + 16 * c + 4 * g + r) * ao;
+                for (int e = 0; e < 16; ++e)
+                    o[c][e] = o[c][e] * am + ld_dev(other + qi * DP + 32 * c + 8 * (e >> 2) + 4 * h + (e & 3)) * ao;
             if (tid == 0) __hip_atomic_store(cnt + bnd, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        // out[query n][dims 16c + 4g ..]: divide by the denominator
+        // out[query n][dims 32c + 8i + 4h ..]: divide by the denominator
         if (qrow < T) {
             float* dst = O + qrow * stride + static_cast<int64_t>(head) * D;
             const float inv = 1.0f / l_run;
 #pragma unroll
-            for (int c = 0; c < NA; ++c)
-                if (16 * c + 4 * g < D) *reinterpret_cast<f32x4*>(dst + 16 * c + 4 * g) = o[c] * inv;
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int dim = 32 * c + 8 * i + 4 * h;
+                    if (dim < D)
+                        *reinterpret_cast<f32x4*>(dst + dim) =
+                            f32x4{o[c][4 * i], o[c][4 * i + 1], o[c][4 * i + 2], o[c][4 * i + 3]} * inv;
+                }
         }
     }
 }
 
-template <int DP>
+// Workgroup slots of the 8-wave form: one per CU (96 KB of LDS at 128 dims,
+// 256 registers a wave).
+int flux_slots() { return static_cast<int>(device_info().cus); }
+
+int padded_dims(int head_dim) { return head_dim <= 32 ? 32 : (head_dim <= 64 ? 64 : 128); }
+
+template <int DP, int NW>
 hipError_t run(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads, int d, float scale,
-               float* part, uint32_t* cnt, int slots, hipStream_t s) {
-    const int64_t nqb = (t + kBQ - 1) / kBQ, ntile = (t + kBK - 1) / kBK, items = n_heads * nqb;
+               float* part, uint32_t* cnt, hipStream_t s) {
+    constexpr int BQ = 32 * NW;
+    const int64_t nqb = (t + BQ - 1) / BQ, ntile = (t + kBK - 1) / kBK, items = n_heads * nqb;
+    const size_t lds = flux_lds_bytes<DP, NW>();
     if (!part) {
         const dim3 grid(static_cast<unsigned>(n_heads), static_cast<unsigned>(nqb));
-        hipLaunchKernelGGL(k_flux_attn<DP>, grid, dim3(kThreads), flux_lds_bytes<DP>(), s, q, k, v, out,
+        hipLaunchKernelGGL((k_flux_attn<DP, NW>), grid, dim3(NW * kWave), lds, s, q, k, v, out,
                            static_cast<int>(t), n_heads, d, scale, nullptr, nullptr, 0);
     } else {
+        const int slots = flux_slots();
         const int64_t per = (items * ntile + slots - 1) / slots;  // >= ntile: more items than slots
-        hipLaunchKernelGGL(k_flux_attn<DP>, dim3(static_cast<unsigned>(slots)), dim3(kThreads), flux_lds_bytes<DP>(),
-                           s, q, k, v, out, static_cast<int>(t), n_heads, d, scale, part, cnt, static_cast<int>(per));
+        hipLaunchKernelGGL((k_flux_attn<DP, NW>), dim3(static_cast<unsigned>(slots)), dim3(NW * kWave),
+                           lds, s, q, k, v, out, static_cast<int>(t), n_heads, d, scale, part, cnt,
+                           static_cast<int>(per));
     }
     return hipGetLastError();
 }
 
-// Workgroup slots: two per CU (64 KB of LDS and 4 waves per SIMD each).
-int flux_slots() { return 2 * static_cast<int>(device_info().cus); }
+// 4-wave workgroups where their blocks of 128 queries are at most one per CU
+// (twice the workgroups, each with about 0.6 of the time), where one such
+// block holds all queries, or where 256-query blocks would be cut although
+// the 128-query ones are at most two per CU: such calls take no workspace, and
+// up to 64 dims two of them share a CU (t = 384, 150 x 64: 63 us one at a
+// time, 44 in pairs).
+bool half_blocks(int64_t t, int n_heads) {
+    const int64_t items = n_heads * ((t + 127) / 128), slots = flux_slots();
+    return t <= 128 || items <= slots || (items <= 2 * slots && n_heads * ((t + 255) / 256) > slots);
+}
 
-int padded_dims(int head_dim) { return head_dim <= 32 ? 32 : (head_dim <= 64 ? 64 : 128); }
+template <int DP>
+hipError_t run_dp(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads, int d, float scale,
+                  float* part, uint32_t* cnt, hipStream_t s) {
+    if (half_blocks(t, n_heads))
+        return run<DP, 4>(q, k, v, out, t, n_heads, d, scale, nullptr, nullptr, s);
+    return run<DP, 8>(q, k, v, out, t, n_heads, d, scale, part, cnt, s);
+}
 
 }  // namespace
 
 size_t flux_attention_workspace(int64_t t, int n_heads, int head_dim) {
-    const int64_t items = n_heads * ((t + kBQ - 1) / kBQ);
+    const int64_t items = n_heads * ((t + 255) / 256);
     const int slots = flux_slots();
-    if (items <= slots) return 0;
-    const int dp = padded_dims(head_dim);
-    return static_cast<size_t>(slots) * 2 * (kBQ * dp + 2 * kBQ) * sizeof(float);
+    if (items <= slots || half_blocks(t, n_heads)) return 0;
+    return static_cast<size_t>(slots) * 2 * piece_floats(256, padded_dims(head_dim)) * sizeof(float);
 }
 
 hipError_t launch_flux_attention(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads,
                                  int head_dim, float scale, float* part, uint32_t* counters, hipStream_t s) {
-    const int slots = flux_slots();
-    if (part && (!counters || static_cast<size_t>(slots) > kArrivalCounters)) return hipErrorInvalidValue;
+    if (part && (!counters || static_cast<size_t>(flux_slots()) > kArrivalCounters)) return hipErrorInvalidValue;
     switch (padded_dims(head_dim)) {
-        case 32: return run<32>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, slots, s);
-        case 64: return run<64>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, slots, s);
-        default: return run<128>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, slots, s);
+        case 32: return run_dp<32>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s);
+        case 64: return run_dp<64>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s);
+        default: return run_dp<128>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s);
     }
 }
 

@@ -1,0 +1,114 @@
+"""FLUX's attention at the edges of its blocks and at values its bf16 limbs do
+not take: 128- and 256-query blocks, 32-key tiles and every padded head width;
+values past 2^64 (2^55 in q), infinities and NaN, which go through f32 matrix
+steps; products that overflow; tiny values; a capture without workspace.
+
+Bound: FLUX_ATTN_TOL of test_gpu_flux_attention.py (1e-5 of the largest
+output) against float64."""
+import numpy as np
+import pytest
+
+from helpers import from_dev, normwise_err, say, to_dev
+
+pytestmark = pytest.mark.gpu
+
+FLUX_ATTN_TOL = 1e-5
+
+
+def exact(q, k, v, h, d):
+    """float64 attention; inputs as f32 arithmetic sees them, so a score past
+    the f32 range is infinite."""
+    t = q.shape[0]
+    q, k, v = (a.astype(np.float64).reshape(t, h, d).transpose(1, 0, 2) for a in (q, k, v))
+    with np.errstate(all="ignore"):
+        s = (q @ k.transpose(0, 2, 1))
+        s = np.where(np.abs(s) > np.finfo(np.float32).max, np.sign(s) * np.inf, s) / np.sqrt(d)
+        w = np.exp(s - s.max(-1, keepdims=True))
+        w = w / w.sum(-1, keepdims=True)
+        w = np.where(w < 1e-45, 0.0, w)
+        out = w @ v
+    return out.transpose(1, 0, 2).reshape(t, h * d)
+
+
+def run(rt, q, k, v, h, d):
+    return from_dev(rt.flux_attention(to_dev(q), to_dev(k), to_dev(v), h, d))
+
+
+def rand(t, h, d):
+    rng = np.random.default_rng(t * 31 + h * 5 + d)
+    return [rng.standard_normal((t, h * d)).astype(np.float32) for _ in range(3)]
+
+
+@pytest.mark.parametrize("t,h,d", [(31, 2, 32), (33, 1, 40), (96, 3, 128), (128, 2, 64), (129, 260, 8), (255, 200, 16),
+                                   (257, 130, 40), (513, 90, 64), (520, 100, 72), (800, 70, 128), (100, 300, 120)])
+def test_flux_attention_block_edges(rt, t, h, d):
+    say(f"[flux limbs] t={t} heads={h} head_dim={d}")
+    q, k, v = rand(t, h, d)
+    got, want = run(rt, q, k, v, h, d), exact(q, k, v, h, d)
+    assert normwise_err(got, want) <= FLUX_ATTN_TOL
+    for hh in range(0, h, 13):
+        sl = slice(hh * d, (hh + 1) * d)
+        assert normwise_err(got[:, sl], want[:, sl]) <= FLUX_ATTN_TOL, hh
+
+
+# (4 heads of 128: 4-wave blocks; 70: 8 waves with blocks cut between two)
+@pytest.mark.parametrize("t,h,d,row", [(300, 4, 128, 0), (300, 4, 128, 290), (300, 4, 40, 64), (800, 70, 128, 31),
+                                       (800, 70, 128, 799), (700, 100, 64, 350)])
+def test_flux_attention_values_without_limbs(rt, t, h, d, row):
+    say(f"[flux limbs wide] t={t} heads={h} head_dim={d} row={row}")
+    q, k, v = rand(t, h, d)
+    head = [slice(i * d, (i + 1) * d) for i in range(4)]
+    # head 0: an infinity and a NaN in v reach their columns of every row
+    v[row, 3], v[row, 5] = np.inf, np.nan
+    # head 1: products that overflow downwards drop the key, here in every row
+    q[:, head[1]] = 0.0
+    q[:, head[1].start + 1] = np.float32(1.7e25)
+    k[:, head[1].start + 1] = 0.0
+    k[row, head[1].start + 1] = np.float32(-1.3e19)
+    # head 2: a key that meets tiny queries with huge values
+    q[:, head[2].start] = np.float32(1e-38)
+    k[row, head[2].start] = np.float32(3.4e38)
+    # head 3: an infinite v, one of opposite sign next to it, and one huge query
+    v[row, head[3].start] = -np.inf
+    q[0, head[3]] = 0.0
+    q[0, head[3].start + 1] = np.float32(3e37)
+    k[:, head[3].start + 1] = np.where(np.arange(t) == row, 1e-37, -1e-37)
+    got, want = run(rt, q, k, v, h, d), exact(q, k, v, h, d)
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(np.isposinf(got), np.isposinf(want))
+        assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    for sl in head + [slice(4 * d, h * d)]:
+        if sl.stop > sl.start:
+            g, w, f = got[:, sl], want[:, sl], fin[:, sl]
+            assert normwise_err(np.where(f, g, 0), np.where(f, w, 0)) <= FLUX_ATTN_TOL
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e18])
+def test_flux_attention_scaled_values(rt, scale):
+    t, h, d = 300, 4, 64
+    say(f"[flux limbs scaled] v x {scale}")
+    q, k, v = rand(t, h, d)
+    v = (v * np.float32(scale)).astype(np.float32)
+    assert normwise_err(run(rt, q, k, v, h, d), exact(q, k, v, h, d)) <= FLUX_ATTN_TOL
+
+
+def test_flux_attention_captured_without_workspace(rt):
+    import torch
+    t, h, d = 700, 100, 128
+    f = rt.library().lib.rt_hip_flux_attention_workspace_bytes
+    say(f"[flux limbs] captured: workspace {rt.workspace_bytes()}, need {f(t, h, d)}")
+    q, k, v = rand(t, h, d)
+    dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
+    out = torch.zeros_like(dq)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rt.flux_attention(dq, dk, dv, h, d, out=out)
+    want = exact(q, k, v, h, d)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert normwise_err(from_dev(out), want) <= FLUX_ATTN_TOL
