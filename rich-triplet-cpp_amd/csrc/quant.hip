@@ -7,14 +7,15 @@
 // f32 value to nearest-even, as flux_dequant_q4k's bfloat() conversion does
 // (shaders/flux.msl:78-79).
 //
-// Quantize: one wave per 256-value super-block, lane l holding values
-// 4l..4l+3 (sub-block l/8).  Every arithmetic step is the reference's
-// (quant_q4k.cpp:71-158) in the same order with the same rounding: min/max
-// are exact whatever the reduction order, the per-sub-block and per-block
-// scalars are computed identically by every lane, IEEE division and
-// reciprocal (hipcc's default correctly-rounded f32 divide), no
-// contraction (the library builds with -ffp-contract=off), and the f16
-// header conversion is the reference's truncating one restated on bits.
+// Quantize: one wave per four 256-value super-blocks, lane l holding values
+// 4l..4l+3 of each (sub-block l/8).  Every arithmetic step gives the bits of
+// the reference's (quant_q4k.cpp:71-158): min/max are exact whatever the
+// reduction order, the scalars of a sub-block and block take IEEE divisions
+// and reciprocals (hipcc's default correctly-rounded f32 divide), no
+// contraction (the library builds with -ffp-contract=off), the division of
+// each value is a correctly rounded one from the sub-block's reciprocal, and
+// the f16 header conversion is the reference's truncating one restated on
+// bits.
 #include "q4k_mfma.hpp"
 #include "rt_common.hpp"
 #include "rt_launch.hpp"
@@ -138,48 +139,113 @@ __device__ __forceinline__ uint32_t f32_to_f16_trunc(float v) {
 }
 
 // std::min / std::max argument order of the reference (first wins on ties).
-__device__ __forceinline__ float ref_min(float a, float b) { return b < a ? b : a; }
 __device__ __forceinline__ float ref_max(float a, float b) { return a < b ? b : a; }
 
-__global__ __launch_bounds__(256) void k_quantize_q4k(const float* __restrict__ w,
-                                                      uint8_t* __restrict__ out, int64_t rows,
-                                                      int64_t cols) {
-    const int64_t nb = cols >> 8;
-    const int64_t blk = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (blk >= rows * nb) return;
+// The value of another lane: DPP control c (0xb1: lane ^ 1, 0x4e: lane ^ 2,
+// 0x141: mirrored within 8 lanes, 0x128: lane ^ 8), lane ^ 16, lane ^ 32.
+template <int C>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), C, 0xf, 0xf, true));
+}
+template <int C>
+__device__ __forceinline__ float dpp_f32(float x) {
+    return __uint_as_float(dpp_u32<C>(__float_as_uint(x)));
+}
+__device__ __forceinline__ uint32_t lane_xor16(uint32_t x, int lane) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return (lane & 16) ? r[0] : r[1];
+}
+__device__ __forceinline__ uint32_t lane_xor32(uint32_t x, int lane) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return (lane & 32) ? r[0] : r[1];
+}
+// The largest / the OR over the 8 lanes l + 8 j.
+__device__ __forceinline__ float max_of_8(float x, int lane) {
+    x = fmaxf(x, dpp_f32<0x128>(x));
+    x = fmaxf(x, __uint_as_float(lane_xor16(__float_as_uint(x), lane)));
+    return fmaxf(x, __uint_as_float(lane_xor32(__float_as_uint(x), lane)));
+}
+__device__ __forceinline__ uint32_t or_of_8(uint32_t x, int lane) {
+    x |= dpp_u32<0x128>(x);
+    x |= lane_xor16(x, lane);
+    return x | lane_xor32(x, lane);
+}
+// x of the lane that has this lane's sub-block (8 lanes) of block B.
+template <int B>
+__device__ __forceinline__ float from_owner(float x) {
+    return __uint_as_float(static_cast<uint32_t>(
+        __builtin_amdgcn_ds_swizzle(static_cast<int>(__float_as_uint(x)), 0x18 | ((2 * B) << 5))));
+}
+
+// The nibble of v: min(15, sat_u8((v + mn) / sc + 0.5)) with r = 1 / sc and
+// lim = 15 sc (exact: 21 bits), or sc = r = lim = 0 for a sub-block whose
+// nibbles are all 0.  Above lim the nibble is 15 either way; NaN and negative
+// sums become 0 in the clamp.  Two remainder steps make q the correctly
+// rounded quotient (P. Markstein, Computation of elementary functions on the
+// IBM RISC System/6000, 1990): the first leaves q within one ulp, the second,
+// on an exact remainder and a correctly rounded r, rounds as a division does.
+// Quotients too small for that are far below the 0.5 that would matter.
+__device__ __forceinline__ uint32_t nibble(float v, float mn, float sc, float r, float lim) {
+    const float x = __builtin_amdgcn_fmed3f(v + mn, 0.0f, lim);
+    float q = x * r;
+    q = __builtin_fmaf(__builtin_fmaf(-sc, q, x), r, q);
+    q = __builtin_fmaf(__builtin_fmaf(-sc, q, x), r, q);
+    return static_cast<uint32_t>(q + 0.5f);
+}
+
+// Bound: the bytes (reading the f32 weight), once the VALU work per value is
+// small: with one block per wave every lane computed its sub-block's and
+// block's scalars (9 divisions, 8 lanes for one sub-block, 64 for one block)
+// and 4 values' nibbles, about 300 instructions per 256 values, and the VALU
+// bound the kernel.  With four blocks per wave the min / max reduction ends
+// with one sub-block in each pair of lanes (reduce-scatter over the blocks),
+// so the scalars are computed once for all four.  8192 x 3072: 57.3 -> 22.5 us
+// (2.0 -> 5.1 TB/s); 8192 x 12288: 214 -> 99 us.
+__global__ __launch_bounds__(256) void k_quantize_q4k(const float* __restrict__ w, uint8_t* __restrict__ out,
+                                                      int64_t blocks) {
+    const int64_t blk0 = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * 4;
+    if (blk0 >= blocks) return;
     const int lane = threadIdx.x & 63;
-    const int64_t row = blk / nb, b = blk % nb;
-    const float* src = w + row * cols + b * 256 + 4 * lane;
-    const f32x4 v = *reinterpret_cast<const f32x4*>(src);
+    f32x4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // (past the end: the last block again, not stored)
+        v[i] = *reinterpret_cast<const f32x4*>(w + min(blk0 + i, blocks - 1) * 256 + 4 * lane);
 
     // Step 1: sub-block (8 lanes) min / max, seeded with +-inf as the
     // reference's loop is, so a NaN input is skipped exactly as there.
-    float smin = __builtin_inff(), smax = -__builtin_inff();
+    float lo[4], hi[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        smin = ref_min(smin, v[e]);
-        smax = ref_max(smax, v[e]);
-    }
+    for (int i = 0; i < 4; ++i) {
+        lo[i] = __builtin_inff();
+        hi[i] = -__builtin_inff();
 #pragma unroll
-    for (int off = 4; off >= 1; off >>= 1) {
-        smin = ref_min(smin, __shfl_xor(smin, off, 64));
-        smax = ref_max(smax, __shfl_xor(smax, off, 64));
+        for (int e = 0; e < 4; ++e) {
+            lo[i] = fminf(lo[i], v[i][e]);
+            hi[i] = fmaxf(hi[i], v[i][e]);
+        }
     }
-    float sub_min, sub_scale;
-    if (smin >= 0.0f) {
-        sub_min = 0.0f;
-        sub_scale = smax > 0.0f ? smax / 15.0f : 0.0f;
-    } else {
+    // lanes with bit 2 (then bit 1) set go on with the later half of the blocks
+    const bool b2 = (lane & 4) != 0, b1 = (lane & 2) != 0;
+    float lo2[2], hi2[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        lo2[i] = fminf(b2 ? lo[i + 2] : lo[i], dpp_f32<0x141>(b2 ? lo[i] : lo[i + 2]));
+        hi2[i] = fmaxf(b2 ? hi[i + 2] : hi[i], dpp_f32<0x141>(b2 ? hi[i] : hi[i + 2]));
+    }
+    float smin = fminf(b1 ? lo2[1] : lo2[0], dpp_f32<0x4e>(b1 ? lo2[0] : lo2[1]));
+    float smax = fmaxf(b1 ? hi2[1] : hi2[0], dpp_f32<0x4e>(b1 ? hi2[0] : hi2[1]));
+    smin = fminf(smin, dpp_f32<0xb1>(smin));
+    smax = fmaxf(smax, dpp_f32<0xb1>(smax));
+    // from here on this lane has sub-block lane / 8 of block (lane & 6) / 2
+    float sub_min = 0.0f, range = smax;
+    if (!(smin >= 0.0f)) {
         sub_min = smin;
-        sub_scale = smax > smin ? (smax - smin) / 15.0f : 0.0f;
+        range = smax > smin ? smax - smin : 0.0f;
     }
+    const float sub_scale = range > 0.0f ? range / 15.0f : 0.0f;
     // Step 2: block maxima over the 8 sub-blocks.
-    float max_scale = ref_max(0.0f, sub_scale), max_min = ref_max(0.0f, -sub_min);
-#pragma unroll
-    for (int off = 8; off <= 32; off <<= 1) {
-        max_scale = ref_max(max_scale, __shfl_xor(max_scale, off, 64));
-        max_min = ref_max(max_min, __shfl_xor(max_min, off, 64));
-    }
+    const float max_scale = max_of_8(ref_max(0.0f, sub_scale), lane);
+    const float max_min = max_of_8(ref_max(0.0f, -sub_min), lane);
     const float d = max_scale > 0.0f ? max_scale / 63.0f : 0.0f;
     const float dmin = max_min > 0.0f ? max_min / 63.0f : 0.0f;
     // Step 3: 6-bit scale and min of this lane's sub-block.
@@ -195,40 +261,45 @@ __global__ __launch_bounds__(256) void k_quantize_q4k(const float* __restrict__ 
     // Step 4: f16 header (truncating).
     const uint32_t d16 = f32_to_f16_trunc(d), m16 = f32_to_f16_trunc(dmin);
     const float dv = f16_bits_to_f32(d16), mvv = f16_bits_to_f32(m16);
-    // Step 6: nibbles with the f16-rounded scales.
-    const float sc = dv * static_cast<float>(sv), mn = mvv * static_cast<float>(mv);
-    uint32_t qn = 0;
+    // Step 6: nibbles with the f16-rounded scales (all 0 for a scale of 0,
+    // infinite or NaN).
+    const float sc0 = dv * static_cast<float>(sv), mn0 = mvv * static_cast<float>(mv);
+    const bool some = sc0 > 0.0f && sc0 < __builtin_inff();
+    const float sc1 = some ? sc0 : 0.0f, r1 = some ? 1.0f / sc0 : 0.0f;
+    uint32_t qn[4];
+    auto block_nibbles = [&](const f32x4& x, float sc, float mn, float r) {
+        const float lim = 15.0f * sc;
+        uint32_t q = 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t q = sc > 0.0f ? min(15u, sat_u8((v[e] + mn) / sc + 0.5f)) : 0u;
-        qn |= q << (8 * e);
-    }
-    uint8_t* ob = out + blk * kQ4kBlockBytes;
+        for (int e = 0; e < 4; ++e) q |= nibble(x[e], mn, sc, r, lim) << (8 * e);
+        return q;
+    };
+    qn[0] = block_nibbles(v[0], from_owner<0>(sc1), from_owner<0>(mn0), from_owner<0>(r1));
+    qn[1] = block_nibbles(v[1], from_owner<1>(sc1), from_owner<1>(mn0), from_owner<1>(r1));
+    qn[2] = block_nibbles(v[2], from_owner<2>(sc1), from_owner<2>(mn0), from_owner<2>(r1));
+    qn[3] = block_nibbles(v[3], from_owner<3>(sc1), from_owner<3>(mn0), from_owner<3>(r1));
     // Value 4*lane+e sits in chunk c = lane/16; lanes with (lane%16) < 8 hold
-    // low nibbles, lane+8 the matching high nibbles.
-    const uint32_t partner = __shfl_xor(qn, 8, 64);
-    if ((lane & 15) < 8) {
-        const int c = lane >> 4;
-        const uint32_t word = qn | (partner << 4);
-        *reinterpret_cast<uint32_t*>(ob + 16 + 32 * c + 4 * (lane & 7)) = word;
-    }
-    // Step 5: pack the 12 scale bytes (pack_scales, quant_q4k.cpp:43-55).
-    uint32_t svs[8], mvs[8];
+    // low nibbles, lane+8 the matching high nibbles.  Of each pair of blocks
+    // the former lanes store the first, the latter the second.
+    const bool b3 = (lane & 8) != 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        svs[j] = __shfl(sv, 8 * j, 64);
-        mvs[j] = __shfl(mv, 8 * j, 64);
+    for (int i = 0; i < 4; i += 2) {
+        const uint32_t own = b3 ? qn[i + 1] : qn[i], got = dpp_u32<0x128>(b3 ? qn[i] : qn[i + 1]);
+        const uint32_t word = b3 ? got | (own << 4) : own | (got << 4);
+        const int64_t blk = blk0 + i + (b3 ? 1 : 0);
+        if (blk < blocks)
+            *reinterpret_cast<uint32_t*>(out + blk * kQ4kBlockBytes + 16 + 32 * (lane >> 4) + 4 * (lane & 7)) = word;
     }
-    if (lane == 0) {
-        uint32_t s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            s0 |= ((svs[j] & 0x3fu) | ((svs[j + 4] & 0x30u) << 2)) << (8 * j);
-            s1 |= ((mvs[j] & 0x3fu) | ((mvs[j + 4] & 0x30u) << 2)) << (8 * j);
-            s2 |= ((svs[j + 4] & 0x0fu) | ((mvs[j + 4] & 0x0fu) << 4)) << (8 * j);
-        }
-        *reinterpret_cast<u32x4*>(ob) = u32x4{d16 | (m16 << 16), s0, s1, s2};
-    }
+    // Step 5: pack the 12 scale bytes (pack_scales, quant_q4k.cpp:43-55), each
+    // sub-block j's share in its place.
+    const int j = lane >> 3, sh = 8 * (j & 3);
+    const bool up = j >= 4;
+    const uint32_t s0 = or_of_8((up ? (sv & 0x30u) << 2 : sv) << sh, lane);
+    const uint32_t s1 = or_of_8((up ? (mv & 0x30u) << 2 : mv) << sh, lane);
+    const uint32_t s2 = or_of_8(up ? ((sv & 0x0fu) | ((mv & 0x0fu) << 4)) << sh : 0u, lane);
+    const int64_t blk = blk0 + (lane >> 1);
+    if (lane < 8 && (lane & 1) == 0 && blk < blocks)
+        *reinterpret_cast<u32x4*>(out + blk * kQ4kBlockBytes) = u32x4{d16 | (m16 << 16), s0, s1, s2};
 }
 
 // Reference row-major Q4_K blocks -> tiled layout (q4k_mfma.hpp): one thread
@@ -304,9 +375,8 @@ hipError_t launch_dequant_q4k_cvt(const void* w, uint16_t* wout, int64_t n, int6
 hipError_t launch_quantize_q4k(const float* w, void* blocks, int64_t n, int64_t k,
                                hipStream_t s) {
     const int64_t nblk = n * (k / 256);
-    const unsigned grid = static_cast<unsigned>((nblk + 3) / 4);
-    hipLaunchKernelGGL(k_quantize_q4k, dim3(grid), dim3(256), 0, s, w,
-                       static_cast<uint8_t*>(blocks), n, k);
+    const unsigned grid = static_cast<unsigned>((nblk + 15) / 16);
+    hipLaunchKernelGGL(k_quantize_q4k, dim3(grid), dim3(256), 0, s, w, static_cast<uint8_t*>(blocks), nblk);
     return hipGetLastError();
 }
 
