@@ -162,6 +162,29 @@ int gemvm(const Proj& p, const float* x, float* y, int m, hipStream_t s) {
     return rt_hip_gemv_bf16(static_cast<const uint16_t*>(p.data), x, y, p.n, p.k, m, s);
 }
 
+// The Q4_K ones of `count` projections that share a launch with the others
+// (m rows on one x): all of those whose rows are whole tiles.
+bool batch_job(const Proj& p) { return p.q4k() && p.n % 16 == 0; }
+
+// y[j][m] = W[j] x[m] for up to three projections: the Q4_K ones in one launch.
+int gemvm_multi(int count, const Proj* const* p, const float* x, float* const* y, int m, hipStream_t s) {
+    const void* w[3];
+    float* yj[3];
+    int64_t n[3];
+    int jobs = 0, rc = RT_HIP_OK;
+    for (int j = 0; j < count; ++j)
+        if (batch_job(*p[j])) {
+            w[jobs] = p[j]->data;
+            yj[jobs] = y[j];
+            n[jobs++] = p[j]->n;
+        }
+    const bool one = m > 1 && jobs > 1;
+    if (one) rc = chk(launch_gemv_batch_q4k_multi(jobs, w, x, yj, n, p[0]->k, m, s), "decoder: batched projections");
+    for (int j = 0; j < count && !rc; ++j)
+        if (!one || !batch_job(*p[j])) rc = gemvm(*p[j], x, y[j], m, s);
+    return rc;
+}
+
 // Split count of a layer's attention for m rows: the window bounds the
 // positions a row reads, else the cache length.  The partials buffer was
 // sized at create for the cache length, and create clamps every window to
@@ -373,11 +396,9 @@ int layer_stepm(rt_hip_decoder* d, int li, int m, hipStream_t s) {
     const auto& c = d->cfg;
     Layer& L = d->layers[li];
     const int H = c.hidden, nq = c.n_heads, nkv = c.n_kv_heads, hd = c.head_dim, F = c.ffn;
-    int rc = chk(launch_rmsnorm_rows(d->hidden, L.attn_norm, nullptr, d->normed, H, m, c.norm_eps, d->gemma, s),
-                 "decoder: rmsnorm");
-    if (!rc) rc = gemvm(L.q, d->normed, d->q, m, s);
-    if (!rc) rc = gemvm(L.k, d->normed, d->k, m, s);
-    if (!rc) rc = gemvm(L.v, d->normed, d->v, m, s);
+    const Proj* qkv[3] = {&L.q, &L.k, &L.v};
+    float* qkv_out[3] = {d->q, d->k, d->v};
+    int rc = gemvm_multi(3, qkv, d->normed, qkv_out, m, s);
     if (rc) return rc;
     QkPrep p;
     p.q = d->q;
@@ -420,25 +441,25 @@ int layer_stepm(rt_hip_decoder* d, int li, int m, hipStream_t s) {
     rc = chk(launch_attention2(a, d->part, d->attn_cnt, s), "decoder: attention");
     if (!rc) rc = gemvm(L.o, d->attn, d->o, m, s);
     if (rc) return rc;
-    if (!d->gemma)
-        rc = chk(launch_add(d->hidden, d->o, d->hidden, static_cast<int64_t>(m) * H, s), "decoder: residual");
-    else
-        rc = chk(launch_rmsnorm_rows(d->o, L.post_attn_norm, d->hidden, d->hidden2, H, m, c.norm_eps, true, s),
-                 "decoder: post-attention norm");
-    if (rc) return rc;
+    // the residual add (Gemma 3: of the post-attention norm) and the FFN's norm
     float* h = d->gemma ? d->hidden2 : d->hidden;
-    rc = chk(launch_rmsnorm_rows(h, L.ffn_norm, nullptr, d->normed, H, m, c.norm_eps, d->gemma, s), "decoder: rmsnorm");
-    if (!rc) rc = gemvm(L.gate, d->normed, d->gate, m, s);
-    if (!rc) rc = gemvm(L.up, d->normed, d->up, m, s);
+    rc = chk(launch_residual_rmsnorm_rows(d->o, d->gemma ? L.post_attn_norm : nullptr, d->hidden, h, L.ffn_norm,
+                                          d->normed, H, m, c.norm_eps, d->gemma, s),
+             "decoder: residual + rmsnorm");
+    const Proj* mlp[2] = {&L.gate, &L.up};
+    float* mlp_out[2] = {d->gate, d->up};
+    if (!rc) rc = gemvm_multi(2, mlp, d->normed, mlp_out, m, s);
     if (rc) return rc;
     const int64_t mf = static_cast<int64_t>(m) * F;
     rc = d->gemma ? chk(launch_gelu_mul(d->gate, d->up, d->act, mf, s), "decoder: gelu")
                   : chk(launch_swiglu(d->gate, d->up, d->act, mf, s), "decoder: swiglu");
     if (!rc) rc = gemvm(L.down, d->act, d->down, m, s);
     if (rc) return rc;
-    if (!d->gemma) return chk(launch_add(d->hidden, d->down, d->hidden, static_cast<int64_t>(m) * H, s), "decoder: residual");
-    return chk(launch_rmsnorm_rows(d->down, L.post_ffn_norm, d->hidden2, d->hidden, H, m, c.norm_eps, true, s),
-               "decoder: post-FFN norm");
+    // the same at the layer's end, with the next layer's norm or the final one
+    const float* next = li + 1 < c.n_layers ? d->layers[li + 1].attn_norm : d->out_norm;
+    return chk(launch_residual_rmsnorm_rows(d->down, d->gemma ? L.post_ffn_norm : nullptr, h, d->hidden, next,
+                                            d->normed, H, m, c.norm_eps, d->gemma, s),
+               "decoder: residual + rmsnorm");
 }
 
 // The whole step for m rows (m = 1: the single-token path).
@@ -447,6 +468,10 @@ int record_step(rt_hip_decoder* d, int m, hipStream_t s) {
     const float escale = c.embed_scale > 0.0f ? c.embed_scale : 1.0f;
     int rc = chk(launch_embed(d->embed, d->embed_format == RT_HIP_BF16, d->dstate + 1, escale, d->hidden, c.hidden, m, s),
                  "decoder: embedding");
+    if (m > 1 && !rc)  // (each layer leaves the norm that the next one reads)
+        rc = chk(launch_rmsnorm_rows(d->hidden, d->layers[0].attn_norm, nullptr, d->normed, c.hidden, m, c.norm_eps,
+                                     d->gemma, s),
+                 "decoder: rmsnorm");
     for (int li = 0; li < c.n_layers && !rc; ++li) rc = m == 1 ? layer_step1(d, li, s) : layer_stepm(d, li, m, s);
     if (rc) return rc;
     const int64_t V = d->lm_head.n, H = c.hidden;
@@ -476,10 +501,7 @@ int record_step(rt_hip_decoder* d, int m, hipStream_t s) {
                      "decoder: argmax");
         return rc;
     }
-    rc = chk(launch_rmsnorm_rows(d->hidden, d->out_norm, nullptr, d->normed, H, m, c.norm_eps, d->gemma, s),
-             "decoder: final norm");
-    if (!rc) rc = gemvm(d->lm_head, d->normed, d->logits, m, s);
-    return rc;
+    return gemvm(d->lm_head, d->normed, d->logits, m, s);
 }
 
 // Queues the copy of `elems` logits to the caller's host buffer.  A pinned
@@ -543,6 +565,20 @@ int run_step(rt_hip_decoder* d, const int32_t* tokens, int m, int32_t pos, hipSt
             take(d->lm_head);
             for (const Layer& L : d->layers)
                 for (const Proj* p : {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down}) take(*p);
+            // launches of several Q4_K projections: as one of all their rows
+            auto take_multi = [&](std::initializer_list<const Proj*> ps) {
+                Proj sum{RT_HIP_Q4K};
+                for (const Proj* p : ps)
+                    if (batch_job(*p)) {
+                        sum.n += p->n;
+                        sum.k = p->k;
+                    }
+                if (sum.n) take(sum);
+            };
+            for (const Layer& L : d->layers) {
+                take_multi({&L.q, &L.k, &L.v});
+                take_multi({&L.gate, &L.up});
+            }
             const int rc = rt_hip_reserve_workspace(need);
             if (rc) return rc;
         }

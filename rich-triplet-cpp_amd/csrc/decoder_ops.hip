@@ -108,6 +108,71 @@ __global__ __launch_bounds__(256) void k_rmsnorm_rows(const float* __restrict__ 
     }
 }
 
+// h = resid + RMSNorm(x, gamma1) or resid + x, stored, and out = RMSNorm(h,
+// gamma2): the end of one sub-layer and the start of the next for a batch of
+// rows.  Each is bound by its launch and one memory round trip, so one launch
+// costs about what either did (with q/k/v and gate/up in one launch each: five
+// launches fewer a layer, Gemma 3 4B's layers at 5 rows 99 -> 80 us each).
+template <bool NORM1, int V>
+__global__ __launch_bounds__(256) void k_residual_rmsnorm_rows(const float* __restrict__ x,
+                                                               const float* __restrict__ gamma1, const float* resid,
+                                                               float* h, const float* __restrict__ gamma2,
+                                                               float* __restrict__ out, int D, float eps, int gemma) {
+    __shared__ float red[4];
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * D;
+    const int n4 = D >> 2, tid = threadIdx.x;
+    const f32x4* x4 = reinterpret_cast<const f32x4*>(x + base);
+    const f32x4* r4 = reinterpret_cast<const f32x4*>(resid + base);
+    const f32x4* g1 = reinterpret_cast<const f32x4*>(gamma1);
+    const f32x4* g2 = reinterpret_cast<const f32x4*>(gamma2);
+    const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 xv[V], av[V], bv[V], rv[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = tid + 256 * v;
+        xv[v] = i < n4 ? x4[i] : z;
+        rv[v] = i < n4 ? r4[i] : z;
+        if constexpr (NORM1) av[v] = i < n4 ? g1[i] : z;
+        bv[v] = i < n4 ? g2[i] : z;
+    }
+    float rms_inv = 1.0f;
+    if constexpr (NORM1) {
+        float sq = 0.0f;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sq = __builtin_fmaf(xv[v][e], xv[v][e], sq);
+        sq = block_sum<256>(sq, red);
+        rms_inv = 1.0f / sqrtf(sq * (1.0f / static_cast<float>(D)) + eps);
+    }
+    f32x4* h4 = reinterpret_cast<f32x4*>(h + base);
+    float sq = 0.0f;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = tid + 256 * v;
+        if (i < n4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                xv[v][e] = rv[v][e] + (NORM1 ? (xv[v][e] * rms_inv) * (gemma ? 1.0f + av[v][e] : av[v][e]) : xv[v][e]);
+            h4[i] = xv[v];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sq = __builtin_fmaf(xv[v][e], xv[v][e], sq);
+    }
+    sq = block_sum<256>(sq, red);
+    rms_inv = 1.0f / sqrtf(sq * (1.0f / static_cast<float>(D)) + eps);
+    f32x4* o4 = reinterpret_cast<f32x4*>(out + base);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = tid + 256 * v;
+        if (i >= n4) break;
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (xv[v][e] * rms_inv) * (gemma ? 1.0f + bv[v][e] : bv[v][e]);
+        o4[i] = o;
+    }
+}
+
 // ---- q/k preparation ---------------------------------------------------------
 // Workgroup (head slot, row m): slots [0, nq) are query heads, [nq, nq+nkv)
 // key heads, [nq+nkv, nq+2nkv) value heads.  Query and key heads take the
@@ -999,6 +1064,28 @@ hipError_t launch_rmsnorm_rows(const float* x, const float* gamma, const float* 
     if (d <= 4096) return rmsnorm_v<4>(x, gamma, resid, out, d, rows, eps, gemma, s);
     if (d <= 8192) return rmsnorm_v<8>(x, gamma, resid, out, d, rows, eps, gemma, s);
     return rmsnorm_v<16>(x, gamma, resid, out, d, rows, eps, gemma, s);
+}
+
+template <int V>
+static hipError_t residual_rmsnorm_v(const float* x, const float* gamma1, const float* resid, float* h,
+                                     const float* gamma2, float* out, int64_t d, int rows, float eps, bool gemma,
+                                     hipStream_t s) {
+    if (gamma1)
+        hipLaunchKernelGGL((k_residual_rmsnorm_rows<true, V>), dim3(static_cast<unsigned>(rows)), dim3(256), 0, s, x,
+                           gamma1, resid, h, gamma2, out, static_cast<int>(d), eps, gemma ? 1 : 0);
+    else
+        hipLaunchKernelGGL((k_residual_rmsnorm_rows<false, V>), dim3(static_cast<unsigned>(rows)), dim3(256), 0, s, x,
+                           gamma1, resid, h, gamma2, out, static_cast<int>(d), eps, gemma ? 1 : 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_residual_rmsnorm_rows(const float* x, const float* gamma1, const float* resid, float* h,
+                                        const float* gamma2, float* out, int64_t d, int rows, float eps, bool gemma,
+                                        hipStream_t s) {
+    if (d % 4 != 0 || d > 16384) return hipErrorInvalidValue;
+    if (d <= 4096) return residual_rmsnorm_v<4>(x, gamma1, resid, h, gamma2, out, d, rows, eps, gemma, s);
+    if (d <= 8192) return residual_rmsnorm_v<8>(x, gamma1, resid, h, gamma2, out, d, rows, eps, gemma, s);
+    return residual_rmsnorm_v<16>(x, gamma1, resid, h, gamma2, out, d, rows, eps, gemma, s);
 }
 
 static PrepArgs prep_args(const QkPrep& p) {

@@ -349,14 +349,25 @@ __device__ __forceinline__ float ld_dev(const float* p) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Several weights on the same x in one launch: the tiles of the `count` jobs
+// one after another (each N a multiple of 16, so a tile has one job); first[j]
+// is job j's first tile.  Unused entries repeat the last job.
+constexpr int kMaxJobs = 3;
+struct BatchJobs {
+    const uint8_t* w[kMaxJobs];
+    float* y[kMaxJobs];
+    int n[kMaxJobs], first[kMaxJobs];
+};
+
 // XP: units of 8 activations a thread holds while staging one chunk.  Up to 4
 // the kernel fits 128 registers, so two workgroups may share a CU.
-template <class F, int Q, int XP, int NW>
+// MULTI: W, n and Y of each tile come from `jobs`; n is the sum.
+template <class F, int Q, int XP, int NW, bool MULTI>
 __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __restrict__ W, const float* __restrict__ X,
                                                          int k, int m, int n, int ks_log, int cslots, int nslots,
                                                          int groups, int per, float* __restrict__ Y, int nchunks,
                                                          int64_t sc_off, float* __restrict__ P,
-                                                         uint32_t* __restrict__ counters) {
+                                                         uint32_t* __restrict__ counters, const BatchJobs jobs) {
     // (the arguments before Y are preloaded into SGPRs at wave launch)
     const BatchShape S{n, k, m, ks_log, groups, nslots, cslots, nchunks, per, static_cast<int>(gridDim.y), NW, sc_off};
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -462,7 +473,19 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
     };
 
     int group = blockIdx.x, chunk = blockIdx.y;
-    auto tile_of = [&](int grp) { return F::tile(W, S.sc_off, 16 * (grp * TW + tw), S.n, S.k, lane); };
+    auto job_of = [&](int t) { return t >= jobs.first[2] ? 2 : (t >= jobs.first[1] ? 1 : 0); };
+    auto tile_of = [&](int grp) {
+        const int t = grp * TW + tw;
+        if constexpr (MULTI) {
+            const int j = job_of(t);
+            const uint8_t* const w = j == 2 ? jobs.w[2] : (j == 1 ? jobs.w[1] : jobs.w[0]);
+            const int n = j == 2 ? jobs.n[2] : (j == 1 ? jobs.n[1] : jobs.n[0]);
+            const int first = j == 2 ? jobs.first[2] : (j == 1 ? jobs.first[1] : 0);
+            return F::tile(w, S.sc_off, 16 * (t - first), n, S.k, lane);
+        } else {
+            return F::tile(W, S.sc_off, 16 * t, S.n, S.k, lane);
+        }
+    };
     typename F::Tile cur = tile_of(group);
     typename F::Slot ring[kDepth];
     // Slot i of this wave in chunk c (none past the chunk's end: an empty
@@ -630,9 +653,17 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 if (tid == 0) __hip_atomic_store(counters + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             if (mine) {
+                float* y = Y;
+                int yn = S.n, yrow = row;
+                if constexpr (MULTI) {
+                    const int j = job_of(group * TW + tw);
+                    y = j == 2 ? jobs.y[2] : (j == 1 ? jobs.y[1] : jobs.y[0]);
+                    yn = j == 2 ? jobs.n[2] : (j == 1 ? jobs.n[1] : jobs.n[0]);
+                    yrow -= 16 * (j == 2 ? jobs.first[2] : (j == 1 ? jobs.first[1] : 0));
+                }
 #pragma unroll
                 for (int q = 0; q < Q; ++q)
-                    if (4 * q + g < S.m) Y[static_cast<int64_t>(4 * q + g) * S.n + row] = v[q];
+                    if (4 * q + g < S.m) y[static_cast<int64_t>(4 * q + g) * yn + yrow] = v[q];
             }
         }
         if (ngroup >= S.groups) break;
@@ -728,8 +759,10 @@ bool plan(int64_t n, int64_t k, int m, bool sliced, BatchShape* out) {
     return cost >= 0.0;
 }
 
-template <class F, int Q>
-hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, int64_t sc_off, hipStream_t s) {
+// jobs: null for one weight w, else n is the sum of theirs (w and y unused).
+template <class F, int Q, bool MULTI = false>
+hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, int64_t sc_off, hipStream_t s,
+               const BatchJobs* jobs = nullptr) {
     BatchShape S;
     if (!plan<F, Q>(n, k, m, true, &S)) return hipErrorInvalidValue;
     float* part = nullptr;
@@ -754,16 +787,17 @@ hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, in
     const int threads = S.waves * kWave;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(static_cast<unsigned>(threads)), lds, s, static_cast<const uint8_t*>(w), x, S.k, S.m, S.n,
-                           S.ks_log, S.cslots, S.nslots, S.groups, S.per, y, S.nchunks, S.sc_off, part, counters);
+                           S.ks_log, S.cslots, S.nslots, S.groups, S.per, y, S.nchunks, S.sc_off, part, counters,
+                           MULTI ? *jobs : BatchJobs{});
         return hipGetLastError();
     };
     const int xp = static_cast<int>((static_cast<int64_t>(S.cslots) * F::kSteps * 4 * m + threads - 1) / threads);
     if constexpr (F::kInt && Q == 2) {
-        if (S.waves == 16) return go(k_gemv_batch<F, Q, 4, 16>);
+        if (S.waves == 16) return go(k_gemv_batch<F, Q, 4, 16, MULTI>);
     }
-    if (xp <= 2) return go(k_gemv_batch<F, Q, 2, kWaves>);
-    if (xp <= 4) return go(k_gemv_batch<F, Q, 4, kWaves>);
-    return go(k_gemv_batch<F, Q, 8, kWaves>);
+    if (xp <= 2) return go(k_gemv_batch<F, Q, 2, kWaves, MULTI>);
+    if (xp <= 4) return go(k_gemv_batch<F, Q, 4, kWaves, MULTI>);
+    return go(k_gemv_batch<F, Q, 8, kWaves, MULTI>);
 }
 
 template <class F>
@@ -803,6 +837,25 @@ hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, i
             return dispatch<BQ4m>(w, x, y, n, k, m, static_cast<int64_t>(q4mat_scales_offset(n, k)), s);
     }
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_gemv_batch_q4k_multi(int count, const void* const* w, const float* x, float* const* y,
+                                       const int64_t* n, int64_t k, int m, hipStream_t s) {
+    if (count < 1 || count > kMaxJobs || m < 2 || m > 8) return hipErrorInvalidValue;
+    BatchJobs jobs;
+    int64_t total = 0;
+    for (int j = 0; j < kMaxJobs; ++j) {
+        const int i = j < count ? j : count - 1;
+        if (n[i] % 16 != 0) return hipErrorInvalidValue;
+        jobs.w[j] = static_cast<const uint8_t*>(w[i]);
+        jobs.y[j] = y[i];
+        jobs.n[j] = static_cast<int>(n[i]);
+        jobs.first[j] = j < count ? static_cast<int>(total / 16) : jobs.first[i];
+        if (j < count) total += n[i];
+    }
+    if (total > 0x7fffffff) return hipErrorInvalidValue;
+    return m <= 4 ? run<BQ4k, 1, true>(nullptr, x, nullptr, total, k, m, 0, s, &jobs)
+                  : run<BQ4k, 2, true>(nullptr, x, nullptr, total, k, m, 0, s, &jobs);
 }
 
 }  // namespace rt_hip

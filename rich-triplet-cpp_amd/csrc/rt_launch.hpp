@@ -139,6 +139,10 @@ hipError_t launch_gemv_bf16_m1(const uint16_t* w, const float* x, float* y, int6
 // the room.
 hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, int64_t n, int64_t k, int m,
                              hipStream_t s);
+// The same for up to three Q4_K weights on one x (m >= 2, each n a multiple of
+// 16): one launch; its workspace is that of one weight of sum(n) rows.
+hipError_t launch_gemv_batch_q4k_multi(int count, const void* const* w, const float* x, float* const* y,
+                                       const int64_t* n, int64_t k, int m, hipStream_t s);
 // Workspace bytes one launch_gemv_batch call takes when they are there.
 size_t gemv_batch_workspace_bytes(int fmt, int64_t n, int64_t k, int m);
 // M = 1 GGUF Q4_0 GEMV (gemv_q40.hip); LDS q40_m1_lds_bytes(k).
@@ -205,6 +209,12 @@ hipError_t launch_embed(const void* table, bool bf16, const int32_t* tokens, flo
 // RMSNorm of `rows` rows of d (gamma or 1 + gamma); with resid: out = resid + norm.
 hipError_t launch_rmsnorm_rows(const float* x, const float* gamma, const float* resid, float* out, int64_t d,
                                int rows, float eps, bool gemma, hipStream_t s);
+// Two steps of the residual stream in one launch, bit for bit as two:
+// h = resid + RMSNorm(x, gamma1) (gamma1 null: resid + x), then
+// out = RMSNorm(h, gamma2).  h may be resid.
+hipError_t launch_residual_rmsnorm_rows(const float* x, const float* gamma1, const float* resid, float* h,
+                                        const float* gamma2, float* out, int64_t d, int rows, float eps, bool gemma,
+                                        hipStream_t s);
 // q/k preparation for m rows at positions pos[0] + row: optional per-head
 // RMSNorm (1 + gamma), RoPE, and the K/V append into the cache.
 struct QkPrep {
