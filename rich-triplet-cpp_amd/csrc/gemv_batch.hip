@@ -328,6 +328,12 @@ __device__ __forceinline__ float quad_max(float v) {
     return v;
 }
 
+__device__ __forceinline__ uint32_t quad_max(uint32_t v) {
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xb1, 0xf, 0xf, false)));
+    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4e, 0xf, 0xf, false)));
+    return v;
+}
+
 // One launch's shape: tile groups of waves / KS tiles (KS = 1 << ks_log); K
 // in `nslots` slots, staged `cslots` at a time.
 // With slices > 1 (grid y) a workgroup takes one chunk alone and the chunks'
@@ -436,7 +442,16 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 // Block (step, m) is the quad of units g = 0..3.
                 float amax = fmaxf(fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))),
                                    fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3]))));
-                amax = quad_max(amax);
+                if constexpr (!F::kMin) {
+                    // fmaxf passes NaNs over; they are the largest of the bit
+                    // patterns (Q4_K's sum carries them)
+                    const bool nan = __builtin_isunordered(a[0], a[1]) | __builtin_isunordered(a[2], a[3]) |
+                                     __builtin_isunordered(b[0], b[1]) | __builtin_isunordered(b[2], b[3]);
+                    amax = nan ? __uint_as_float(0x7fc00000u) : amax;
+                    amax = __uint_as_float(quad_max(__float_as_uint(amax)));
+                } else {
+                    amax = quad_max(amax);
+                }
                 float sc, inv;
                 q4k_mfma::sub_block_scale(amax, sc, inv);
                 uint32_t a0, a1, a2, b0, b1, b2;

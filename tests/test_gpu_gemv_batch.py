@@ -120,3 +120,25 @@ def test_batched_gemv_without_workspace_room(rt, orc):
         graph.replay()
         torch.cuda.synchronize()
         assert normwise_err(from_dev(y), x.astype(np.float64) @ v.T) <= GEMV_TOL
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "bf16", "q4_0", "q4mat"])
+def test_batched_gemv_nonfinite_rows(rt, orc, fmt):
+    """One NaN or infinity in a row of x makes that row of y NaN or infinite,
+    as an f32 sum with nonzero terms would, and leaves the other rows' bits."""
+    n, k = 40, 768
+    for m, bad in [(3, 1), (8, 6)]:
+        rng = np.random.default_rng(m)
+        w, _ = weights(rt, orc, fmt, rng, n, k)
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        clean = run(rt, fmt, w, x, n, k)
+        for value in (np.nan, np.inf, -np.inf):
+            for at in (0, 421, k - 1):
+                say(f"[gemv batch {fmt}] M = {m}, {value} at {at}")
+                z = x.copy()
+                z[bad, at] = value
+                y = run(rt, fmt, w, z, n, k)
+                assert not np.isfinite(y[bad]).any()
+                if np.isnan(value):
+                    assert np.isnan(y[bad]).all()
+                assert np.array_equal(np.delete(y, bad, 0), np.delete(clean, bad, 0))
