@@ -367,14 +367,19 @@ struct BatchJobs {
 
 // XP: units of 8 activations a thread holds while staging one chunk.  Up to 4
 // the kernel fits 128 registers, so two workgroups may share a CU.
-// MULTI: W, n and Y of each tile come from `jobs`; n is the sum.
-template <class F, int Q, int XP, int NW, bool MULTI>
+// FORM kMulti: W, n and Y of each tile come from `jobs`; n is the sum.  kBias:
+// bias[n] is added as a row is stored (a form of its own: a test of the pointer
+// in the others cost Q4_K batches of 8 rows 1.4%).
+enum Form { kOne = 0, kMulti = 1, kBias = 2 };
+template <class F, int Q, int XP, int NW, int FORM>
 __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __restrict__ W, const float* __restrict__ X,
                                                          int k, int m, int n, int ks_log, int cslots, int nslots,
                                                          int groups, int per, float* __restrict__ Y, int nchunks,
                                                          int64_t sc_off, float* __restrict__ P,
-                                                         uint32_t* __restrict__ counters, const BatchJobs jobs) {
+                                                         uint32_t* __restrict__ counters,
+                                                         const float* __restrict__ bias, const BatchJobs jobs) {
     // (the arguments before Y are preloaded into SGPRs at wave launch)
+    constexpr bool MULTI = FORM == kMulti;
     const BatchShape S{n, k, m, ks_log, groups, nslots, cslots, nchunks, per, static_cast<int>(gridDim.y), NW, sc_off};
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int kLimb = limb_bytes<F>(Q), kCst = cst_bytes<F>(Q), kThreads = NW * kWave;
@@ -611,7 +616,8 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
         if (last_chunk) {
             // Row n of the tile, activation row 4q + g.
             const int row = 16 * (group * TW + tw) + (lane & 15);
-            float v[Q];
+            float v[Q], add = 0.0f;
+            if constexpr (FORM == kBias) add = bias[min(row, S.n - 1)];
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
                 v[q] = F::kInt ? acc[q] : (C[q][0] + C[q][1]) + C[q][2];
@@ -668,6 +674,9 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 if (tid == 0) __hip_atomic_store(counters + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             if (mine) {
+                if constexpr (FORM == kBias)
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) v[q] += add;
                 float* y = Y;
                 int yn = S.n, yrow = row;
                 if constexpr (MULTI) {
@@ -775,9 +784,9 @@ bool plan(int64_t n, int64_t k, int m, bool sliced, BatchShape* out) {
 }
 
 // jobs: null for one weight w, else n is the sum of theirs (w and y unused).
-template <class F, int Q, bool MULTI = false>
+template <class F, int Q, int FORM>
 hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, int64_t sc_off, hipStream_t s,
-               const BatchJobs* jobs = nullptr) {
+               const float* bias, const BatchJobs* jobs = nullptr) {
     BatchShape S;
     if (!plan<F, Q>(n, k, m, true, &S)) return hipErrorInvalidValue;
     float* part = nullptr;
@@ -802,23 +811,27 @@ hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, in
     const int threads = S.waves * kWave;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(static_cast<unsigned>(threads)), lds, s, static_cast<const uint8_t*>(w), x, S.k, S.m, S.n,
-                           S.ks_log, S.cslots, S.nslots, S.groups, S.per, y, S.nchunks, S.sc_off, part, counters,
-                           MULTI ? *jobs : BatchJobs{});
+                           S.ks_log, S.cslots, S.nslots, S.groups, S.per, y, S.nchunks, S.sc_off, part, counters, bias,
+                           FORM == kMulti ? *jobs : BatchJobs{});
         return hipGetLastError();
     };
     const int xp = static_cast<int>((static_cast<int64_t>(S.cslots) * F::kSteps * 4 * m + threads - 1) / threads);
     if constexpr (F::kInt && Q == 2) {
-        if (S.waves == 16) return go(k_gemv_batch<F, Q, 4, 16, MULTI>);
+        if (S.waves == 16) return go(k_gemv_batch<F, Q, 4, 16, FORM>);
     }
-    if (xp <= 2) return go(k_gemv_batch<F, Q, 2, kWaves, MULTI>);
-    if (xp <= 4) return go(k_gemv_batch<F, Q, 4, kWaves, MULTI>);
-    return go(k_gemv_batch<F, Q, 8, kWaves, MULTI>);
+    if (xp <= 2) return go(k_gemv_batch<F, Q, 2, kWaves, FORM>);
+    if (xp <= 4) return go(k_gemv_batch<F, Q, 4, kWaves, FORM>);
+    return go(k_gemv_batch<F, Q, 8, kWaves, FORM>);
 }
 
 template <class F>
 hipError_t dispatch(const void* w, const float* x, float* y, int64_t n, int64_t k, int m, int64_t sc_off,
-                    hipStream_t s) {
-    return m <= 4 ? run<F, 1>(w, x, y, n, k, m, sc_off, s) : run<F, 2>(w, x, y, n, k, m, sc_off, s);
+                    hipStream_t s, const float* bias) {
+    if (bias)
+        return m <= 4 ? run<F, 1, kBias>(w, x, y, n, k, m, sc_off, s, bias)
+                      : run<F, 2, kBias>(w, x, y, n, k, m, sc_off, s, bias);
+    return m <= 4 ? run<F, 1, kOne>(w, x, y, n, k, m, sc_off, s, nullptr)
+                  : run<F, 2, kOne>(w, x, y, n, k, m, sc_off, s, nullptr);
 }
 
 template <class F>
@@ -842,14 +855,14 @@ size_t gemv_batch_workspace_bytes(int fmt, int64_t n, int64_t k, int m) {
 }
 
 hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, int64_t n, int64_t k, int m,
-                             hipStream_t s) {
+                             hipStream_t s, const float* bias) {
     if (m < 1 || m > 8) return hipErrorInvalidValue;
     switch (fmt) {
-        case RT_HIP_Q4K: return dispatch<BQ4k>(w, x, y, n, k, m, 0, s);
-        case RT_HIP_BF16: return dispatch<BBf16>(w, x, y, n, k, m, 0, s);
-        case RT_HIP_Q4_0: return dispatch<BQ40>(w, x, y, n, k, m, 0, s);
+        case RT_HIP_Q4K: return dispatch<BQ4k>(w, x, y, n, k, m, 0, s, bias);
+        case RT_HIP_BF16: return dispatch<BBf16>(w, x, y, n, k, m, 0, s, bias);
+        case RT_HIP_Q4_0: return dispatch<BQ40>(w, x, y, n, k, m, 0, s, bias);
         case RT_HIP_Q4MAT:
-            return dispatch<BQ4m>(w, x, y, n, k, m, static_cast<int64_t>(q4mat_scales_offset(n, k)), s);
+            return dispatch<BQ4m>(w, x, y, n, k, m, static_cast<int64_t>(q4mat_scales_offset(n, k)), s, bias);
     }
     return hipErrorInvalidValue;
 }
@@ -869,8 +882,8 @@ hipError_t launch_gemv_batch_q4k_multi(int count, const void* const* w, const fl
         if (j < count) total += n[i];
     }
     if (total > 0x7fffffff) return hipErrorInvalidValue;
-    return m <= 4 ? run<BQ4k, 1, true>(nullptr, x, nullptr, total, k, m, 0, s, &jobs)
-                  : run<BQ4k, 2, true>(nullptr, x, nullptr, total, k, m, 0, s, &jobs);
+    return m <= 4 ? run<BQ4k, 1, kMulti>(nullptr, x, nullptr, total, k, m, 0, s, nullptr, &jobs)
+                  : run<BQ4k, 2, kMulti>(nullptr, x, nullptr, total, k, m, 0, s, nullptr, &jobs);
 }
 
 }  // namespace rt_hip

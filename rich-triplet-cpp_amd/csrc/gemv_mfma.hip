@@ -60,7 +60,11 @@ struct Jobs {
 // (the first index of the strict maximum, NaN never chosen:
 // transformer5.cpp:382-391), one key per 16-row tile in Rope::keys; a
 // second launch folds those (launch_argmax_reduce).
-enum Epi { kEpiNone = 0, kEpiRope = 1, kEpiAdd = 2, kEpiArgmax = 3 };
+// kEpiBias: add the row's bias (aux).  A bias added by a second launch costs
+// that launch and a round trip of y: 3072 x 3072 called eagerly 13.3 us with
+// two launches, 10.4 with one.
+enum Epi { kEpiNone = 0, kEpiRope = 1, kEpiAdd = 2, kEpiArgmax = 3, kEpiBias = 4 };
+constexpr bool adds(int epi) { return epi == kEpiAdd || epi == kEpiBias; }
 
 struct Rope {
     const float* inv_freq = nullptr;  // [head_dim / 2], device
@@ -454,7 +458,7 @@ __device__ __forceinline__ void q4k_tiles(int blk, const float* __restrict__ X, 
 
     // The epilogue's own operands, loaded right behind the prologue so that
     // their latency passes while the weights stream rather than after the
-    // last product: the value a row adds to (kEpiAdd), the position and the
+    // last product: the value a row adds to (kEpiAdd, kEpiBias), the position and the
     // row's rotation frequency (kEpiRope).  Lanes past 16 and tile slots past
     // the last tile read a row of the job that exists, unused.
     const int row = row0 + ln.n;
@@ -465,6 +469,7 @@ __device__ __forceinline__ void q4k_tiles(int blk, const float* __restrict__ X, 
     using GF = const __attribute__((address_space(1))) float;
     float y_old = 0.0f;
     if constexpr (EPI == kEpiAdd) y_old = ((GF*)yj)[min(row, n_job - 1)];
+    if constexpr (EPI == kEpiBias) y_old = ((GF*)aux)[min(row, n_job - 1)];
     int rpos = 0;
     float rfreq = 0.0f;
     if constexpr (EPI == kEpiRope) {
@@ -478,7 +483,7 @@ __device__ __forceinline__ void q4k_tiles(int blk, const float* __restrict__ X, 
     // alone (XP * nthreads >= K/4, checked by the host), then convert.
     // (The residual load above is younger still: this wait leaves it.)
     if constexpr (CW == 0) {
-    wait_vmcnt<3 * D + (EPI == kEpiAdd ? 1 : 0)>();
+    wait_vmcnt<3 * D + (adds(EPI) ? 1 : 0)>();
     // x past the register batch (K above XP * nthreads * 4): loaded after
     // the weight prologue, so its waits are full ones; large K only.
     float rest_sq = 0.0f;
@@ -602,7 +607,7 @@ __device__ __forceinline__ void q4k_tiles(int blk, const float* __restrict__ X, 
     };
     if (KS == 1) {
         const float out = finish(v);
-        if (lane < 16 && keep) yj[drow] = EPI == kEpiAdd ? y_old + out : out;
+        if (lane < 16 && keep) yj[drow] = adds(EPI) ? y_old + out : out;
         keep_key(out);
     } else {
         float* red = reinterpret_cast<float*>(lds + lds_bytes(K));  // [TPW][KS][16]
@@ -614,7 +619,7 @@ __device__ __forceinline__ void q4k_tiles(int blk, const float* __restrict__ X, 
 #pragma unroll
             for (int q = 1; q < KS; ++q) s += rp[q * 16 + (lane & 15)];
             const float out = finish(s);
-            if (lane < 16 && keep) yj[drow] = EPI == kEpiAdd ? y_old + out : out;
+            if (lane < 16 && keep) yj[drow] = adds(EPI) ? y_old + out : out;
             keep_key(out);
         }
     }
@@ -644,12 +649,12 @@ __global__ __launch_bounds__(CW > 0 ? 1024 : kMaxThreads) void k_gemv_q4k_mfma(
 // The same with a layer operation applied to x while it is staged (XOp).
 // Pointers first, then the 32-bit arguments: no padding, so all fourteen
 // leading dwords (aux, gamma or up, included) are preloaded.
-template <int XP, bool J34, int XOP, int EPI, int CW>
+template <int XP, bool TILED, bool J34, int XOP, int EPI, int CW>
 __global__ __launch_bounds__(CW > 0 ? 1024 : kMaxThreads) void k_gemv_q4k_xop(
     const float* __restrict__ X, const float* __restrict__ aux, const uint8_t* w0, const uint8_t* w1, int K,
     uint32_t split, int nthreads, int n0, int n1, int tile1, const Jobs jobs, float eps, const Rope rope) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    q4k_tiles<4, XP, true, J34, XOP, EPI, CW>(static_cast<int>(blockIdx.x), X, K, split, nthreads, w0, w1, n0, n1,
+    q4k_tiles<4, XP, TILED, J34, XOP, EPI, CW>(static_cast<int>(blockIdx.x), X, K, split, nthreads, w0, w1, n0, n1,
                                                tile1, jobs, lds, aux, eps, rope);
 }
 
@@ -721,8 +726,9 @@ hipError_t run(const Jobs& jobs, const float* x, const XArgs& xa, int64_t k, int
         hipLaunchKernelGGL((k_gemv_q4k_postnorm<J34>), g, b, lds, s, x, xa.pn.b, xa.aux, jobs.w[0], jobs.w[1],
                            static_cast<int>(k), split, jobs.n[0], jobs.n[1], jobs, xa.eps, xa.pn);
     } else {
-        static_assert(D == 4 && TILED, "x operations and RoPE run on the tiled layout, ring depth 4");
-        hipLaunchKernelGGL((k_gemv_q4k_xop<XP, J34, XOP, EPI, CW>), g, b, lds, s, x, xa.aux, jobs.w[0], jobs.w[1],
+        static_assert(D == 4 && (TILED || EPI == kEpiBias),
+                      "x operations and RoPE run on the tiled layout, ring depth 4");
+        hipLaunchKernelGGL((k_gemv_q4k_xop<XP, TILED, J34, XOP, EPI, CW>), g, b, lds, s, x, xa.aux, jobs.w[0], jobs.w[1],
                            static_cast<int>(k), split, all * kWave, jobs.n[0], jobs.n[1], jobs.tile0[1], jobs,
                            xa.eps, xa.rope);
     }
@@ -740,8 +746,8 @@ hipError_t run_xp(const Jobs& jobs, const float* x, const XArgs& xa, int64_t k, 
     // At most 16 float4 per thread in registers, 8 with an x operation (its
     // second vector doubles the registers); the rest of a longer x is
     // staged by a loop after them.
-    constexpr bool kPlain = XOP == kXNone && EPI == kEpiNone;
-    if (jobs.count > 2) {
+    constexpr bool kPlain = XOP == kXNone;  // (kHasRest: 16 f32x4, then the loop)
+    if (EPI != kEpiBias && jobs.count > 2) {
         if (per <= 2) return run<D, 2, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
         if (per <= 3) return run<D, 3, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
         if (per <= 4) return run<D, 4, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
@@ -1061,6 +1067,13 @@ hipError_t launch_gemv_q4k_bf16_fused(int count, const void* const* w, float* co
         case kXRmsNorm1: return fused_xp<kXRmsNorm1, kEpiNone>(jobs, ks, q4k_wgs, wb, yb, nb_rows, x, xa, k, lds, s);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_gemv_q4k_bias(const void* w, const float* x, const float* bias, float* y, int64_t n, int64_t k,
+                                hipStream_t s) {
+    XArgs xa;
+    xa.aux = bias;
+    return dispatch<false, kXNone, kEpiBias>(make_jobs(1, &w, &y, &n), x, k, s, xa);
 }
 
 hipError_t launch_gemv_q4k_mfma(const void* w, const float* x, float* y, int64_t n, int64_t k,

@@ -42,6 +42,9 @@ uint32_t* arrival_counters(hipStream_t s, hipError_t* err);
 
 hipError_t launch_gemv_q4k_mfma(const void* w, const float* x, float* y, int64_t n, int64_t k,
                                 hipStream_t s);
+// The same plus bias[n] in one launch.
+hipError_t launch_gemv_q4k_bias(const void* w, const float* x, const float* bias, float* y, int64_t n, int64_t k,
+                                hipStream_t s);
 // Up to four M = 1 Q4_K GEMVs sharing x, K; `tiled`: the weights are in the
 // tiled layout (q4k_mfma.hpp) rather than reference row-major blocks.
 // FLUX attention (flux_attention.hip): q, k, v, out [t][n_heads * head_dim]
@@ -137,8 +140,9 @@ hipError_t launch_gemv_bf16_m1(const uint16_t* w, const float* x, float* y, int6
 // is read once for all m rows.  Long K at several rows is split over
 // workgroups through the library workspace where that has (or may grow to)
 // the room.
+// `bias` (n floats, may be null) is added to every row.
 hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, int64_t n, int64_t k, int m,
-                             hipStream_t s);
+                             hipStream_t s, const float* bias = nullptr);
 // The same for up to three Q4_K weights on one x (m >= 2, each n a multiple of
 // 16): one launch; its workspace is that of one weight of sum(n) rows.
 hipError_t launch_gemv_batch_q4k_multi(int count, const void* const* w, const float* x, float* const* y,
