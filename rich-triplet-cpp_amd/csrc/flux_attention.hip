@@ -557,7 +557,7 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
     }
 }
 
-// Workgroup slots of the 8-wave form: one per CU (96 KB of LDS at 128 dims,
+// Workgroup slots of the 8-wave form: one per CU (152 KB of LDS at 128 dims,
 // 256 registers a wave).
 int flux_slots() { return static_cast<int>(device_info().cus); }
 
