@@ -992,7 +992,8 @@ def bench_flux_attention(args, rt, torch):
     """FLUX.1 attention at 1024x1024 (metal_flux.mm:254-272 over
     flux.cpp:287-321): t = 4352 tokens (4096 image + 256 text), 24 heads of
     128, f32 throughout.  One launch per step, captured in a graph; it is
-    the roofline kernel (matrix cores; the peak quoted is the f32 unit's).  Algorithmic flops: 2 t^2 d per
+    the roofline kernel (matrix cores: six bf16 products for each f32 one, so the peak is a sixth of
+    bf16's).  Algorithmic flops: 2 t^2 d per
     head for the scores and 2 t^2 d for the weighted sum of v."""
     import numpy as np
     t, h, d = 4352, 24, 128
@@ -1007,8 +1008,8 @@ def bench_flux_attention(args, rt, torch):
     flops = 4 * t * t * d * h
     tf = flops / (ms * 1e-3) / 1e12
     log(f"[bench] flux attention {ms * 1e3:.1f} us, {tf:.1f} TFLOP/s f32")
-    roof = {"bound": "mfma", "achieved": round(tf, 2), "peak": F32_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": round(tf / F32_PEAK_TFLOPS, 4), "traffic": None,
+    roof = {"bound": "mfma", "achieved": round(tf, 2), "peak": round(BF16_PEAK_TFLOPS / 6, 1), "unit": "TFLOP/s",
+            "frac": round(6 * tf / BF16_PEAK_TFLOPS, 4), "traffic": None,
             "kernel": "k_flux_attn<128, 8> (f32 as 3 bf16 limbs, 6 products on MFMA 32x32x16, online "
                       "softmax, 256 queries x 32-key tiles)",
             "us_per_launch": round(ms * 1e3, 2), "flops_per_launch": flops}
