@@ -8,26 +8,30 @@
 //  * B is the weight tile: lane l = (n = l%16, g = l/16) supplies 8 weights
 //    of row n; the same 8 positions of the activations stand in A, so each
 //    format picks the positions its bytes hold (Fmt::kX*).
-//  * A row i = 4t + lambda (lambda < 3) is limb lambda of activation row
-//    4q + t.  Rows i with lambda == 3 or past M hold whatever lies in LDS:
-//    a row of A reaches only its own row of the result, and theirs are unused.
-//  * The output lane (n, g) holds C[4g + r][n], r = 0..3: the three limb
-//    dots of activation row 4q + g for weight row n, combined in the lane.
+//  * A row i = 4t + lambda (lambda < Fmt::kLimbs) is limb lambda of activation
+//    row 4q + t.  Rows i with no limb or past M hold whatever lies in LDS: a
+//    row of A reaches only its own row of the result, and theirs are unused.
+//  * The output lane (n, g) holds C[4g + r][n], r = 0..3: the limb dots of
+//    activation row 4q + g for weight row n, combined in the lane.
 //
 // Exact activation limbs, so that the MFMA products are exact:
 //  * BF16 weights (v_mfma_f32_16x16x32_bf16): three bf16 limbs with
 //    h + m + l == x exactly.  Products of bf16 values are exact in f32, so
 //    only the f32 accumulation rounds, as in an f32 dot product.
 //  * 4-bit weights (v_mfma_i32_16x16x32_i8): the step is one 32-value block
-//    with one scale, and x carries the int8 limbs of the M = 1 kernel
-//    (q4k_mfma.hpp): per block a power-of-two s and A0 + A1/256 + A2/65536
-//    == x / s to 2.5e-7 * absmax.  Each limb dot is an exact int32.
-//    - Q4_K: nibbles 0..15, so R = C0 * 65536 + C1 * 256 + C2 stays below
-//      32 * 15 * 2^22 < 2^31 and is converted once; the minimum's term,
-//      -(dmin * mv_j) * sum(x), is a contraction over the super-block's eight
-//      sub-blocks and runs on v_mfma_f32_16x16x4_f32 (quant_q4k.cpp:482-523).
-//    - Q4_0, Q4Mat: signed values (nibble - 8, or the two's-complement
-//      nibble) as int8 multiples of 16, so no offset term is left.
+//    with one scale, and x is a fixed-point integer of int8 limbs times a
+//    power of two per block.  Each limb dot is an exact int32.
+//    - Q4_K: the three limbs of the M = 1 kernel (q4k_mfma.hpp), within 2.5e-7
+//      of the block's absmax.  Nibbles 0..15, so R = C0 * 65536 + C1 * 256 +
+//      C2 stays below 32 * 15 * 2^22 < 2^31 and is converted once; the
+//      minimum's term, -(dmin * mv_j) * sum(x), is a contraction over the
+//      super-block's eight sub-blocks and runs on v_mfma_f32_16x16x4_f32
+//      (quant_q4k.cpp:482-523).
+//    - Q4_0, Q4Mat: four limbs (fixed4()), within 2^-30 of the block's absmax:
+//      an f32 sum of the block's products rounds by more, also where a value
+//      stands beside one a thousand times as large.  Signed values (nibble - 8,
+//      or the two's-complement nibble) as int8 multiples of 16, so no offset
+//      term is left.  The fourth limb's row of A costs no MFMA.
 //
 // Work split: a workgroup of 8 waves stages all M rows as limbs in LDS, KS
 // waves share a 16-row tile's K (slots ks, ks + KS, ...) and their sums meet
@@ -47,9 +51,11 @@
 //   Q4_K  8192 x 3072  M = 4: 8.4 -> 7.7   M = 8: 10.0 -> 9.9
 //   Q4_K  3072 x 8192  M = 4: 11.8 -> 10.3 M = 8: 14.5 -> 13.6
 //   BF16  3072 x 3072  M = 4: 10.8 -> 8.1  M = 8: 11.7 -> 10.2
-//   Q4_0  4096 x 4096  M = 4: 19.3 -> 6.2  M = 8: 30.2 -> 8.4 (VALU before)
-//   Q4_0  4096 x 11008 M = 4: 248 -> 12.5  M = 8: 626 -> 15.7
-//   Q4Mat 4096 x 4096  M = 4: 16.4 -> 6.6  M = 8: 53.2 -> 9.4 (VALU before)
+//   Q4_0  4096 x 4096  M = 4: 18.6 -> 6.3  M = 8: 29.3 -> 9.2 (VALU before)
+//   Q4_0  4096 x 11008 M = 4: 246 -> 11.4  M = 8: 616 -> 15.3
+//   Q4Mat 4096 x 4096  M = 4: 15.9 -> 6.4  M = 8: 52.1 -> 9.7 (VALU before)
+// (With three limbs Q4_0 and Q4Mat took 5% less at M = 8 and the same at M = 4,
+// and were up to 4 times as far from float64 as the VALU kernels.)
 #include "q4k_mfma.hpp"
 #include "rt_common.hpp"
 #include "rt_launch.hpp"
@@ -71,6 +77,7 @@ constexpr uint32_t kNoRead = 0x7ffffff0u;
 
 struct BBf16 {
     static constexpr bool kInt = false, kMin = false;
+    static constexpr int kLimbs = 3;
     static constexpr int kSteps = 4;  // 128 values
     static constexpr int kX0 = 8, kX1 = 4;  // lane group g: values 8g.. and 8g + 4..
     static constexpr bool kTail = true;     // K need not be whole slots
@@ -110,6 +117,7 @@ __device__ __forceinline__ long pair64(uint32_t lo, uint32_t hi) {
 
 struct BQ4k {
     static constexpr bool kInt = true, kMin = true;
+    static constexpr int kLimbs = 3;
     static constexpr int kSteps = 8;  // one super-block
     static constexpr int kX0 = 8, kX1 = 4;
     static constexpr bool kTail = false;
@@ -184,6 +192,33 @@ __device__ __forceinline__ void gather4(uint32_t v, uint32_t (&o)[4]) {
     o[2] = e[1];
     o[3] = d[1];
 }
+// The scale of a block for four limbs and the exponent that takes its values
+// to integers below 2^30: v * 2^e = A0 * 2^24 + A1 * 2^16 + A2 * 2^8 + A3, each
+// multiplied by a weight * 16, so a limb dot's unit is k = 2^-(e + 4).  Blocks
+// below 2^-115 share the scale whose k is f32's smallest value: values keep
+// bits down to 2^-145.  An Inf/NaN makes k non-finite, and with it the output.
+__device__ __forceinline__ void block_scale4(float amax, float& k, int& e) {
+    const uint32_t bits = __float_as_uint(amax), eb = max((bits >> 23) & 0xffu, 11u);
+    const float s = __uint_as_float((eb - 5u) << 23);
+    k = eb == 0xffu ? amax : s * 0x1p-28f;
+    e = 156 - static_cast<int>(eb);
+}
+// The four limb words (planes A0 .. A3; value i in byte i) of four values.  The
+// bytes of R + 0x808080 are the digits of R in base 256 with the low three
+// biased by 128; flipping their bit 7 makes them int8.
+__device__ __forceinline__ void fixed4(const f32x4 v, int e, uint32_t (&w)[4]) {
+    uint32_t b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        b[i] = static_cast<uint32_t>(static_cast<int>(__builtin_rintf(__builtin_ldexpf(v[i], e)))) + 0x808080u;
+    // perm(hi, lo, sel): byte j of the result is byte sel_j of {hi:lo}
+    const uint32_t l01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u), l23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
+    const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x07030602u), h23 = __builtin_amdgcn_perm(b[3], b[2], 0x07030602u);
+    w[3] = __builtin_amdgcn_perm(l23, l01, 0x05040100u) ^ 0x80808080u;
+    w[2] = __builtin_amdgcn_perm(l23, l01, 0x07060302u) ^ 0x80808080u;
+    w[1] = __builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u;
+    w[0] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+}
 // Signed nibbles of v (two's complement) as int8 multiples of 16.
 __device__ __forceinline__ long signed16(uint32_t v) { return pair64((v << 4) & 0xf0f0f0f0u, v & 0xf0f0f0f0u); }
 
@@ -194,6 +229,7 @@ __device__ __forceinline__ long signed16(uint32_t v) { return pair64((v << 4) & 
 // block: values 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3.
 struct BQ40 {
     static constexpr bool kInt = true, kMin = false;
+    static constexpr int kLimbs = 4;
     static constexpr int kSteps = 8;
     static constexpr int kX0 = 4, kX1 = 16;  // values 4g.. and 4g + 16..
     static constexpr bool kTail = false;
@@ -233,8 +269,8 @@ struct BQ40 {
         transpose4(y);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            o.ds[2 * j] = 0.0625f * f16_bits_to_f32(dd[j] & 0xffffu);
-            o.ds[2 * j + 1] = 0.0625f * f16_bits_to_f32(dd[j] >> 16);
+            o.ds[2 * j] = f16_bits_to_f32(dd[j] & 0xffffu);
+            o.ds[2 * j + 1] = f16_bits_to_f32(dd[j] >> 16);
             o.b[2 * j] = signed16(x[j] ^ 0x88888888u);
             o.b[2 * j + 1] = signed16(y[j] ^ 0x88888888u);
         }
@@ -247,6 +283,7 @@ struct BQ40 {
 // 8g + 7, the even ones in its low nibbles.
 struct BQ4m {
     static constexpr bool kInt = true, kMin = false;
+    static constexpr int kLimbs = 4;
     static constexpr int kSteps = 8;
     static constexpr int kX0 = 8, kX1 = 4;
     static constexpr bool kTail = true;
@@ -287,8 +324,8 @@ struct BQ4m {
         transpose4(y);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            o.ds[2 * j] = 0.0625f * __uint_as_float(d0[j]);
-            o.ds[2 * j + 1] = 0.0625f * __uint_as_float(d1[j]);
+            o.ds[2 * j] = __uint_as_float(d0[j]);
+            o.ds[2 * j + 1] = __uint_as_float(d1[j]);
             o.b[2 * j] = signed16(x[j]);
             o.b[2 * j + 1] = signed16(y[j]);
         }
@@ -296,15 +333,23 @@ struct BQ4m {
 };
 
 // LDS of one staged slot for Q row groups:
-//   4-bit: limbs [4 step pairs][4Q rows][4 g][3 lambda][2 steps][8 bytes], then
-//          scales s / 65536 [4Q rows][8 steps] and (Q4_K) sums of x, the same shape;
-//   BF16:  limbs [4 steps][4Q rows][4 g][3 lambda][16 bytes].
+//   4-bit: limbs [4 step pairs][4Q rows][4 g][kLimbs][2 steps][8 bytes], then
+//          the units of the limb dots [4Q rows][8 steps] and (Q4_K) sums of x,
+//          the same shape;
+//   BF16:  limbs [4 steps][4Q rows][4 g][kLimbs][16 bytes].
 // Step (pair) records are 16 bytes longer than their limbs, which spreads the
 // lanes of a staging write, one step after another, over the banks.
-__host__ __device__ constexpr int step_bytes(int q) { return q * 768 + 16; }
+template <class F>
+__host__ __device__ constexpr int row_bytes() {  // of one step (pair)
+    return 64 * F::kLimbs;
+}
+template <class F>
+__host__ __device__ constexpr int step_bytes(int q) {
+    return q * 4 * row_bytes<F>() + 16;
+}
 template <class F>
 __host__ __device__ constexpr int limb_bytes(int q) {
-    return 4 * step_bytes(q);
+    return 4 * step_bytes<F>(q);
 }
 template <class F>
 __host__ __device__ constexpr int cst_bytes(int q) {
@@ -383,6 +428,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
     const BatchShape S{n, k, m, ks_log, groups, nslots, cslots, nchunks, per, static_cast<int>(gridDim.y), NW, sc_off};
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int kLimb = limb_bytes<F>(Q), kCst = cst_bytes<F>(Q), kThreads = NW * kWave;
+    constexpr int kRow = row_bytes<F>(), kStep = step_bytes<F>(Q), kG = 16 * F::kLimbs;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KS = 1 << S.ks_log, ks = wave & (KS - 1), tw = wave >> S.ks_log, TW = NW >> S.ks_log;
@@ -457,23 +503,29 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 } else {
                     amax = quad_max(amax);
                 }
-                float sc, inv;
-                q4k_mfma::sub_block_scale(amax, sc, inv);
-                uint32_t a0, a1, a2, b0, b1, b2;
-                q4k_mfma::limb_words(a, inv, a0, a1, a2);
-                q4k_mfma::limb_words(b, inv, b0, b1, b2);
-                float sum = 0.0f;
+                uint32_t wa[4], wb[4];
+                float unit, sum = 0.0f;
+                if constexpr (F::kLimbs == 4) {
+                    int ex;
+                    block_scale4(amax, unit, ex);
+                    fixed4(a, ex, wa);
+                    fixed4(b, ex, wb);
+                } else {
+                    float sc, inv;
+                    q4k_mfma::sub_block_scale(amax, sc, inv);
+                    unit = sc * (1.0f / 65536.0f);
+                    q4k_mfma::limb_words(a, inv, wa[0], wa[1], wa[2]);
+                    q4k_mfma::limb_words(b, inv, wb[0], wb[1], wb[2]);
+                }
                 if constexpr (F::kMin)
                     sum = quad_sum(((a[0] + a[1]) + (a[2] + a[3])) + ((b[0] + b[1]) + (b[2] + b[3])));
                 if (in) {
-                    uint8_t* const dst =
-                        lds + (u.r >> 3) * step_bytes(Q) + u.m * 192 + (u.r & 3) * 48 + ((u.r & 4) << 1);
-                    *reinterpret_cast<u32x2*>(dst) = u32x2{a0, b0};
-                    *reinterpret_cast<u32x2*>(dst + 16) = u32x2{a1, b1};
-                    *reinterpret_cast<u32x2*>(dst + 32) = u32x2{a2, b2};
+                    uint8_t* const dst = lds + (u.r >> 3) * kStep + u.m * kRow + (u.r & 3) * kG + ((u.r & 4) << 1);
+#pragma unroll
+                    for (int l = 0; l < F::kLimbs; ++l) *reinterpret_cast<u32x2*>(dst + 16 * l) = u32x2{wa[l], wb[l]};
                     if ((u.r & 3) == 0) {
                         const uint32_t o = (u.r >> 5) * kCst + u.m * 32 + (u.r & 28);
-                        *reinterpret_cast<float*>(cst + o) = sc * (1.0f / 65536.0f);
+                        *reinterpret_cast<float*>(cst + o) = unit;
                         if constexpr (F::kMin) *reinterpret_cast<float*>(sums + o) = sum;
                     }
                 }
@@ -482,7 +534,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 bf16_limbs4(a, ha, ma, la);
                 bf16_limbs4(b, hb, mb, lb);
                 if (in) {
-                    u32x4* d4 = reinterpret_cast<u32x4*>(lds + (u.r >> 2) * step_bytes(Q) + u.m * 192 + (u.r & 3) * 48);
+                    u32x4* d4 = reinterpret_cast<u32x4*>(lds + (u.r >> 2) * kStep + u.m * kRow + (u.r & 3) * kG);
                     d4[0] = u32x4{ha[0], ha[1], hb[0], hb[1]};
                     d4[1] = u32x4{ma[0], ma[1], mb[0], mb[1]};
                     d4[2] = u32x4{la[0], la[1], lb[0], lb[1]};
@@ -528,7 +580,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
 
     // This lane's A rows: (t, lambda) = ((l % 16) / 4, l % 4) of each group q.
     const int ai = lane & 15;
-    const uint32_t a_base = static_cast<uint32_t>((ai >> 2) * 192 + g * 48 + min(ai & 3, 2) * 16);
+    const uint32_t a_base = static_cast<uint32_t>((ai >> 2) * kRow + g * kG + min(ai & 3, F::kLimbs - 1) * 16);
     // Sums as an f32 A operand: row i = 4t + q of it is activation row 4q + t.
     const uint32_t s_base = static_cast<uint32_t>((min(ai & 3, Q - 1) * 4 + (ai >> 2)) * 32 + 4 * g);
 
@@ -546,7 +598,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
             for (int st = 0; st < 4; ++st)
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
-                    const bf16x8 A = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lb + st * step_bytes(Q) + q * 768));
+                    const bf16x8 A = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lb + st * kStep + q * 4 * kRow));
                     C[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, slot.v[st]), C[q], 0,
                                                                    0, 0);
                 }
@@ -569,7 +621,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 const f32x4 k0 = kp[0], k1 = kp[1];
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    const u32x4 a2 = *reinterpret_cast<const u32x4*>(lb + p * step_bytes(Q) + q * 768);
+                    const u32x4 a2 = *reinterpret_cast<const u32x4*>(lb + p * kStep + q * 4 * kRow);
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         const int j = 2 * p + e;
@@ -583,8 +635,9 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                                                   << 8) + static_cast<uint32_t>(c[2]);
                             acc[q] = __builtin_fmaf(w.ds[j], static_cast<float>(static_cast<int>(tot)) * kj, acc[q]);
                         } else {
-                            const int hi = c[0] * 256 + c[1];
-                            const float dot = __builtin_fmaf(static_cast<float>(hi), 256.0f, static_cast<float>(c[2]));
+                            // (multiples of 16 below 2^28: both halves convert exactly)
+                            const int hi = c[0] * 256 + c[1], lo = c[2] * 256 + c[3];
+                            const float dot = __builtin_fmaf(static_cast<float>(hi), 65536.0f, static_cast<float>(lo));
                             acc[q] = __builtin_fmaf(w.ds[j], dot * kj, acc[q]);
                         }
                     }

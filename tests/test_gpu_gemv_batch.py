@@ -5,11 +5,11 @@ K % 32), K staged in one chunk, in several, and split over workgroups, and
 outputs long enough for workgroups that walk several tile groups.
 
 Reference: float64 products of the dequantized weights (the oracle's
-decoders).  Bound, per row of y: the activation limbs of the 4-bit formats
-are within 2.5e-7 of a block's absmax (q4k_mfma.hpp) and f32 sums round by
-2^-24 a step, so each output is within 4e-7 * sum|w x|-like terms; taken
-normwise over the output that is below 1e-5 at every size here, the bound
-the single-row GEMVs are held to.
+decoders).  Bound, per row of y: Q4_K's activation limbs are within 2.5e-7 of
+a block's absmax (q4k_mfma.hpp), those of Q4_0 and Q4Mat within 2^-30, and f32
+sums round by 2^-24 a step, so each output is within 4e-7 * sum|w x|-like
+terms; taken normwise over the output that is below 1e-5 at every size here,
+the bound the single-row GEMVs are held to.
 """
 import numpy as np
 import pytest

@@ -11,6 +11,10 @@ Two bars:
   * normwise 1e-5 against the oracle's reference-order f32 product
     (quant_q4k.cpp:482-523) for every kernel family: row-major and tiled
     M = 1, the RMSNorm-fused launch, batched M = 2..8;
+  * batched Q4_0 and Q4Mat (M = 2..8, four limbs, error <= 2^-30 * the block's
+    absmax) against float64, as an f32 sum of each block's products and of the
+    blocks rounds, at these activations, at ordinary ones, at a block's values
+    beside one 10^6 times as large, and at values down to f32's smallest;
   * per element, bit for bit, where the reference's f32 result is exact:
     hand-built Q4_K blocks (d, dmin powers of two, 3-bit scales) and
     activations that are 3-bit integers times a per-sub-block power of two
@@ -21,7 +25,7 @@ Two bars:
 import numpy as np
 import pytest
 
-from helpers import GEMV_TOL, from_dev, normwise_err, say, to_dev
+from helpers import GEMV_TOL, from_dev, normwise_err, rel_rms, say, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -44,6 +48,14 @@ def wide_activation(rng, m, k, kind):
     if kind == "subblock_scales":  # every sub-block its own scale, 2^-20 .. 2^8
         s = np.exp2(rng.integers(-20, 9, (m, k // 32))).astype(np.float32)
         return (rng.standard_normal((m, k // 32, 32)) * s[..., None]).astype(np.float32).reshape(m, k)
+    if kind == "normal":
+        return rng.standard_normal((m, k)).astype(np.float32)
+    if kind == "one_large":  # one block holds a value 10^6 times the rest
+        x = (1e-3 * rng.standard_normal((m, k))).astype(np.float32)
+        x[:, 5] = 1000.0
+        return x
+    if kind == "smallest":  # around f32's smallest normal value, 2^-126
+        return (rng.standard_normal((m, k)) * 2.0 ** -122).astype(np.float32)
     raise ValueError(kind)
 
 
@@ -99,6 +111,55 @@ def test_batched(rt, orc, kind, m):
     want = orc.q4k_matmul_t(blocks, n, k, x)
     for r in range(m):
         assert normwise_err(got[r], want[r]) <= GEMV_TOL, (r, normwise_err(got[r], want[r]))
+
+
+def signed4_weights(rt, rng, fmt, n, k, scales):
+    """Device bytes and float64 values of a random Q4_0 or Q4Mat weight with the given block scales [n, k / 32]."""
+    if fmt == "q4mat":
+        packed = rng.integers(0, 256, n * k // 2, dtype=np.uint8)
+        q = np.stack([packed & 15, packed >> 4], -1).reshape(n, k // 32, 32).astype(np.int64)
+        q = np.where(q > 7, q - 16, q)
+        w = rt.q4mat_upload(packed, scales.astype(np.float32).reshape(-1), n, k)
+        return rt.Q4MAT, w, (q * scales.astype(np.float32).astype(np.float64)[..., None]).reshape(n, k)
+    b = rng.integers(0, 256, (n * k // 32, 18), dtype=np.uint8)
+    d = scales.astype(np.float16).reshape(-1)
+    b[:, :2] = d[:, None].view(np.uint8)
+    q = np.concatenate([b[:, 2:] & 15, b[:, 2:] >> 4], 1).astype(np.int64) - 8
+    return rt.Q4_0, to_dev(b.reshape(-1)), (q * d.astype(np.float64)[:, None]).reshape(n, k)
+
+
+# f32 sums of 32 products and then of K / 32 blocks round by 2^-24 / sqrt(3) of
+# their size a step; a random sum of `s` terms has the size sqrt(s), so the rms
+# over K / 32 steps is 2^-24 / sqrt(3) * sqrt(K / 64): 2.4e-7 at K = 3072, 4.5e-7
+# at 11008.
+@pytest.mark.parametrize("kind", KINDS + ["normal", "one_large", "smallest"])
+@pytest.mark.parametrize("fmt", ["q4_0", "q4mat"])
+def test_batched_signed4(rt, kind, fmt):
+    for n, k, m in [(300, 3072, 2), (300, 3072, 8), (1024, 3072, 5), (128, 11008, 4), (40, 512, 7)]:
+        say(f"[wide x] {fmt} {n} x {k}, M = {m} kind={kind}")
+        rng = np.random.default_rng(n + k + m + len(kind))
+        code, w, v = signed4_weights(rt, rng, fmt, n, k, 0.002 + 0.004 * rng.random((n, k // 32)))
+        if kind == "smallest":
+            code, w, v = signed4_weights(rt, rng, fmt, n, k, 200.0 + 400.0 * rng.random((n, k // 32)))
+        x = wide_activation(rng, m, k, kind)
+        got, want = from_dev(rt.gemv(code, w, to_dev(x), n, k)), x.astype(np.float64) @ v.T
+        bound = 2.0 ** -24 / np.sqrt(3.0) * np.sqrt(k / 64.0)
+        for r in range(m):
+            # (rel_rms floors its denominator at 1e-30: scaled clear of that)
+            err = rel_rms(got[r] * 2.0 ** 100, want[r] * 2.0 ** 100)
+            assert err <= max(bound, 2e-7), (n, k, m, r, err)
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q4mat"])
+def test_batched_signed4_exact_inputs(rt, fmt):
+    """Integer activations times powers of two, power-of-two scales: every
+    product and partial sum has few bits, so any correct kernel gives them."""
+    for n, k, m in [(100, 2048, 3), (64, 768, 8)]:
+        say(f"[exact x] {fmt} {n} x {k}, M = {m}")
+        rng = np.random.default_rng(n + k)
+        code, w, v = signed4_weights(rt, rng, fmt, n, k, np.exp2(rng.integers(-8, -4, (n, k // 32)).astype(np.float64)))
+        x = exact_activation(rng, m, k, spread=6)
+        assert np.array_equal(from_dev(rt.gemv(code, w, to_dev(x), n, k)), (x.astype(np.float64) @ v.T).astype(np.float32))
 
 
 # ---- exactly representable case ---------------------------------------------
