@@ -584,11 +584,13 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
     // Sums as an f32 A operand: row i = 4t + q of it is activation row 4q + t.
     const uint32_t s_base = static_cast<uint32_t>((min(ai & 3, Q - 1) * 4 + (ai >> 2)) * 32 + 4 * g);
 
-    f32x4 C[Q];
+    // C: the even and the odd BF16 steps' dots of a chunk.  acc: the sum over
+    // chunks, or over 4-bit slots.  Short chains round less than one long one.
+    f32x4 C[2][Q];
     float acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        C[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        C[0][q] = C[1][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         acc[q] = 0.0f;
     }
     auto consume = [&](const typename F::Slot& slot, int sl) {
@@ -599,8 +601,8 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
                     const bf16x8 A = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lb + st * kStep + q * 4 * kRow));
-                    C[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, slot.v[st]), C[q], 0,
-                                                                   0, 0);
+                    C[st & 1][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, slot.v[st]),
+                                                                           C[st & 1][q], 0, 0, 0);
                 }
         } else {
             Dec4 w;
@@ -666,6 +668,14 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                     issue(next, ngroup, nchunk, ii - S.per, ring[j]);
             }
         }
+        if constexpr (!F::kInt) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const f32x4 c = C[0][q] + C[1][q];
+                acc[q] += (c[0] + c[1]) + c[2];
+                C[0][q] = C[1][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
         if (last_chunk) {
             // Row n of the tile, activation row 4q + g.
             const int row = 16 * (group * TW + tw) + (lane & 15);
@@ -673,8 +683,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
             if constexpr (FORM == kBias) add = bias[min(row, S.n - 1)];
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
-                v[q] = F::kInt ? acc[q] : (C[q][0] + C[q][1]) + C[q][2];
-                C[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                v[q] = acc[q];
                 acc[q] = 0.0f;
             }
             if (S.ks_log) {

@@ -142,3 +142,25 @@ def test_batched_gemv_nonfinite_rows(rt, orc, fmt):
                 if np.isnan(value):
                     assert np.isnan(y[bad]).all()
                 assert np.array_equal(np.delete(y, bad, 0), np.delete(clean, bad, 0))
+
+
+# rms error of ordinary rows against float64, relative to the result:
+#  * f32 steps round by 2^-24 / sqrt(3) of their size, a random sum of s steps
+#    grows as sqrt(s): over n steps 2^-24 / sqrt(3) * sqrt(n / 2).
+#  * BF16: chains of half a chunk's 32-value steps, at most 100 steps a chunk.
+@pytest.mark.parametrize("fmt,n,k,m,steps,limbs", [("bf16", 12288, 12288, 8, 100, 0.0), ("bf16", 1024, 3072, 4, 96, 0.0)])
+def test_batched_gemv_rounding(rt, fmt, n, k, m, steps, limbs):
+    import torch
+    say(f"[gemv batch rounding] {fmt} {n} x {k}, M = {m}")
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    w = torch.randn((n, k), device="cuda", generator=g) * 0.02
+    if fmt == "bf16":
+        code, data, v = rt.BF16, w.bfloat16().view(torch.int16), w.bfloat16()
+    else:
+        code, data = rt.Q4K, rt.quantize_q4k(w)
+        v = rt.dequant_q4k(data, n, k).reshape(n, k)
+    x = torch.randn((m, k), device="cuda", generator=g)
+    y = rt.gemv(code, data, x, n, k).double()
+    want = torch.cat([x.double() @ v[i:i + 2048].double().T.contiguous() for i in range(0, n, 2048)], 1)
+    bound = (limbs ** 2 + (2.0 ** -24 / 3 ** 0.5) ** 2 * steps / 2) ** 0.5
+    assert float((y - want).norm() / want.norm()) <= bound
