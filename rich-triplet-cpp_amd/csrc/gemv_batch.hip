@@ -24,9 +24,9 @@
 //    - Q4_K: the three limbs of the M = 1 kernel (q4k_mfma.hpp), within 2.5e-7
 //      of the block's absmax.  Nibbles 0..15, so R = C0 * 65536 + C1 * 256 +
 //      C2 stays below 32 * 15 * 2^22 < 2^31 and is converted once; the
-//      minimum's term, -(dmin * mv_j) * sum(x), is a contraction over the
-//      super-block's eight sub-blocks and runs on v_mfma_f32_16x16x4_f32
-//      (quant_q4k.cpp:482-523).
+//      minimum's term, -(dmin * mv_j) * sum(x) with x as the limbs hold it, is
+//      a contraction over the super-block's eight sub-blocks and runs on
+//      v_mfma_f32_16x16x4_f32 (quant_q4k.cpp:482-523).
 //    - Q4_0, Q4Mat: four limbs (fixed4()), within 2^-30 of the block's absmax:
 //      an f32 sum of the block's products rounds by more, also where a value
 //      stands beside one a thousand times as large.  Signed values (nibble - 8,
@@ -362,17 +362,11 @@ __host__ __device__ constexpr int slot_lds(int q) {
 constexpr int red_bytes(int waves, int q) { return waves * q * kWave * 4; }
 
 // Sum and max over the aligned quad of lanes (every lane gets the same bits).
-__device__ __forceinline__ float quad_sum(float v) {
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, false));
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) {
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xb1, 0xf, 0xf, false));
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4e, 0xf, 0xf, false));
     return v;
 }
-__device__ __forceinline__ float quad_max(float v) {
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, false)));
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, false)));
-    return v;
-}
-
 __device__ __forceinline__ uint32_t quad_max(uint32_t v) {
     v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xb1, 0xf, 0xf, false)));
     v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4e, 0xf, 0xf, false)));
@@ -493,16 +487,11 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                 // Block (step, m) is the quad of units g = 0..3.
                 float amax = fmaxf(fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))),
                                    fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3]))));
-                if constexpr (!F::kMin) {
-                    // fmaxf passes NaNs over; they are the largest of the bit
-                    // patterns (Q4_K's sum carries them)
-                    const bool nan = __builtin_isunordered(a[0], a[1]) | __builtin_isunordered(a[2], a[3]) |
-                                     __builtin_isunordered(b[0], b[1]) | __builtin_isunordered(b[2], b[3]);
-                    amax = nan ? __uint_as_float(0x7fc00000u) : amax;
-                    amax = __uint_as_float(quad_max(__float_as_uint(amax)));
-                } else {
-                    amax = quad_max(amax);
-                }
+                // fmaxf passes NaNs over; they are the largest of the bit patterns
+                const bool nan = __builtin_isunordered(a[0], a[1]) | __builtin_isunordered(a[2], a[3]) |
+                                 __builtin_isunordered(b[0], b[1]) | __builtin_isunordered(b[2], b[3]);
+                amax = nan ? __uint_as_float(0x7fc00000u) : amax;
+                amax = __uint_as_float(quad_max(__float_as_uint(amax)));
                 uint32_t wa[4], wb[4];
                 float unit, sum = 0.0f;
                 if constexpr (F::kLimbs == 4) {
@@ -514,11 +503,13 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                     float sc, inv;
                     q4k_mfma::sub_block_scale(amax, sc, inv);
                     unit = sc * (1.0f / 65536.0f);
-                    q4k_mfma::limb_words(a, inv, wa[0], wa[1], wa[2]);
-                    q4k_mfma::limb_words(b, inv, wb[0], wb[1], wb[2]);
+                    uint32_t bits = 0;
+                    q4k_mfma::limb_words(a, inv, wa[0], wa[1], wa[2], bits);
+                    q4k_mfma::limb_words(b, inv, wb[0], wb[1], wb[2], bits);
+                    // the sum of the 32 R, |R| <= 2^22, exactly: what the limbs
+                    // leave out of x then meets w = P - min, half as large as P
+                    sum = static_cast<float>(static_cast<int>(quad_sum(bits) - (0x4b400000u << 5))) * unit;
                 }
-                if constexpr (F::kMin)
-                    sum = quad_sum(((a[0] + a[1]) + (a[2] + a[3])) + ((b[0] + b[1]) + (b[2] + b[3])));
                 if (in) {
                     uint8_t* const dst = lds + (u.r >> 3) * kStep + u.m * kRow + (u.r & 3) * kG + ((u.r & 4) << 1);
 #pragma unroll
@@ -607,9 +598,9 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
         } else {
             Dec4 w;
             F::decode(slot, lane, w);
-            // The minimum's term of this super-block, added to the row sums
-            // below: kept apart to the end, the two halves of each sum would
-            // grow several times larger than the sum and round accordingly.
+            // The minimum's term of this super-block, where its sum starts:
+            // kept apart to the end, the two halves of each sum would grow
+            // several times larger than the sum and round accordingly.
             f32x4 mins = {0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (F::kMin) {
                 const uint8_t* const sb = sums + sl * kCst + s_base;
@@ -621,6 +612,7 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
             for (int q = 0; q < Q; ++q) {
                 const f32x4* kp = reinterpret_cast<const f32x4*>(cst + sl * kCst + (q * 4 + g) * 32);
                 const f32x4 k0 = kp[0], k1 = kp[1];
+                float sum = F::kMin ? mins[q] : 0.0f;
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
                     const u32x4 a2 = *reinterpret_cast<const u32x4*>(lb + p * kStep + q * 4 * kRow);
@@ -635,16 +627,16 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                             // |R * nibble| sums below 2^31 (see above); the shifts wrap, the total does not
                             const uint32_t tot = (((static_cast<uint32_t>(c[0]) << 8) + static_cast<uint32_t>(c[1]))
                                                   << 8) + static_cast<uint32_t>(c[2]);
-                            acc[q] = __builtin_fmaf(w.ds[j], static_cast<float>(static_cast<int>(tot)) * kj, acc[q]);
+                            sum = __builtin_fmaf(w.ds[j], static_cast<float>(static_cast<int>(tot)) * kj, sum);
                         } else {
                             // (multiples of 16 below 2^28: both halves convert exactly)
                             const int hi = c[0] * 256 + c[1], lo = c[2] * 256 + c[3];
                             const float dot = __builtin_fmaf(static_cast<float>(hi), 65536.0f, static_cast<float>(lo));
-                            acc[q] = __builtin_fmaf(w.ds[j], dot * kj, acc[q]);
+                            sum = __builtin_fmaf(w.ds[j], dot * kj, sum);
                         }
                     }
                 }
-                if constexpr (F::kMin) acc[q] += mins[q];
+                acc[q] += sum;
             }
         }
     };

@@ -88,11 +88,16 @@ __device__ __forceinline__ void sub_block_scale(float amax, float& s, float& inv
 //     A2 = byte 0 - 128, A1 = byte 1 - 128 (as int8: the byte with bit 7 flipped),
 //     A0 = byte 2 - 64 (bytes 0..128: + 64 carries into no neighbour, then the flip),
 // so that R = 65536 A0 + 256 A1 + A2 with |A0| <= 64.  v_perm gathers each plane.
-__device__ __forceinline__ void limb_words(const f32x4 v, float inv, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+// `bits` gains the four 0x4B400000 + R.
+__device__ __forceinline__ void limb_words(const f32x4 v, float inv, uint32_t& w0, uint32_t& w1, uint32_t& w2,
+                                           uint32_t& bits) {
     uint32_t b[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        b[e] = __float_as_uint(__builtin_fmaf(v[e] * inv, 65536.0f, 12582912.0f)) + 0x8080u;
+    for (int e = 0; e < 4; ++e) {
+        b[e] = __float_as_uint(__builtin_fmaf(v[e] * inv, 65536.0f, 12582912.0f));
+        bits += b[e];
+        b[e] += 0x8080u;
+    }
     // perm(hi, lo, sel): byte j of the result is byte sel_j of {hi:lo}
     const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);  // bytes 0 of both, then bytes 1
     const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
@@ -101,6 +106,10 @@ __device__ __forceinline__ void limb_words(const f32x4 v, float inv, uint32_t& w
     w2 = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
     w1 = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
     w0 = (__builtin_amdgcn_perm(h23, h01, 0x05040100u) + 0x40404040u) ^ 0x80808080u;
+}
+__device__ __forceinline__ void limb_words(const f32x4 v, float inv, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+    uint32_t unused = 0;
+    limb_words(v, inv, w0, w1, w2, unused);
 }
 
 // Limbs of 4 activations (one f32x4) of a sub-block whose 8 holders are the

@@ -148,7 +148,11 @@ def test_batched_gemv_nonfinite_rows(rt, orc, fmt):
 #  * f32 steps round by 2^-24 / sqrt(3) of their size, a random sum of s steps
 #    grows as sqrt(s): over n steps 2^-24 / sqrt(3) * sqrt(n / 2).
 #  * BF16: chains of half a chunk's 32-value steps, at most 100 steps a chunk.
-@pytest.mark.parametrize("fmt,n,k,m,steps,limbs", [("bf16", 12288, 12288, 8, 100, 0.0), ("bf16", 1024, 3072, 4, 96, 0.0)])
+#  * Q4_K: the blocks of 32, and the limbs' steps of 2^-20 where a block's
+#    absmax is 2 to 4 (rms 2^-20 / sqrt(12)).
+@pytest.mark.parametrize("fmt,n,k,m,steps,limbs", [("bf16", 12288, 12288, 8, 100, 0.0), ("bf16", 1024, 3072, 4, 96, 0.0),
+                                                   ("q4k", 1024, 3072, 5, 96, 2.0 ** -20 / 12 ** 0.5),
+                                                   ("q4k", 4096, 4096, 8, 128, 2.0 ** -20 / 12 ** 0.5)])
 def test_batched_gemv_rounding(rt, fmt, n, k, m, steps, limbs):
     import torch
     say(f"[gemv batch rounding] {fmt} {n} x {k}, M = {m}")
