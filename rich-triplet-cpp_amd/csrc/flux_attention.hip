@@ -35,9 +35,12 @@
 //    leaves lane (h, n) holding O[query n][dims 32c + 8i + 4h + r].
 // From a tile of K or V that holds a value of 2^64 or more, an infinity or a
 // NaN, or throughout a block with a query of 2^55 or more, the block takes f32
-// MFMA steps on the values in memory: products that overflow and infinities
+// MFMA steps on the staged f32 tiles: products that overflow and infinities
 // then behave as in f32 arithmetic (a limb's product could overflow to the
 // other sign).  A loop of its own: the limb loop has no registers to spare.
+// It costs what f32 steps do: t = 4352, 24 x 128 with an infinity in one head
+// 2790 us, in the middle tile of all 2090 (with f32 MFMA throughout 2070; with
+// the operands read from memory step by step 10650 and 7020).
 //
 // The head is padded to DP in {32, 64, 128} dims with zeros (they add
 // nothing to a score and are never stored).  Keys past T are masked to -inf
@@ -479,26 +482,43 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
         }
         __builtin_amdgcn_s_setprio(0);
         if (kTwo && !second) lds_barrier();
-        // The rest of a block that met a value without limbs, in f32 from memory.
-        for (int tile = t0 + nt; tile < t1; ++tile) {
-            const int base = tile * kBK;
-            s = f32x16{};
-#pragma unroll 1
-            for (int a = 0; a < DP / 2; ++a) {
-                const int dim = 2 * a + h;
-                const float ka = base + n < T && dim < D ? kb[(base + n) * stride + dim] : 0.0f;
-                const float qa = qrow < T && dim < D ? qb[qrow * stride + dim] : 0.0f;
-                s = __builtin_amdgcn_mfma_f32_32x32x2f32(ka, qa, s, 0, 0, 0);
-            }
-            softmax(s, base);
+        // The rest of a block that met a value without limbs, in f32.  The raw
+        // copies of a tile, every wave's share, hold it whole: K units of 4 dims
+        // at 16 bytes a lane, V units of one dim at 4.  Half h takes dims 8a + 4h
+        // .. + 3 of a step.
+        if (nt < t1 - t0) {
+            const uint8_t* const shares = lds + 15 * kPlane;
+            constexpr int kShare = raw_wave_bytes<DP, NW>(), kRows = NT / DP;
+            const float* const qp = qb + min(qrow, T - 1) * stride;  // (rows past T are not stored)
+            copies_wait();
+            for (int tile = t0 + nt; tile < t1; ++tile) {
+                load_tile(tile - t0);
+                copies_wait();
+                __syncthreads();
+                s = f32x16{};
+#pragma unroll 4
+                for (int a = 0; a < DP / 8; ++a) {
+                    const int id = n * (DP / 8) + a, tt = id % NT, dim = 8 * a + 4 * h;
+                    const f32x4 ka = *reinterpret_cast<const f32x4*>(shares + (tt >> 6) * kShare +
+                                                                     (2 * (id / NT) + h) * 1024 + (tt & 63) * 16);
+                    const f32x4 qa = *reinterpret_cast<const f32x4*>(qp + min(dim, D - 4));
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int key = base + 8 * (e >> 2) + 4 * h + (e & 3);
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    const float va = key < T && 32 * c + n < D ? vb[key * stride + 32 * c + n] : 0.0f;
-                    o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, s[e], o[c], 0, 0, 0);
+                    for (int e = 0; e < 4; ++e)
+                        s = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[e], dim < D ? qa[e] : 0.0f, s, 0, 0, 0);
                 }
+                softmax(s, tile * kBK);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {  // key 8 (e / 4) + 4h + e % 4
+                    const int quad = 2 * (e >> 2) + h;
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) {
+                        const int tt = (quad % kRows) * DP + 32 * c + n;
+                        const float va = *reinterpret_cast<const float*>(
+                            shares + (tt >> 6) * kShare + KU * 2048 + (4 * (quad / kRows) + (e & 3)) * 256 + (tt & 63) * 4);
+                        o[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, s[e], o[c], 0, 0, 0);
+                    }
+                }
+                __syncthreads();  // every wave has read this tile's shares
             }
         }
         l_run += other_half(l_run, h);

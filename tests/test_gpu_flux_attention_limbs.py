@@ -51,7 +51,58 @@ def test_flux_attention_block_edges(rt, t, h, d):
         assert normwise_err(got[:, sl], want[:, sl]) <= FLUX_ATTN_TOL, hh
 
 
-# (4 heads of 128: 4-wave blocks; 70: 8 waves with blocks cut between two)
+def form(t, h):
+    """(waves of a workgroup, blocks cut between two of them) on this device."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    small, large = h * -(-t // 128), h * -(-t // 256)
+    if t <= 128 or small <= cus or (small <= 2 * cus and large > cus):
+        return 4, False
+    return 8, large > cus
+
+
+# Values in the first, second, a middle and the last tile of 32 keys, in 4-wave
+# blocks and 8-wave ones, whole and cut between two workgroups.
+FORMS = [(300, 4, 128, 4, False), (300, 4, 40, 4, False), (512, 100, 128, 8, False), (700, 100, 128, 8, True),
+         (700, 100, 64, 8, True), (1200, 60, 32, 8, True)]
+
+
+@pytest.mark.parametrize("t,h,d,waves,cut", FORMS)
+@pytest.mark.parametrize("where", ["first", "second", "middle", "last"])
+def test_flux_attention_wide_values_every_form(rt, t, h, d, waves, cut, where):
+    if form(t, h) != (waves, cut):
+        pytest.skip(f"{h} heads of {t} queries run as {form(t, h)} on this device")
+    row = {"first": 0, "second": 40, "middle": t // 2, "last": t - 1}[where]
+    test_flux_attention_values_without_limbs(rt, t, h, d, row)
+
+
+def test_flux_attention_wide_values_cost(rt):
+    """One infinity costs a call at most what f32 matrix steps do: 16 / 6 of the
+    limbs' matrix time, less than 3 times the call, where loads from memory in
+    place of the staged tiles took 5 to 9 times."""
+    import torch
+    t, h, d = 1280, 24, 128
+    say(f"[flux wide cost] t={t} heads={h}")
+    q, k, v = (to_dev(a) for a in rand(t, h, d))
+    out = torch.empty_like(q)
+
+    def time_of():
+        best = 1e9
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                rt.flux_attention(q, k, v, h, d, out=out)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    clean = time_of()
+    v[0, ::d] = float("inf")  # every head's first value: every block is in f32 throughout
+    assert time_of() <= 3.5 * clean
+
+
 @pytest.mark.parametrize("t,h,d,row", [(300, 4, 128, 0), (300, 4, 128, 290), (300, 4, 40, 64), (800, 70, 128, 31),
                                        (800, 70, 128, 799), (700, 100, 64, 350)])
 def test_flux_attention_values_without_limbs(rt, t, h, d, row):
