@@ -47,13 +47,16 @@
 // about 100 per slot at M <= 4 and 140 at M <= 8.  Keeping K inside the
 // workgroup saves the merge through memory that every K longer than one slice
 // used to pay (1.7 us).  Measured, before -> now, us per launch in a graph:
-//   Q4_K  3072 x 3072  M = 4: 7.8 -> 5.6   M = 8: 9.3 -> 7.8
-//   Q4_K  8192 x 3072  M = 4: 8.4 -> 7.7   M = 8: 10.0 -> 9.9
-//   Q4_K  3072 x 8192  M = 4: 11.8 -> 10.3 M = 8: 14.5 -> 13.6
-//   BF16  3072 x 3072  M = 4: 10.8 -> 8.1  M = 8: 11.7 -> 10.2
-//   Q4_0  4096 x 4096  M = 4: 18.6 -> 6.3  M = 8: 29.3 -> 9.2 (VALU before)
-//   Q4_0  4096 x 11008 M = 4: 246 -> 11.4  M = 8: 616 -> 15.3
-//   Q4Mat 4096 x 4096  M = 4: 15.9 -> 6.4  M = 8: 52.1 -> 9.7 (VALU before)
+//   Q4_K  3072 x 3072   M = 4: 7.9 -> 6.0    M = 8: 9.7 -> 8.4
+//   Q4_K  8192 x 3072   M = 4: 8.5 -> 7.3    M = 8: 10.4 -> 10.1
+//   Q4_K  3072 x 8192   M = 4: 11.5 -> 10.5  M = 8: 14.5 -> 13.1
+//   Q4_K  12288 x 12288 M = 4: 27.9 -> 28.8  M = 8: 32.1 -> 32.4
+//   Q4_K  256 x 65536   M = 4: 23.0 -> 13.9  M = 8: 28.7 -> 20.2
+//   BF16  3072 x 3072   M = 4: 10.0 -> 7.2   M = 8: 11.1 -> 8.7
+//   BF16  12288 x 12288 M = 4: 52.2 -> 53.0  M = 8: 58.0 -> 58.3
+//   Q4_0  4096 x 4096   M = 4: 18.7 -> 6.2   M = 8: 29.1 -> 9.2 (VALU before)
+//   Q4_0  4096 x 11008  M = 4: 246 -> 10.5   M = 8: 616 -> 14.8
+//   Q4Mat 4096 x 4096   M = 4: 15.6 -> 6.4   M = 8: 52.0 -> 9.6 (VALU before)
 // (With three limbs Q4_0 and Q4Mat took 5% less at M = 8 and the same at M = 4,
 // and were up to 4 times as far from float64 as the VALU kernels.)
 #include "q4k_mfma.hpp"
@@ -646,7 +649,8 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
         const bool last_chunk = S.slices > 1 || chunk + 1 == S.nchunks;
         const int ngroup = last_chunk ? group + static_cast<int>(gridDim.x) : group, nchunk = last_chunk ? 0 : chunk + 1;
         const typename F::Tile next = tile_of(min(ngroup, S.groups - 1));
-        const int cs = chunk_slots(chunk);
+        // (no products in a wave whose tile lies past the last row)
+        const int cs = 16 * (group * TW + tw) < S.n ? chunk_slots(chunk) : 0;
         for (int i = 0; i < S.per; i += kDepth) {
 #pragma unroll
             for (int j = 0; j < kDepth; ++j) {
@@ -764,22 +768,48 @@ bool two_fit(int64_t cs, int m, int q) {
            cs * F::kSteps * 4 * m <= 4 * kWaves * kWave;
 }
 
-// The launch shape: the least estimated time over the splits of K between
-// the waves of a workgroup (KS) and, with `sliced`, between workgroups.  In
-// units of 0.1 us above the launch, fitted to Q4_K times at N x K = 1024 ..
-// 10240 x 3072, 3072 x 8192 and 2560 x 10240 and BF16 ones at 3072 and 8192
-// x 3072 and 3072 x 8192, M = 2, 4 and 8:
-//   staging   1.3 per 1024 activations (every workgroup, each chunk it takes;
-//             once when one chunk holds all of K), 12 (BF16 20) more per
-//             further chunk;
-//   slots     7 (M <= 4) or 9 per 4-bit slot of each wave, 6 per BF16 slot;
-//   3 for the waves' reduction, 14 + 5 slices for a merge through memory
-//             (6 at M > 4; BF16 15 + 5);
-//   two workgroups of one CU overlap: each then takes 1.2 times as long (1.5
-//             at M > 4, BF16 1.7).
-// The best of the shapes swept is within 5% of the one taken at those sizes
-// (Q4_K 3072 x 8192, M = 4: 10.3 us in 4 slices, 11.5 in one; M = 8: 13.5,
-// 16.9).
+// The launch shape: the least estimated time over the splits of K between the
+// waves of a workgroup (KS) and, with `sliced`, between workgroups.  Costs in
+// units of 0.1 us above the launch: one workgroup alone on its CU, and (".2")
+// two that share it, as the grid of a shape makes them (`turns`: how many
+// workgroups, or pairs of them, a CU runs one after another).
+//   stage  per 1024 activations staged: every slice, and in an unsliced launch
+//          every chunk of every turn (once when one chunk holds all of K)
+//   slot   per weight slot of each wave
+//   again  per staging that waits for the products before it
+//   red    per turn, the waves' sums where KS > 1
+//   merge, slice, sums   a merge through memory, per slice, and per 10^6 partial sums
+//   turn, turn1          per turn after the first, sliced and not
+//   narrow per slot and halving of KS: fewer waves of a tile read longer runs
+//          of a row each
+// Fitted to times of every split at 46 sizes from 16 x 256 to 262144 x 1024 and
+// 16 x 131072 at M = 2, 4, 5 and 8, in each format: the shape taken is within
+// 1.1% of the best of a size on average, and within 13% but for BF16 128256 x
+// 2048 (26%: 114 us with KS = 1, 90 with 8).
+struct Cost {
+    double stage, stage2, slot, slot2, again, red, merge, slice, sums, turn, turn1, narrow;
+};
+template <class F, int Q>
+constexpr Cost cost_of() {
+    if constexpr (!F::kInt)
+        return Q == 1 ? Cost{1.7, 2.0, 10.0, 19.0, 1.4, 0.34, 18.0, 3.7, 38.0, 11.0, 12.0, 0.05}
+                      : Cost{1.4, 1.8, 11.0, 21.0, 2.2, 5.0, 10.0, 4.9, 30.0, 15.0, 4.3, 0.099};
+    else if constexpr (F::kMin)
+        return Q == 1 ? Cost{1.4, 2.1, 9.6, 18.0, 16.0, 3.0, 9.4, 4.2, 28.0, 12.0, 0.18, 0.063}
+                      : Cost{1.7, 2.3, 9.8, 18.0, 0.23, 2.6, 11.0, 5.7, 15.0, 10.0, 6.1, 0.05};
+    else
+        return Q == 1 ? Cost{1.5, 2.1, 7.6, 14.0, 11.0, 2.0, 8.2, 4.1, 29.0, 18.0, 5.0, 0.13}
+                      : Cost{1.2, 2.3, 9.8, 15.0, 2.5, 1.6, 9.2, 5.5, 14.0, 12.0, 6.6, 0.051};
+}
+
+// Workgroups of `cs`-slot chunks that share a CU in an unsliced launch: two
+// where they fit; BF16 streams as fast from one (65536 x 2560, M = 4: 62.6 us
+// against 66.1).
+template <class F>
+int64_t unsliced_per_cu(int64_t cs, int m, int q) {
+    return F::kInt && two_fit<F>(cs, m, q) ? 2 : 1;
+}
+
 template <class F, int Q>
 bool plan(int64_t n, int64_t k, int m, bool sliced, BatchShape* out) {
     const int64_t cus = device_info().cus;
@@ -802,36 +832,39 @@ bool plan(int64_t n, int64_t k, int m, bool sliced, BatchShape* out) {
                           static_cast<int>(nslots), static_cast<int>(nslots), 1, static_cast<int>(p), 1, 16, 0};
         return true;
     }
+    constexpr Cost C = cost_of<F, Q>();
     double cost = -1.0;
     const int fs = tune_param("BATCH_SLICES", 0), fk = tune_param("BATCH_KS", -1);
-    for (int64_t slices = 1; slices <= (sliced ? 8 : 1); ++slices) {
-        if (slices > 1 && (slices < cmin || slices > nslots)) continue;
+    static const int kSlices[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128};
+    for (const int64_t slices : kSlices) {
+        if (slices > 1 && (!sliced || slices < cmin || slices > nslots)) continue;
         if (fs && slices != fs) continue;
         const int64_t nchunks = slices > 1 ? slices : cmin;
         const int64_t cs = (nslots + nchunks - 1) / nchunks;
         if (cs * (nchunks - 1) >= nslots) continue;  // an empty last chunk
-        const int64_t occ = two_fit<F>(cs, m, Q) ? 2 : 1;
+        const double stage = static_cast<double>(cs * F::kSteps * 32 * m) / 1024.0;
+        const int64_t per_cu = slices > 1 ? (two_fit<F>(cs, m, Q) ? 2 : 1) : unsliced_per_cu<F>(cs, m, Q);
         for (int lg = 0; lg <= 3; ++lg) {
             if (fk >= 0 && lg != fk) continue;
             const int64_t groups = (tiles + (kWaves >> lg) - 1) / (kWaves >> lg);
-            if (slices > 1 && (groups > static_cast<int64_t>(kArrivalCounters) || groups * slices > occ * cus)) continue;
-            const double share = slices > 1 && groups * slices > cus ? (F::kInt ? (Q == 1 ? 1.2 : 1.5) : 1.7) : 1.0;
-            const double rounds = slices > 1 ? 1.0 : static_cast<double>((groups + cus - 1) / cus);
-            const double stage = 1.3 * static_cast<double>(cs * F::kSteps * 32 * m) / 1024.0;
-            const double slot = F::kInt ? (Q == 1 ? 7.0 : 9.0) : 6.0, again = F::kInt ? 12.0 : 20.0;
-            const double merge = (F::kInt ? 14.0 : 15.0) + (F::kInt && Q == 2 ? 6.0 : 5.0) * static_cast<double>(slices);
-            const double per = static_cast<double>((cs + (1 << lg) - 1) >> lg);
-            const double restage = nchunks > 1 ? rounds * static_cast<double>(nchunks) : 1.0;
-            double t = slices > 1 ? share * (stage + per * slot) + merge
-                                  : restage * (stage + again) - again + rounds * static_cast<double>(nchunks) * per * slot;
-            if (lg) t += 3.0 * rounds;
+            if (slices > 1 && groups > static_cast<int64_t>(kArrivalCounters)) continue;
+            const int64_t per = (cs + (1 << lg) - 1) >> lg, all = groups * slices;
+            const bool shared = per_cu == 2 && all > cus;
+            const double turns = static_cast<double>((all + cus - 1) / cus) * (shared ? 0.5 : 1.0);
+            const double n_stage = slices == 1 && nchunks == 1 ? 1.0 : turns * static_cast<double>(slices > 1 ? 1 : nchunks);
+            const double n_slot = turns * static_cast<double>(per * (slices > 1 ? 1 : nchunks));
+            double t = n_stage * stage * (shared ? C.stage2 : C.stage) + n_slot * (shared ? C.slot2 : C.slot);
+            t += C.narrow * static_cast<double>(3 - lg) * n_slot + (lg ? C.red * turns : 0.0);
+            if (slices > 1)
+                t += C.merge + C.slice * static_cast<double>(slices) + C.sums * static_cast<double>(slices * m * n) * 1e-6 +
+                     C.turn * (turns - 1.0);
+            else
+                t += C.turn1 * (turns - 1.0) + (nchunks > 1 ? C.again * (n_stage - 1.0) : 0.0);
             if (cost >= 0.0 && t >= cost) continue;
             cost = t;
-            int64_t p = (cs + (1 << lg) - 1) >> lg;
-            p = (p + kDepth - 1) / kDepth * kDepth;
             *out = BatchShape{static_cast<int>(n),      static_cast<int>(k),  m, lg, static_cast<int>(groups),
                               static_cast<int>(nslots), static_cast<int>(cs), static_cast<int>(nchunks),
-                              static_cast<int>(p),      static_cast<int>(slices), kWaves, 0};
+                              static_cast<int>((per + kDepth - 1) / kDepth * kDepth), static_cast<int>(slices), kWaves, 0};
         }
     }
     return cost >= 0.0;
@@ -856,10 +889,8 @@ hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, in
     }
     S.sc_off = sc_off;
     const size_t lds = static_cast<size_t>(S.cslots) * slot_lds<F>(Q) + red_bytes(S.waves, Q);
-    // Two workgroups per CU where they fit; BF16 streams as fast from one
-    // (65536 x 2560, M = 4: 62.6 us against 66.1).
-    const int64_t slots =
-        (F::kInt && S.waves == kWaves && two_fit<F>(S.cslots, m, Q) ? 2 : 1) * static_cast<int64_t>(device_info().cus);
+    const int64_t slots = (S.waves == kWaves ? unsliced_per_cu<F>(S.cslots, m, Q) : 1) *
+                          static_cast<int64_t>(device_info().cus);
     const dim3 grid(static_cast<unsigned>(S.slices > 1 || S.groups < slots ? S.groups : slots),
                     static_cast<unsigned>(S.slices));
     const int threads = S.waves * kWave;
@@ -873,6 +904,7 @@ hipError_t run(const void* w, const float* x, float* y, int64_t n, int64_t k, in
     if constexpr (F::kInt && Q == 2) {
         if (S.waves == 16) return go(k_gemv_batch<F, Q, 4, 16, FORM>);
     }
+    if (xp <= 1) return go(k_gemv_batch<F, Q, 1, kWaves, FORM>);
     if (xp <= 2) return go(k_gemv_batch<F, Q, 2, kWaves, FORM>);
     if (xp <= 4) return go(k_gemv_batch<F, Q, 4, kWaves, FORM>);
     return go(k_gemv_batch<F, Q, 8, kWaves, FORM>);

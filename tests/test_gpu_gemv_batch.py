@@ -168,3 +168,49 @@ def test_batched_gemv_rounding(rt, fmt, n, k, m, steps, limbs):
     want = torch.cat([x.double() @ v[i:i + 2048].double().T.contiguous() for i in range(0, n, 2048)], 1)
     bound = (limbs ** 2 + (2.0 ** -24 / 3 ** 0.5) ** 2 * steps / 2) ** 0.5
     assert float((y - want).norm() / want.norm()) <= bound
+
+
+@pytest.mark.parametrize("fmt,n,k,m", [("q4k", 16, 131072, 8), ("q4k", 256, 65536, 5), ("bf16", 40, 131072, 3),
+                                       ("bf16", 256, 65536, 8), ("q4_0", 12288, 12288, 8), ("q4mat", 250, 35840, 7)])
+def test_batched_gemv_long_k(rt, fmt, n, k, m):
+    """K of many chunks: summed over workgroups, in up to 128 slices, and over
+    more workgroups than the device holds at once (12288 x 12288); at most 4 times
+    the time of a square of as many weights (kept inside few workgroups, up to 17)."""
+    import torch
+    say(f"[gemv batch long k] {fmt} {n} x {k}, M = {m}")
+    gen = torch.Generator(device="cuda").manual_seed(k)
+
+    def make(n, k):
+        if fmt == "q4mat":
+            off, w = rt.library().lib.rt_hip_q4mat_scales_offset(n, k), torch.empty(rt.q4mat_bytes(n, k), dtype=torch.uint8, device="cuda")
+            w[:n * k // 2] = torch.randint(0, 256, (n * k // 2,), dtype=torch.uint8, device="cuda", generator=gen)
+            w[off:off + n * k // 8] = (0.002 + 0.004 * torch.rand(n * k // 32, device="cuda", generator=gen)).view(torch.uint8)
+            return rt.Q4MAT, w
+        if fmt == "q4_0":
+            b = torch.randint(0, 256, (n * k // 32, 18), dtype=torch.uint8, device="cuda", generator=gen)
+            b[:, :2] = (0.002 + 0.004 * torch.rand(n * k // 32, device="cuda", generator=gen)).half()[:, None].view(torch.uint8)
+            return rt.Q4_0, b.reshape(-1)
+        w = torch.randn((n, k), device="cuda", generator=gen) * 0.02
+        return (rt.BF16, w.bfloat16().view(torch.int16)) if fmt == "bf16" else (rt.Q4K, rt.quantize_q4k(w))
+
+    def time_of(code, w, x, n, k):
+        y, best = torch.empty((m, n), device="cuda"), 1e9
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                rt.gemv(code, w, x, n, k, y=y)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return y, best
+
+    code, w = make(n, k)
+    v = w.view(torch.bfloat16) if fmt == "bf16" else rt.dequant(code, w, n, k)
+    x = torch.randn((m, k), device="cuda", generator=gen)
+    y, t = time_of(code, w, x, n, k)
+    want = torch.cat([x.double() @ v.reshape(n, k)[i:i + 2048].double().T.contiguous() for i in range(0, n, 2048)], 1)
+    assert float((y.double() - want).abs().amax() / want.abs().amax()) <= GEMV_TOL
+    side = max(1024, int((n * k) ** 0.5) // 256 * 256)
+    code, w = make(side, side)
+    assert t <= 4 * time_of(code, w, x[:, :side].contiguous(), side, side)[1]
