@@ -583,8 +583,6 @@ int rt_hip_flux_attention(const float* q, const float* k, const float* v, float*
     if (t == 0) return RT_HIP_OK;
     hipError_t e;
     if (!state_for_current(&e)) return hip_fail(e, fn);
-    // the scale of flux.cpp:290 and metal_flux.mm:264, in f32
-    const float scale = 1.0f / std::sqrt(static_cast<float>(head_dim));
     const hipStream_t s = static_cast<hipStream_t>(stream);
     float* part = nullptr;
     uint32_t* counters = nullptr;
@@ -595,7 +593,7 @@ int rt_hip_flux_attention(const float* q, const float* k, const float* v, float*
         counters = part ? arrival_counters(s, &e) : nullptr;
         if (!counters) part = nullptr;
     }
-    return check_stream_launch(launch_flux_attention(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s),
+    return check_stream_launch(launch_flux_attention(q, k, v, out, t, n_heads, head_dim, part, counters, s),
                                fn);
 }
 

@@ -12,11 +12,12 @@
 // in tiles of 32 keys through LDS rings.
 //
 // f32 products on the bf16 matrix cores.  Every f32 factor is split into three
-// bf16 limbs with h + m + l == x exactly (24 bits of significand), and a
-// product is the six limb products hh, hm, mh, mm, hl, lh on
-// v_mfma_f32_32x32x16_bf16: products of bf16 values are exact in f32 and the
-// three left out (ml, lm, ll) are below 2^-25 of the product, under the
-// rounding of one f32 multiplication.  The matrix cores do a bf16 product at
+// bf16 limbs with h + m + l == x exactly (24 bits of significand; K and Q where
+// the last bit is 2^-133 or more, V and P always, see kUp), and a product is the
+// six limb products hh, hm, mh, mm, hl, lh on v_mfma_f32_32x32x16_bf16: products
+// of bf16 values are exact in f32 and the three left out (ml, lm, ll) are
+// together below 2^-24 of the product, at most the rounding of one f32
+// multiplication.  The matrix cores do a bf16 product at
 // 16 times the f32 rate, so six cost 3/8 of one f32 product.  Q's limbs live
 // in registers (split once per block), K's and V's are split as each tile is
 // staged, P's in the registers its scores were computed in:
@@ -28,13 +29,14 @@
 //  * Online softmax per query: the running maximum; each half of a query's
 //    keys keeps its own denominator (added at the end); the accumulator is
 //    rescaled by exp(m_old - m_new) where a maximum of the wave moved
-//    (flux.msl:232-271).
+//    (flux.msl:232-271).  Exponentials are powers of two: log2(e) and the scale
+//    are in Q's limbs.
 //  * O^T += V^T P^T: lane (h, n) supplies P[query n] of the eight keys it
 //    holds in registers 8s .. 8s + 7 and V[those keys][dim 32c + n], which V's
 //    LDS rows (one per dim, keys in that order) hold as 16 bytes; the result
 //    leaves lane (h, n) holding O[query n][dims 32c + 8i + 4h + r].
-// From a tile of K or V that holds a value of 2^64 or more, an infinity or a
-// NaN, or throughout a block with a query of 2^55 or more, the block takes f32
+// From a tile that holds a value of 2^64 or more in K, of 2^48 in V, an infinity
+// or a NaN, or throughout a block with a query of 2^55 or more, the block takes f32
 // MFMA steps on the staged f32 tiles: products that overflow and infinities
 // then behave as in f32 arithmetic (a limb's product could overflow to the
 // other sign).  A loop of its own: the limb loop has no registers to spare.
@@ -63,6 +65,8 @@
 //  * Tiles go through LDS copies of the raw f32 (no registers), are split once
 //    and read by all 8 waves: blocks of 128 queries halve the reuse of the
 //    splits and are taken only where 256 leave CUs idle.
+#include <cmath>
+
 #include "rt_common.hpp"
 #include "rt_launch.hpp"
 
@@ -73,10 +77,15 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBK = 32;  // keys per tile
-constexpr float kLog2e = 1.44269504088896341f;
 constexpr uint32_t kNoRead = 0x7ffffff0u;  // past every tile's range: reads zeros
 
-__device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
+// V and the weights P enter the limbs times 2^16: bf16 has f32's exponents but 7
+// bits, so the third limb of a value below 2^-109 would fall below bf16's
+// smallest value, 2^-133.  With the factor every bit of an f32 value (2^-149 and
+// up) is in reach.  (The matrix unit keeps bf16 values below 2^-126.)
+constexpr float kUp = 0x1p16f, kDown = 0x1p-32f;
+
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // LDS: a ring of two tiles of K limbs [3][32 keys][DP] bf16, then one of three
 // tiles of V limbs [3][DP dims][32 keys], then each wave's share of a tile's
@@ -131,8 +140,9 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, 
 }
 // Adds the squares of a pair's high limbs to acc: NaN or infinite once one of
 // them is NaN or 2^64 or more in magnitude.  A sum that stays finite bounds
-// every value of K and V, and with |q| < 2^55 a score (128 products below
-// 2^119) and each of its limb products stays finite too.
+// every value of K and, times 2^16, of V; with |q| < 2^55 a score (128 products
+// below 2^119) and each of its limb products stays finite too, and so does a
+// sum of T < 2^31 products of V and P (2^64 2^16 each).
 constexpr float kQLimit = 0x1p55f;
 __device__ __forceinline__ float limb_check(uint32_t h, float acc) {
     const bf16x2 v = __builtin_bit_cast(bf16x2, h);
@@ -182,7 +192,7 @@ __device__ __forceinline__ float other_half(float x, int h) {
 template <int DP, int NW>
 __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux_attn(const float* __restrict__ Q, const float* __restrict__ K,
                                                           const float* __restrict__ V, float* __restrict__ O, int T,
-                                                          int n_heads, int D, float scale, float* __restrict__ part,
+                                                          int n_heads, int D, float scale2, float* __restrict__ part,
                                                           uint32_t* __restrict__ cnt, int per) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t arrival;
@@ -284,7 +294,8 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
                 for (int e = 0; e < 2; ++e) {
                     uint32_t x, y, z;
                     const uint8_t* const src = raw + KU * 2048 + (4 * i + 2 * e) * 256 + lane * 4;
-                    split2(*reinterpret_cast<const float*>(src), *reinterpret_cast<const float*>(src + 256), x, y, z);
+                    split2(*reinterpret_cast<const float*>(src) * kUp, *reinterpret_cast<const float*>(src + 256) * kUp, x, y,
+                           z);
                     a[e] = x;
                     b[e] = y;
                     c[e] = z;
@@ -319,10 +330,12 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
         for (int a = 0; a < KS; ++a) {
             float x[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = 16 * a + 8 * h < D ? qx[a][e >> 2][e & 3] : 0.0f;
+            for (int e = 0; e < 8; ++e) {
+                x[e] = 16 * a + 8 * h < D ? qx[a][e >> 2][e & 3] : 0.0f;
+                qbad |= !(fabsf(x[e]) < kQLimit);
+                x[e] *= scale2;  // (the scores then come out scaled)
+            }
             split8(x, qh[a], qm[a], ql[a]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qbad |= !(fabsf(x[e]) < kQLimit);
             __builtin_amdgcn_sched_barrier(0);
         }
         f32x16 o[NC];  // o[c][4i + r]: O[query n][dim 32c + 8i + 4h + r]
@@ -330,12 +343,11 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
         for (int c = 0; c < NC; ++c) o[c] = f32x16{};
         float m_run = -__builtin_inff(), l_run = 0.0f;  // of query n; l of this half's keys
 
-        // Scores of query n scaled, masked and turned into weights; the
-        // running state and the accumulator moved to the new maximum.
+        // Scores of query n, times scale log2(e), masked and turned into weights;
+        // the running state (m in powers of two) and the accumulator moved to
+        // the new maximum.
         auto softmax = [&](f32x16& s, int base) {
             float mx = -__builtin_inff();
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s[e] *= scale;
             if (base + kBK > T) {
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
@@ -345,11 +357,11 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
             for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
             mx = fmaxf(mx, other_half(mx, h));
             const float m_new = fmaxf(m_run, mx);  // finite for finite scores: key `base` is valid
-            const float alpha = exp_fast(m_run - m_new);  // 0 on the first tile
+            const float alpha = exp2_fast(m_run - m_new);  // 0 on the first tile
             float sum = 0.0f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                s[e] = exp_fast(s[e] - m_new);  // -inf -> 0
+                s[e] = exp2_fast(s[e] - m_new);  // -inf -> 0
                 sum += s[e];
             }
             l_run = l_run * alpha + sum;
@@ -463,8 +475,9 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
             softmax(s, (t0 + i) * kBK);
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const float p[8] = {s[8 * t], s[8 * t + 1], s[8 * t + 2], s[8 * t + 3],
-                                    s[8 * t + 4], s[8 * t + 5], s[8 * t + 6], s[8 * t + 7]};
+                float p[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) p[e] = s[8 * t + e] * kUp;
                 split8(p, ph[t], pm[t], pl[t]);
             }
             // (opaque: the compiler would compute them in the next phase)
@@ -486,7 +499,11 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
         // copies of a tile, every wave's share, hold it whole: K units of 4 dims
         // at 16 bytes a lane, V units of one dim at 4.  Half h takes dims 8a + 4h
         // .. + 3 of a step.
+        float unit = kDown;  // of o
         if (nt < t1 - t0) {
+            unit = 1.0f;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) o[c] *= kDown;
             const uint8_t* const shares = lds + 15 * kPlane;
             constexpr int kShare = raw_wave_bytes<DP, NW>(), kRows = NT / DP;
             const float* const qp = qb + min(qrow, T - 1) * stride;  // (rows past T are not stored)
@@ -506,6 +523,7 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
                     for (int e = 0; e < 4; ++e)
                         s = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[e], dim < D ? qa[e] : 0.0f, s, 0, 0, 0);
                 }
+                s *= scale2;
                 softmax(s, tile * kBK);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {  // key 8 (e / 4) + 4h + e % 4
@@ -536,24 +554,31 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
                 for (int e = 0; e < 16; ++e) st_dev(mine + qi * DP + 32 * c + 8 * (e >> 2) + 4 * h + (e & 3), o[c][e]);
             if (h == 0) {
                 st_dev(mine + BQ * DP + qi, m_run);
-                st_dev(mine + BQ * DP + BQ + qi, l_run);
+                st_dev(mine + BQ * DP + BQ + qi, unit == 1.0f ? -l_run : l_run);  // l > 0: its sign is o's unit
             }
             wait_vmcnt<0>();
             __syncthreads();
-            // acq_rel at agent scope: the release orders this piece's state
-            // stores before the arrival, and the acquire orders the merging
-            // piece's loads of the other state after it.
-            if (tid == 0) arrival = __hip_atomic_fetch_add(cnt + bnd, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            // Relaxed: the state went out in agent-scope stores that every wave
+            // has waited for before the barrier, and the merging piece reads it
+            // with agent-scope loads once the arrival's result is known.  (A
+            // release wrote the XCD's whole L2 back: 700 tokens, 100 heads of 64
+            // 134 us, 121 without.)
+            if (tid == 0) arrival = __hip_atomic_fetch_add(cnt + bnd, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
             if (arrival == 0) continue;  // the other piece merges
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             // Merge: m = max, each side scaled by exp(m_side - m).  Two terms,
             // so the result does not depend on which piece merges.
             const float* other = part + (static_cast<int64_t>(bnd) * 2 + (1 - piece)) * kPiece;
-            const float mo = ld_dev(other + BQ * DP + qi), lo = ld_dev(other + BQ * DP + BQ + qi);
+            const float mo = ld_dev(other + BQ * DP + qi), lu = ld_dev(other + BQ * DP + BQ + qi), lo = fabsf(lu);
+            const float unit_o = __builtin_signbit(lu) ? 1.0f : kDown;
             const float m = fmaxf(m_run, mo);
-            const float am = exp_fast(m_run - m), ao = exp_fast(mo - m);
+            float am = exp2_fast(m_run - m), ao = exp2_fast(mo - m);
             l_run = l_run * am + lo * ao;
+            if (unit != unit_o) {
+                am *= unit;
+                ao *= unit_o;
+                unit = 1.0f;
+            }
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -564,7 +589,7 @@ __global__ __launch_bounds__(NW* kWave, NW == 4 && DP <= 64 ? 2 : 1) void k_flux
         // out[query n][dims 32c + 8i + 4h ..]: divide by the denominator
         if (qrow < T) {
             float* dst = O + qrow * stride + static_cast<int64_t>(head) * D;
-            const float inv = 1.0f / l_run;
+            const float inv = unit / l_run;
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -585,20 +610,21 @@ int flux_slots() { return static_cast<int>(device_info().cus); }
 int padded_dims(int head_dim) { return head_dim <= 32 ? 32 : (head_dim <= 64 ? 64 : 128); }
 
 template <int DP, int NW>
-hipError_t run(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads, int d, float scale,
-               float* part, uint32_t* cnt, hipStream_t s) {
+hipError_t run(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads, int d, float* part, uint32_t* cnt, hipStream_t s) {
     constexpr int BQ = 32 * NW;
     const int64_t nqb = (t + BQ - 1) / BQ, ntile = (t + kBK - 1) / kBK, items = n_heads * nqb;
     const size_t lds = flux_lds_bytes<DP, NW>();
+    // log2(e) / sqrt(d): the scale of flux.cpp:290 and metal_flux.mm:264
+    const float scale2 = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(d)));
     if (!part) {
         const dim3 grid(static_cast<unsigned>(n_heads), static_cast<unsigned>(nqb));
         hipLaunchKernelGGL((k_flux_attn<DP, NW>), grid, dim3(NW * kWave), lds, s, q, k, v, out,
-                           static_cast<int>(t), n_heads, d, scale, nullptr, nullptr, 0);
+                           static_cast<int>(t), n_heads, d, scale2, nullptr, nullptr, 0);
     } else {
         const int slots = flux_slots();
         const int64_t per = (items * ntile + slots - 1) / slots;  // >= ntile: more items than slots
         hipLaunchKernelGGL((k_flux_attn<DP, NW>), dim3(static_cast<unsigned>(slots)), dim3(NW * kWave),
-                           lds, s, q, k, v, out, static_cast<int>(t), n_heads, d, scale, part, cnt,
+                           lds, s, q, k, v, out, static_cast<int>(t), n_heads, d, scale2, part, cnt,
                            static_cast<int>(per));
     }
     return hipGetLastError();
@@ -616,11 +642,10 @@ bool half_blocks(int64_t t, int n_heads) {
 }
 
 template <int DP>
-hipError_t run_dp(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads, int d, float scale,
-                  float* part, uint32_t* cnt, hipStream_t s) {
+hipError_t run_dp(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads, int d, float* part, uint32_t* cnt, hipStream_t s) {
     if (half_blocks(t, n_heads))
-        return run<DP, 4>(q, k, v, out, t, n_heads, d, scale, nullptr, nullptr, s);
-    return run<DP, 8>(q, k, v, out, t, n_heads, d, scale, part, cnt, s);
+        return run<DP, 4>(q, k, v, out, t, n_heads, d, nullptr, nullptr, s);
+    return run<DP, 8>(q, k, v, out, t, n_heads, d, part, cnt, s);
 }
 
 }  // namespace
@@ -633,12 +658,12 @@ size_t flux_attention_workspace(int64_t t, int n_heads, int head_dim) {
 }
 
 hipError_t launch_flux_attention(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads,
-                                 int head_dim, float scale, float* part, uint32_t* counters, hipStream_t s) {
+                                 int head_dim, float* part, uint32_t* counters, hipStream_t s) {
     if (part && (!counters || static_cast<size_t>(flux_slots()) > kArrivalCounters)) return hipErrorInvalidValue;
     switch (padded_dims(head_dim)) {
-        case 32: return run_dp<32>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s);
-        case 64: return run_dp<64>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s);
-        default: return run_dp<128>(q, k, v, out, t, n_heads, head_dim, scale, part, counters, s);
+        case 32: return run_dp<32>(q, k, v, out, t, n_heads, head_dim, part, counters, s);
+        case 64: return run_dp<64>(q, k, v, out, t, n_heads, head_dim, part, counters, s);
+        default: return run_dp<128>(q, k, v, out, t, n_heads, head_dim, part, counters, s);
     }
 }
 

@@ -55,7 +55,7 @@ hipError_t launch_gemv_q4k_bias(const void* w, const float* x, const float* bias
 // null otherwise.
 size_t flux_attention_workspace(int64_t t, int n_heads, int head_dim);
 hipError_t launch_flux_attention(const float* q, const float* k, const float* v, float* out, int64_t t, int n_heads,
-                                 int head_dim, float scale, float* part, uint32_t* counters, hipStream_t s);
+                                 int head_dim, float* part, uint32_t* counters, hipStream_t s);
 
 // Decode attention (attention.hip): head_dim 128, n_q / n_kv in {1, 2, 3, 4};
 // `part` holds attention_decode_workspace(...) bytes.

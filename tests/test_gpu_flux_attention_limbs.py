@@ -1,7 +1,7 @@
 """FLUX's attention at the edges of its blocks and at values its bf16 limbs do
 not take: 128- and 256-query blocks, 32-key tiles and every padded head width;
-values past 2^64 (2^55 in q), infinities and NaN, which go through f32 matrix
-steps; products that overflow; tiny values; a capture without workspace.
+values past 2^64 (2^48 in v, 2^55 in q), infinities and NaN, which go through f32
+matrix steps; products that overflow; tiny values; a capture without workspace.
 
 Bound: FLUX_ATTN_TOL of test_gpu_flux_attention.py (1e-5 of the largest
 output) against float64."""
@@ -143,6 +143,36 @@ def test_flux_attention_scaled_values(rt, scale):
     q, k, v = rand(t, h, d)
     v = (v * np.float32(scale)).astype(np.float32)
     assert normwise_err(run(rt, q, k, v, h, d), exact(q, k, v, h, d)) <= FLUX_ATTN_TOL
+
+
+# (2^100: normwise_err measures against 1e-30 at least)
+@pytest.mark.parametrize("t,h,d", [(300, 4, 64), (700, 100, 128), (512, 100, 32)])
+@pytest.mark.parametrize("scale", [1e-33, 1e-35, 1e-37])
+def test_flux_attention_tiny_columns(rt, t, h, d, scale):
+    """v of f32's smallest normal values in some dims keeps f32's bits there,
+    beside ordinary dims."""
+    say(f"[flux limbs tiny] t={t} heads={h} head_dim={d} v x {scale}")
+    q, k, v = rand(t, h, d)
+    tiny = np.arange(h * d) % 3 == 0
+    v = np.where(tiny, v * np.float32(scale), v).astype(np.float32)
+    got, want = run(rt, q, k, v, h, d), exact(q, k, v, h, d)
+    assert normwise_err(got[:, ~tiny], want[:, ~tiny]) <= FLUX_ATTN_TOL
+    assert normwise_err(got[:, tiny] * 2.0 ** 100, want[:, tiny] * 2.0 ** 100) <= FLUX_ATTN_TOL
+
+
+def test_flux_attention_tiny_weights(rt):
+    """Weights of 2^-122 on every key that has a value keep f32's bits.  Bound: a
+    weight's exponent of 122 rounds by 122 * 2^-24 = 7.3e-6 in q and as much in
+    the subtracted maximum."""
+    t, h, d = 600, 3, 64
+    say("[flux limbs tiny] weights")
+    q, k, v = rand(t, h, d)
+    q[:], k[:] = 0.0, 0.0
+    q[:, ::d], k[:, ::d] = 8.0, -42.25
+    k[77, ::d], v[77] = 42.25, 0.0
+    got, want = run(rt, q, k, v, h, d), exact(q, k, v, h, d)
+    assert 0 < np.abs(want).max() < 1e-33
+    assert normwise_err(got * 2.0 ** 120, want * 2.0 ** 120) <= 2e-5
 
 
 def test_flux_attention_captured_without_workspace(rt):
