@@ -823,7 +823,13 @@ GemmPlan plan_gemm(int w_fmt, bool a_bf16, int64_t m, int64_t n, int64_t k) {
     const bool four_bit = w_fmt == RT_HIP_Q4MAT || w_fmt == RT_HIP_Q4_0;
     // Every BF16 K % 64 == 0 is whole 64-wide steps (a step count that is not a
     // multiple of four runs up to three steps of zeros: 2 of 20 at K = 1152).
-    p.pipe = w_fmt == RT_HIP_BF16 || (k % 256 == 0 && (w_fmt == RT_HIP_Q4K || four_bit));
+    // Of at most three steps and few rows, the pipeline's four steps and the
+    // launch that converts A cost more than k_gemm's steps one after another
+    // (9 x 1024 x 128: 8.7 us against 10.1 with f32 A, 6.6 against 8.2 with
+    // bf16; 33 x 1024 x 64: 8.5 against 8.9 with f32 A, 7.7 against 7.1 with
+    // bf16; 64 x 64 x 64: 12.0 against 10.3).
+    const bool few = a_bf16 ? m <= 32 && k <= 3 * BK : m <= 48 && k <= 2 * BK;
+    p.pipe = (w_fmt == RT_HIP_BF16 && !few) || (k % 256 == 0 && (w_fmt == RT_HIP_Q4K || four_bit));
     if (!p.pipe) return p;
     // A Q4_K weight is dequantized (bf16, round-to-nearest-even of the exact
     // f32 value, as the reference's flux_dequant_q4k) either inside the GEMM
@@ -858,7 +864,9 @@ GemmPlan plan_gemm(int w_fmt, bool a_bf16, int64_t m, int64_t n, int64_t k) {
     // the CUs idle: up to 4 slices of K (8 for k_gemm_ws), summed afterwards
     // in a fixed order (deterministic).  Slices are multiples of 64 values
     // (256 for k_gemm_ws, whose slices start on super-blocks).
-    if (!p.big && 2 * p.mt * p.nt <= cus && n % 4 == 0) {
+    // Not below a round of four steps, which a slice of one or two runs as well
+    // (1024 x 1024 x 128: 14.3 us whole, 16.9 in two).
+    if (!p.big && 2 * p.mt * p.nt <= cus && n % 4 == 0 && k >= 4 * BK) {
         const int cap = p.ws ? 8 : 4, unit = p.ws ? 256 : 64;
         int splits = static_cast<int>(cus / (p.mt * p.nt));
         splits = splits > cap ? cap : splits;

@@ -29,6 +29,40 @@ def test_bf16_gemm_k64(rt, m, n, k, a_bf16):
     assert same_operand_err(c - bias, a, w) <= 2 * GEMM_TOL_SAME_OPERANDS  # 2: the bias subtracted again in f32
 
 
+# Few rows and at most three steps of K take the kernel without a pipeline:
+# both sides of each line, and the one-slice launches of short K.
+@pytest.mark.parametrize("m,n,k,a_bf16", [(9, 68, 64, False), (48, 132, 128, False), (49, 132, 128, False),
+                                          (9, 132, 192, True), (32, 1024, 192, True), (33, 1024, 192, True),
+                                          (9, 1024, 192, False), (300, 1028, 128, True), (1000, 516, 128, False)])
+def test_bf16_gemm_short_k(rt, m, n, k, a_bf16):
+    test_bf16_gemm_k64(rt, m, n, k, a_bf16)
+
+
+def test_bf16_gemm_short_k_cost(rt):
+    """K of two steps over many rows is not summed from slices of one step: it
+    costs less than K of eight."""
+    import torch
+    say("[gemm k64] short K cost")
+    m = n = 1024
+
+    def time_of(k):
+        a = torch.randn((m, k), device="cuda").bfloat16()
+        w = torch.randn((n, k), device="cuda").bfloat16()
+        c, best = torch.empty((m, n), device="cuda"), 1e9
+        for _ in range(6):
+            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            s.record()
+            for _ in range(50):
+                rt.gemm(rt.BF16, a, w.view(torch.int16), n, k, c=c)
+            e.record()
+            torch.cuda.synchronize()
+            best = min(best, s.elapsed_time(e))
+        return best
+
+    assert rt.library().lib.rt_hip_gemm_workspace_bytes(rt.BF16, rt.BF16, m, n, 128) == 0
+    assert time_of(128) < time_of(512)
+
+
 @pytest.mark.parametrize("fmt,k", [("q4_0", 320), ("q4mat", 1152)])
 def test_4bit_gemm_k64(rt, fmt, k):
     import torch
