@@ -8,6 +8,7 @@ output) against float64."""
 import numpy as np
 import pytest
 
+from fresh_process import run_case
 from helpers import from_dev, normwise_err, say, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -176,20 +177,5 @@ def test_flux_attention_tiny_weights(rt):
 
 
 def test_flux_attention_captured_without_workspace(rt):
-    import torch
-    t, h, d = 700, 100, 128
-    f = rt.library().lib.rt_hip_flux_attention_workspace_bytes
-    say(f"[flux limbs] captured: workspace {rt.workspace_bytes()}, need {f(t, h, d)}")
-    q, k, v = rand(t, h, d)
-    dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
-    out = torch.zeros_like(dq)
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        rt.flux_attention(dq, dk, dv, h, d, out=out)
-    want = exact(q, k, v, h, d)
-    for _ in range(3):
-        out.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert normwise_err(from_dev(out), want) <= FLUX_ATTN_TOL
+    say("[flux limbs] captured without workspace")
+    run_case("flux")

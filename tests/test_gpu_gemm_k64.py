@@ -8,7 +8,8 @@ operands against float64 (as test_gpu_gemm.py)."""
 import numpy as np
 import pytest
 
-from helpers import GEMM_TOL_SAME_OPERANDS, from_dev, normwise_err, same_operand_err, say
+from fresh_process import run_case
+from helpers import GEMM_TOL_SAME_OPERANDS, same_operand_err, say
 
 pytestmark = pytest.mark.gpu
 
@@ -83,28 +84,7 @@ def test_4bit_gemm_k64(rt, fmt, k):
     assert same_operand_err(rt.gemm(code, a, w, n, k), a, wide) <= GEMM_TOL_SAME_OPERANDS
 
 
-@pytest.mark.parametrize("a_bf16", [False, True])
-def test_bf16_gemm_k64_captured_without_workspace(rt, a_bf16):
-    import torch
-    m, n, k = 200, 256, 1152
-    lib = rt.library().lib
-    while lib.rt_hip_gemm_workspace_bytes(rt.BF16, rt.F32, m, n, k) <= rt.workspace_bytes() and m < 20000:
-        m *= 2
-    say(f"[gemm k64] captured {m} x {n} x {k}, workspace {rt.workspace_bytes()} bytes")
-    g = torch.Generator(device="cuda").manual_seed(2)
-    a = torch.randn((m, k), device="cuda", generator=g)
-    if a_bf16:
-        a = a.to(torch.bfloat16)
-    w = (torch.randn((n, k), device="cuda", generator=g) * 0.02).to(torch.bfloat16)
-    c = torch.zeros((m, n), device="cuda")
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        rt.gemm(rt.BF16, a, w.view(torch.int16), n, k, c=c)
-    for _ in range(3):
-        c.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert same_operand_err(c, a, w) <= GEMM_TOL_SAME_OPERANDS
-    eager = from_dev(rt.gemm(rt.BF16, a, w.view(torch.int16), n, k))
-    assert normwise_err(from_dev(c), eager) <= GEMM_TOL_SAME_OPERANDS
+@pytest.mark.parametrize("case", ["gemm_f32", "gemm_bf16", "gemm_q4_0", "gemm_q4mat"])
+def test_gemm_k64_captured_without_workspace(rt, case):
+    say(f"[gemm k64] captured without workspace: {case}")
+    run_case(case)

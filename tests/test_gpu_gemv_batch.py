@@ -14,6 +14,7 @@ the bound the single-row GEMVs are held to.
 import numpy as np
 import pytest
 
+from fresh_process import run_case
 from helpers import GEMV_TOL, f32_to_bf16_rne, bf16_bits_to_f32, from_dev, normwise_err, say, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -97,29 +98,11 @@ def test_batched_gemv_long_output(rt, orc, fmt):
             assert np.array_equal(y[:, r0:r1], y[:, :r1 - r0]), r0
 
 
-def test_batched_gemv_without_workspace_room(rt, orc):
+def test_batched_gemv_without_workspace_room(rt):
     """A shape that is split over workgroups, captured without room to grow the
     workspace, keeps K inside its workgroups: accepted, and right."""
-    import torch
-    lib = rt.library().lib
-    m, k = 8, 12288
-    n = 64
-    while lib.rt_hip_gemv_workspace_bytes(rt.Q4_0, n, k, m) <= rt.workspace_bytes() and n < 4096:
-        n *= 2
-    rng = np.random.default_rng(5)
-    w, v = weights(rt, orc, "q4_0", rng, n, k)
-    x = rng.standard_normal((m, k)).astype(np.float32)
-    dx, y = to_dev(x), torch.zeros((m, n), device="cuda")
-    say(f"[gemv batch] Q4_0 {n} x {k} captured, workspace {rt.workspace_bytes()} bytes")
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        rt.gemv(rt.Q4_0, w, dx, n, k, y=y)
-    for _ in range(3):
-        y.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert normwise_err(from_dev(y), x.astype(np.float64) @ v.T) <= GEMV_TOL
+    say("[gemv batch] Q4_0 captured without workspace")
+    run_case("gemv_q4_0")
 
 
 @pytest.mark.parametrize("fmt", ["q4k", "bf16", "q4_0", "q4mat"])
