@@ -161,10 +161,18 @@ bool capturing(hipStream_t s) {
     return st != hipStreamCaptureStatusNone;
 }
 
+// hipMalloc whose failure leaves no error pending: a caller that goes on
+// without the memory, or comes back later, would find it after its next launch.
+hipError_t try_malloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 // Grows st's workspace to `bytes` (caller holds g_mu); `capture`: the
 // caller's stream is being captured, so no allocation may happen.
 hipError_t grow_workspace(DeviceState* st, size_t bytes, bool capture) {
-    const int rc = st->ws.reserve(bytes, capture, [](void** p, size_t n) { return static_cast<int>(hipMalloc(p, n)); });
+    const int rc = st->ws.reserve(bytes, capture, [](void** p, size_t n) { return static_cast<int>(try_malloc(p, n)); });
     if (rc == WorkspacePool::kRefused) return hipErrorStreamCaptureUnsupported;
     return static_cast<hipError_t>(rc);
 }
@@ -174,7 +182,7 @@ hipError_t grow_workspace(DeviceState* st, size_t bytes, bool capture) {
 hipError_t make_counters(DeviceState* st) {
     if (st->counters) return hipSuccess;
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, kArrivalCounters * sizeof(uint32_t));
+    hipError_t e = try_malloc(&p, kArrivalCounters * sizeof(uint32_t));
     if (e != hipSuccess) return e;
     e = hipMemset(p, 0, kArrivalCounters * sizeof(uint32_t));
     if (e == hipSuccess) e = hipDeviceSynchronize();

@@ -121,8 +121,24 @@ def flux(rt):
     replays(rt, lambda: rt.flux_attention(dq, dk, dv, h, d, out=out), out, check)
 
 
+def failed_growth(rt):
+    """A workspace that cannot be allocated is an error of that call alone."""
+    import torch
+    y = rt.gemv(rt.BF16, torch.zeros((16, 256), dtype=torch.int16, device="cuda"), torch.ones((2, 256), device="cuda"),
+                16, 256)
+    try:
+        rt.reserve_workspace(1 << 46)
+        raise AssertionError("64 TiB of workspace")
+    except rt.RtHipError as e:
+        assert e.code == 4  # RT_HIP_E_OOM
+    x = torch.ones((2, 256), device="cuda")
+    rt.gemv(rt.BF16, torch.zeros((16, 256), dtype=torch.int16, device="cuda"), x, 16, 256, y=y)
+    assert (y == 0).all()
+
+
 CASES = {"gemv_q4_0": gemv_q4_0, "gemm_f32": lambda rt: gemm(rt, False), "gemm_bf16": lambda rt: gemm(rt, True),
-         "gemm_q4_0": lambda rt: gemm_4bit(rt, "q4_0"), "gemm_q4mat": lambda rt: gemm_4bit(rt, "q4mat"), "flux": flux}
+         "gemm_q4_0": lambda rt: gemm_4bit(rt, "q4_0"), "gemm_q4mat": lambda rt: gemm_4bit(rt, "q4mat"), "flux": flux,
+         "failed_growth": failed_growth}
 
 if __name__ == "__main__":
     sys.path.insert(0, HERE)

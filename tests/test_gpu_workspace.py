@@ -5,11 +5,13 @@ and the fused BF16 GEMV + argmax (its key in the workspace) keeps writing
 the buffers those calls used on every replay.  A later eager GEMM that needs
 more workspace replaces the buffer; the old one must stay valid (retired,
 not freed), so replays after the growth still match the oracle.  Growth
-during capture is refused with an error instead of allocating.
+during capture is refused with an error instead of allocating, and growth that
+fails leaves nothing behind.
 """
 import numpy as np
 import pytest
 
+from fresh_process import run_case
 from helpers import GEMV_TOL, from_dev, normwise_err, say, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +101,9 @@ def test_graph_replays_survive_workspace_growth(rt, orc):
             rt.gemm(rt.Q4K, a2, blocks, gn, gk, c=c2)
     torch.cuda.synchronize()
     check("replay 4, after a refused capture")
+
+
+def test_failed_growth_leaves_no_error(rt):
+    """An allocation that fails leaves no error behind for the next launch's check."""
+    say("[workspace] failed growth")
+    run_case("failed_growth")
