@@ -56,6 +56,25 @@ def test_q4k_tiled_large_k(rt, orc, n, k):
     assert normwise_err(from_dev(y2).reshape(-1), want2) <= GEMV_TOL
 
 
+@pytest.mark.parametrize("n,k", [(40, 9216), (3072, 10240), (9000, 9216), (300, 17408), (300, GEMMA27_DOWN_K)])
+def test_q4k_tiled_residual_and_bias_long_k(rt, orc, n, k):
+    """resid += W . x, and W . x + bias, where x has more values than the register
+    batches of a workgroup's threads hold: 8 f32x4 a thread (K above 8192 at 256
+    threads), and 16, past which the rest is staged by a loop.  The residual form
+    once left out what lay past 8."""
+    say(f"[large k] Q4_K residual, bias N={n} K={k}")
+    rng = np.random.default_rng(n + k)
+    blocks = q4k_weight(orc, rng, n, k)
+    x = rng.standard_normal((1, k)).astype(np.float32)
+    r = rng.standard_normal(n).astype(np.float32)
+    want = r + orc.q4k_matmul_t(blocks, n, k, x).reshape(-1)
+    resid = to_dev(r)
+    rt.gemv_q4k_tiled_residual(rt.q4k_tile(to_dev(blocks), n, k), to_dev(x), resid, n, k)
+    assert normwise_err(from_dev(resid), want) <= GEMV_TOL
+    y = rt.linear_forward(rt.Q4K, to_dev(blocks), to_dev(x), n, k, bias=to_dev(r))
+    assert normwise_err(from_dev(y).reshape(-1), want) <= GEMV_TOL
+
+
 def test_q4k_tiled_swiglu_residual_gemma27_down(rt, orc):
     """The MLP's down projection and its residual add at Gemma-3-27B's ffn:
     resid += W . (silu(gate) * up)."""
