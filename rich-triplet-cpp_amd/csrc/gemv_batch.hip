@@ -942,7 +942,7 @@ size_t gemv_batch_workspace_bytes(int fmt, int64_t n, int64_t k, int m) {
 
 hipError_t launch_gemv_batch(int fmt, const void* w, const float* x, float* y, int64_t n, int64_t k, int m,
                              hipStream_t s, const float* bias) {
-    if (m < 1 || m > 8) return hipErrorInvalidValue;
+    if (m < 2 || m > 8) return hipErrorInvalidValue;
     switch (fmt) {
         case RT_HIP_Q4K: return dispatch<BQ4k>(w, x, y, n, k, m, 0, s, bias);
         case RT_HIP_BF16: return dispatch<BBf16>(w, x, y, n, k, m, 0, s, bias);

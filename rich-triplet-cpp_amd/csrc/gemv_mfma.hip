@@ -745,14 +745,17 @@ hipError_t run_xp(const Jobs& jobs, const float* x, const XArgs& xa, int64_t k, 
     const int64_t per = (k / 4 + xthreads - 1) / xthreads;
     // At most 16 float4 per thread in registers, 8 with an x operation (its
     // second vector doubles the registers); the rest of a longer x is
-    // staged by a loop after them.
-    constexpr bool kPlain = XOP == kXNone;  // (kHasRest: 16 f32x4, then the loop)
-    if (EPI != kEpiBias && jobs.count > 2) {
-        if (per <= 2) return run<D, 2, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-        if (per <= 3) return run<D, 3, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-        if (per <= 4) return run<D, 4, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-        if (per <= 8 || !kPlain) return run<D, 8, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-        if constexpr (kPlain) return run<D, 16, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+    // staged by a loop after them, in the instances that kHasRest names: those
+    // of 16 where no x operation runs, whatever the epilogue.
+    constexpr bool kPlain = XOP == kXNone;
+    if constexpr (EPI != kEpiBias) {  // (the bias form has one job)
+        if (jobs.count > 2) {
+            if (per <= 2) return run<D, 2, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+            if (per <= 3) return run<D, 3, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+            if (per <= 4) return run<D, 4, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+            if (per <= 8 || !kPlain) return run<D, 8, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+            if constexpr (kPlain) return run<D, 16, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+        }
     }
     if (per <= 2) return run<D, 2, TILED, false, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
     if (per <= 3) return run<D, 3, TILED, false, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
@@ -851,7 +854,8 @@ hipError_t dispatch(const Jobs& jobs, const float* x, int64_t k, hipStream_t s, 
         return jobs.count > 2 ? run<4, 2, TILED, true, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s)
                               : run<4, 2, TILED, false, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s);
     } else {
-        if (sh.cw == 8) return run_xp<4, TILED, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s);
+        if constexpr (TILED)  // (row-major weights run no converter waves)
+            if (sh.cw == 8) return run_xp<4, TILED, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s);
         if constexpr (XOP != kXNone || EPI != kEpiNone) {
             return run_xp<4, TILED, XOP, EPI>(jobs, x, xa, k, ks, waves, s);
         } else {

@@ -1,7 +1,6 @@
 // q4mat.hip -- the reference's own 4-bit format, Q4Mat (include/rt/quant.hpp:
 // 23-75, src/quant_q4.cpp:17-156), on the GPU: the M = 1 GEMV (batches:
-// gemv_batch.hip), and the
-// dequantization to bf16 / f32 that the any-M GEMM and the parity tests use;
+// gemv_batch.hip), and the dequantization to bf16 / f32 that the any-M GEMM and the parity tests use;
 // plus the GGUF Q4_0 dequantization for the same GEMM path.
 //
 // Q4Mat storage, one device buffer (rt_hip.h):
@@ -17,7 +16,7 @@
 //     sum_j x_j w_j = scale * (sum_j (nib_j ^ 8) x_j - 8 * sum_j x_j):
 // the XOR flips bit 3 of every nibble at once (v ^ 0x88888888) and the
 // group's sum of x is precomputed when x is staged.  A lane owns whole
-// groups (one 16-byte and one 4-byte load), x [M][K] sits in LDS
+// groups (one 16-byte and one 4-byte load), x sits in LDS
 // chunk-major (16-byte chunk c of group g at (c*NG + g)*16, so the lanes of
 // one LDS read hit consecutive chunks), rows are reduced across the wave.
 // Numerics: f32, factorized and reordered against the reference's
@@ -41,38 +40,35 @@ __device__ __forceinline__ float dpp_f(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 
-// x[M][K] -> LDS chunk-major per row, with the per-group sums.  Thread f
-// handles 16-byte chunk f of the flattened x; a group's 8 chunks are 8
-// consecutive threads (DPP sum within the aligned 8-lane group).
-template <int M>
+// x -> LDS chunk-major, with the per-group sums.  Thread f handles 16-byte
+// chunk f of x; a group's 8 chunks are 8 consecutive threads (DPP sum within
+// the aligned 8-lane group).
 __device__ __forceinline__ void stage_x(const float* __restrict__ X, int K, f32x4* xs, float* sums) {
     const int NG = K >> 5, nx4 = K >> 2;
-    for (int f0 = 0; f0 < M * nx4; f0 += kT) {
+    for (int f0 = 0; f0 < nx4; f0 += kT) {
         const int f = f0 + static_cast<int>(threadIdx.x);
-        const bool in = f < M * nx4;
+        const bool in = f < nx4;
         const f32x4 v = reinterpret_cast<const f32x4*>(X)[in ? f : 0];
         float s = (v[0] + v[1]) + (v[2] + v[3]);
         s += dpp_f<0xb1>(s);   // lane ^ 1
         s += dpp_f<0x4e>(s);   // lane ^ 2
         s += dpp_f<0x141>(s);  // half-row mirror: lane i <-> 7 - i
         if (in) {
-            const int m = f / nx4, c = f - m * nx4;
-            xs[m * nx4 + (c & 7) * NG + (c >> 3)] = v;
-            if ((c & 7) == 0) sums[m * NG + (c >> 3)] = s;
+            xs[(f & 7) * NG + (f >> 3)] = v;
+            if ((f & 7) == 0) sums[f >> 3] = s;
         }
     }
     lds_barrier();
 }
 
-template <int M>
 __global__ __launch_bounds__(kT) void k_gemv_q4mat(const uint8_t* __restrict__ P, const float* __restrict__ S,
                                                    const float* __restrict__ X, float* __restrict__ Y, int N,
                                                    int K) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int NG = K >> 5, nx4 = K >> 2;
     f32x4* const xs = reinterpret_cast<f32x4*>(lds);
-    float* const sums = reinterpret_cast<float*>(lds + static_cast<size_t>(16) * M * nx4);
-    stage_x<M>(X, K, xs, sums);
+    float* const sums = reinterpret_cast<float*>(lds + static_cast<size_t>(16) * nx4);
+    stage_x(X, K, xs, sums);
 
     const int lane = threadIdx.x & 63;
     const int NW = static_cast<int>(gridDim.x) * (kT / kWave);
@@ -81,9 +77,7 @@ __global__ __launch_bounds__(kT) void k_gemv_q4mat(const uint8_t* __restrict__ P
         const int64_t row0 = static_cast<int64_t>(r) * K;
         const BufRsrc rp = make_rsrc(P + row0 / 2, K / 2);
         const BufRsrc rs = make_rsrc(S + row0 / 32, static_cast<int64_t>(NG) * 4);
-        float acc[M];
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[m] = 0.0f;
+        float acc = 0.0f;
         // Two groups per lane in flight: both loads issued before either is used.
         for (int g0 = 0; g0 < NG; g0 += 128) {
             u32x4 q[2];
@@ -99,51 +93,31 @@ __global__ __launch_bounds__(kT) void k_gemv_q4mat(const uint8_t* __restrict__ P
             for (int u = 0; u < 2; ++u) {
                 const int g = g0 + 64 * u + lane;
                 const int gg = g < NG ? g : 0;
+                float dc[4];
 #pragma unroll
-                for (int m = 0; m < M; ++m) {
-                    const f32x4* xm = xs + m * nx4;
-                    float dc[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        // dword c: bytes 4c..4c+3 = values 8c..8c+7 (low nibble even)
-                        const uint32_t v = q[u][c] ^ 0x88888888u;
-                        const uint32_t lo = v & 0x0f0f0f0fu, hi = (v >> 4) & 0x0f0f0f0fu;
-                        const f32x4 a = xm[(2 * c) * NG + gg], b = xm[(2 * c + 1) * NG + gg];
-                        float t = ubyte_f32(lo, 0) * a[0];
-                        t = __builtin_fmaf(ubyte_f32(hi, 0), a[1], t);
-                        t = __builtin_fmaf(ubyte_f32(lo, 1), a[2], t);
-                        t = __builtin_fmaf(ubyte_f32(hi, 1), a[3], t);
-                        t = __builtin_fmaf(ubyte_f32(lo, 2), b[0], t);
-                        t = __builtin_fmaf(ubyte_f32(hi, 2), b[1], t);
-                        t = __builtin_fmaf(ubyte_f32(lo, 3), b[2], t);
-                        t = __builtin_fmaf(ubyte_f32(hi, 3), b[3], t);
-                        dc[c] = t;
-                    }
-                    const float dot = (dc[0] + dc[1]) + (dc[2] + dc[3]);
-                    const float blk = sc[u] * __builtin_fmaf(-8.0f, sums[m * NG + gg], dot);
-                    acc[m] += g < NG ? blk : 0.0f;
+                for (int c = 0; c < 4; ++c) {
+                    // dword c: bytes 4c..4c+3 = values 8c..8c+7 (low nibble even)
+                    const uint32_t v = q[u][c] ^ 0x88888888u;
+                    const uint32_t lo = v & 0x0f0f0f0fu, hi = (v >> 4) & 0x0f0f0f0fu;
+                    const f32x4 a = xs[(2 * c) * NG + gg], b = xs[(2 * c + 1) * NG + gg];
+                    float t = ubyte_f32(lo, 0) * a[0];
+                    t = __builtin_fmaf(ubyte_f32(hi, 0), a[1], t);
+                    t = __builtin_fmaf(ubyte_f32(lo, 1), a[2], t);
+                    t = __builtin_fmaf(ubyte_f32(hi, 1), a[3], t);
+                    t = __builtin_fmaf(ubyte_f32(lo, 2), b[0], t);
+                    t = __builtin_fmaf(ubyte_f32(hi, 2), b[1], t);
+                    t = __builtin_fmaf(ubyte_f32(lo, 3), b[2], t);
+                    t = __builtin_fmaf(ubyte_f32(hi, 3), b[3], t);
+                    dc[c] = t;
                 }
+                const float dot = (dc[0] + dc[1]) + (dc[2] + dc[3]);
+                const float blk = sc[u] * __builtin_fmaf(-8.0f, sums[gg], dot);
+                acc += g < NG ? blk : 0.0f;
             }
         }
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const float v = bf16_gemv::wave_sum(acc[m], lane);
-            if (lane == m) Y[static_cast<int64_t>(m) * N + r] = v;
-        }
+        const float v = bf16_gemv::wave_sum(acc, lane);
+        if (lane == 0) Y[r] = v;
     }
-}
-
-template <int M>
-hipError_t run_gemv(const uint8_t* p, const float* sc, const float* x, float* y, int64_t n, int64_t k, hipStream_t s) {
-    const size_t lds = q4mat_gemv_lds_bytes(k);
-    const int64_t waves = kT / kWave;
-    const int64_t cus = device_info().cus;
-    int64_t wgs = (n + waves - 1) / waves;
-    const int64_t cap = 8 * cus;  // grid-stride beyond eight workgroups per CU
-    wgs = wgs > cap ? cap : wgs;
-    hipLaunchKernelGGL(k_gemv_q4mat<M>, dim3(static_cast<unsigned>(wgs)), dim3(kT), lds, s, p, sc, x, y,
-                       static_cast<int>(n), static_cast<int>(k));
-    return hipGetLastError();
 }
 
 // ---- dequantization --------------------------------------------------------
@@ -228,7 +202,13 @@ size_t q4mat_gemv_lds_bytes(int64_t k) { return static_cast<size_t>(k) * 4 + sta
 
 hipError_t launch_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_t k, hipStream_t s) {
     const auto* p = static_cast<const uint8_t*>(w);
-    return run_gemv<1>(p, reinterpret_cast<const float*>(p + q4mat_scales_offset(n, k)), x, y, n, k, s);
+    const auto* sc = reinterpret_cast<const float*>(p + q4mat_scales_offset(n, k));
+    const int64_t waves = kT / kWave, cap = 8 * static_cast<int64_t>(device_info().cus);
+    int64_t wgs = (n + waves - 1) / waves;
+    wgs = wgs > cap ? cap : wgs;  // grid-stride beyond eight workgroups per CU
+    hipLaunchKernelGGL(k_gemv_q4mat, dim3(static_cast<unsigned>(wgs)), dim3(kT), q4mat_gemv_lds_bytes(k), s, p, sc, x, y,
+                       static_cast<int>(n), static_cast<int>(k));
+    return hipGetLastError();
 }
 
 hipError_t launch_dequant_4bit(int fmt, const void* w, void* out, bool bf16, int64_t n, int64_t k, hipStream_t s) {

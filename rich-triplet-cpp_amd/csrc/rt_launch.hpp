@@ -135,7 +135,7 @@ hipError_t launch_gemv_q4k_bf16_fused(int count, const void* const* w, float* co
 size_t bf16_m1_lds_bytes(int64_t k);
 hipError_t launch_gemv_bf16_m1(const uint16_t* w, const float* x, float* y, int64_t n, int64_t k,
                                uint64_t* key, hipStream_t s);
-// Batched GEMV, m <= 8, Q4_K or Q4_0 (K % 256 == 0), Q4Mat (K % 32 == 0) or
+// Batched GEMV, 2 <= m <= 8, Q4_K or Q4_0 (K % 256 == 0), Q4Mat (K % 32 == 0) or
 // BF16 (K % 8 == 0) on the matrix cores (gemv_batch.hip): every weight byte
 // is read once for all m rows.  Long K at several rows is split over
 // workgroups through the library workspace where that has (or may grow to)
