@@ -18,9 +18,9 @@
  * given stream (NULL = the legacy default stream); a status of 0 means the
  * launch was accepted.  Calls on different streams may run concurrently,
  * except calls that use the per-device library workspace -- argmax, GEMM,
- * and GEMV with m > 1 (its K-slice partials and arrival counters): those
- * must not overlap on one device (issue them on one stream, or order the
- * streams).
+ * decode and FLUX attention, and GEMV with m > 1 (its K-slice partials and
+ * arrival counters), of any format and size: those must not overlap on one
+ * device (issue them on one stream, or order the streams).
  *
  * Weight byte formats (verbatim, as the reference holds them in memory):
  *   RT_HIP_Q4K   144-byte GGUF Q4_K super-blocks, K/256 per row
@@ -87,14 +87,23 @@ int rt_hip_init(int ordinal);
 /* ---- workspace ------------------------------------------------------------
  * Some calls take scratch from a per-device library workspace: the GEMM (bf16
  * copies of f32 A and of a Q4_K weight shared by several M tiles, split-K
- * partials), the batched GEMV (K-slice partials), decode attention (split
- * partials) and argmax (8 bytes per row).  It grows on demand (the reference
+ * partials), the batched GEMV of every format (K-slice partials), decode
+ * attention (split partials), FLUX attention (the states of blocks cut between
+ * workgroups) and argmax (8 bytes per row).  It grows on demand (the reference
  * likewise grows its Metal scratch on demand, src/metal_ops.mm:378-423).  A
  * replaced buffer is kept until the process ends, because a hipGraph that
  * captured a call still writes the buffer that call used on every replay.
- * Growth allocates, so it is refused while the stream is being captured
- * (RT_HIP_E_HIP, "... before capture"): reserve what a graph's calls need
- * first.  The *_workspace_bytes functions give one call's need (-1 for
+ * Growth allocates, so it does not happen while the stream is being captured:
+ * reserve what a graph's calls need first.  Without it
+ *  - the batched GEMV keeps K inside its workgroups (short outputs of long K
+ *    take several times as long), FLUX attention keeps its blocks whole (a
+ *    partly empty last round), and a GEMM with K % 256 != 0 runs a kernel
+ *    without a pipeline (up to 3 times as long; Q4_0 and Q4Mat weights need
+ *    room for their bf16 copy all the same): slower, the same to rounding;
+ *  - everything else is refused (RT_HIP_E_HIP, "... before capture"), among it
+ *    a GEMM with K % 256 == 0, for most of whose formats no such kernel exists.
+ * The same holds where the memory cannot be allocated.
+ * The *_workspace_bytes functions give one call's need (-1 for
  * invalid sizes); rt_hip_workspace_bytes the current size of the current
  * device's workspace.  Calls that share the workspace must not overlap on a
  * device (one stream, or ordered streams). */
@@ -302,7 +311,9 @@ int rt_hip_attention_decode_noalloc(const float* q, const float* k_cache, const 
  * overlap q, k or v.  Products and sums to f32 accuracy (each f32 factor as
  * three bf16 values that add up to it, on the matrix cores; online softmax
  * over tiles of 32 keys): results match the reference to f32 rounding and
- * are deterministic.  With more 256-query blocks (n_heads * ceil(t / 256))
+ * are deterministic.  Infinities, NaN and values past 2^64 in k, 2^48 in v or
+ * 2^55 in q behave as in f32 arithmetic, and the query blocks that meet one go
+ * on in f32 matrix steps, at 1.7 to 2.4 times the cost.  With more 256-query blocks (n_heads * ceil(t / 256))
  * than CUs, the work is divided evenly over one workgroup per CU and the
  * blocks cut between two of them keep their partial states in the library
  * workspace (see above): rt_hip_flux_attention_workspace_bytes gives the need
@@ -345,10 +356,11 @@ int rt_hip_gemv_bf16(const uint16_t* w, const float* x, float* y, int64_t n, int
  * all M rows.  Replace: Q4Mat::matmul_q4_t / matmul_q4_t_blas for small M
  * (src/quant_q4.cpp:92-156) and metal_matmul_q4_t (metal_ops.hpp:54-55,
  * src/metal_ops.mm:117-161, 578-619).  w = s(nibble) * scale, summed in f32
- * (factorized: agreement to f32 rounding, normwise 1e-5).  K % 32 == 0 and
- * K up to what one workgroup's LDS holds for one row of x and its group
- * sums (4.125 bytes per value: K up to about 39 700 in gfx950's 160 KB);
- * larger M is split into launches that fit.
+ * (factorized: agreement to f32 rounding, normwise 1e-5); with m > 1 x enters
+ * as integers within 2^-30 of each 32-value block's largest value, whose sums
+ * over a block are exact.  K % 32 == 0 and K up to what one workgroup's LDS
+ * holds for one row of x and its group sums (4.125 bytes per value: K up to
+ * about 39 700 in gfx950's 160 KB), at every m.
  * rt_hip_q4mat_bytes / _scales_offset: the buffer size and where the
  * scales start (-1 for invalid n, k). */
 int64_t rt_hip_q4mat_bytes(int64_t n, int64_t k);
@@ -359,7 +371,7 @@ int rt_hip_gemv_q4mat(const void* w, const float* x, float* y, int64_t n, int64_
 /* GGUF Q4_0 weights streamed as 18-byte blocks.
  * Replace: Q4Mat::matmul_q4_t on GgufFile::decode_q4_0_to_q4mat output
  * (src/quant_q4.cpp:92-114, src/gguf.cpp:392-450) and metal_matmul_q4_t
- * (metal_ops.hpp:54-55).  Requires K % 256 == 0. */
+ * (metal_ops.hpp:54-55).  Requires K % 256 == 0.  (m > 1: x as for Q4Mat.) */
 int rt_hip_gemv_q4_0(const void* blocks, const float* x, float* y, int64_t n, int64_t k,
                      int32_t m, rt_hip_stream stream);
 

@@ -1010,8 +1010,8 @@ int rt_hip_linear_forward(int32_t format, const void* w, const float* bias, cons
     if (m <= RT_HIP_GEMV_MAX_M) {
         // The bias in the GEMV's own launch where its kernel adds it (Q4_K
         // 3072 x 3072, one row, called eagerly: 10.4 us against 13.3 with a
-        // second launch); one that overlaps y is read after the products are
-        // stored.
+        // second launch; the one-row kernels of the other formats have no such
+        // form); one that overlaps y is read after the products are stored.
         const bool fused = bias && (format == RT_HIP_Q4K || m > 1) && !overlaps(y, m * n * 4, bias, n * 4);
         const float* in = fused ? bias : nullptr;
         const auto rows = static_cast<int32_t>(m);
