@@ -487,13 +487,11 @@ __global__ __launch_bounds__(NW * kWave) void k_gemv_batch(const uint8_t* __rest
                     a = f32x4{xa[i][0], xa[i][2], xb[i][0], xb[i][2]};
                     b = f32x4{xa[i][1], xa[i][3], xb[i][1], xb[i][3]};
                 }
-                // Block (step, m) is the quad of units g = 0..3.
-                float amax = fmaxf(fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))),
-                                   fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3]))));
-                // fmaxf passes NaNs over; they are the largest of the bit patterns
-                const bool nan = __builtin_isunordered(a[0], a[1]) | __builtin_isunordered(a[2], a[3]) |
-                                 __builtin_isunordered(b[0], b[1]) | __builtin_isunordered(b[2], b[3]);
-                amax = nan ? __uint_as_float(0x7fc00000u) : amax;
+                // Block (step, m) is the quad of units g = 0..3.  A NaN stays in the
+                // maximum, and is the largest of the bit patterns.
+                auto max2 = [](float p, float q) { return __builtin_elementwise_maximum(p, q); };
+                float amax = max2(max2(max2(fabsf(a[0]), fabsf(a[1])), max2(fabsf(a[2]), fabsf(a[3]))),
+                                  max2(max2(fabsf(b[0]), fabsf(b[1])), max2(fabsf(b[2]), fabsf(b[3]))));
                 amax = __uint_as_float(quad_max(__float_as_uint(amax)));
                 uint32_t wa[4], wb[4];
                 float unit, sum = 0.0f;
