@@ -747,15 +747,17 @@ hipError_t run_xp(const Jobs& jobs, const float* x, const XArgs& xa, int64_t k, 
     // second vector doubles the registers); the rest of a longer x is
     // staged by a loop after them, in the instances that kHasRest names: those
     // of 16 where no x operation runs, whatever the epilogue.
+    // (No call launches the bias form of three and four jobs, nor converter
+    // waves on row-major weights.  Taken out, these instances move the others,
+    // and a layer's kernels, which about fill the instruction cache together,
+    // meet in it: Llama-3.2-3B's engine token 1051 -> 1062 us.)
     constexpr bool kPlain = XOP == kXNone;
-    if constexpr (EPI != kEpiBias) {  // (the bias form has one job)
-        if (jobs.count > 2) {
-            if (per <= 2) return run<D, 2, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-            if (per <= 3) return run<D, 3, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-            if (per <= 4) return run<D, 4, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-            if (per <= 8 || !kPlain) return run<D, 8, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-            if constexpr (kPlain) return run<D, 16, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
-        }
+    if (EPI != kEpiBias && jobs.count > 2) {
+        if (per <= 2) return run<D, 2, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+        if (per <= 3) return run<D, 3, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+        if (per <= 4) return run<D, 4, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+        if (per <= 8 || !kPlain) return run<D, 8, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
+        if constexpr (kPlain) return run<D, 16, TILED, true, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
     }
     if (per <= 2) return run<D, 2, TILED, false, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
     if (per <= 3) return run<D, 3, TILED, false, XOP, EPI, CW>(jobs, x, xa, k, ks, waves, s);
@@ -854,8 +856,7 @@ hipError_t dispatch(const Jobs& jobs, const float* x, int64_t k, hipStream_t s, 
         return jobs.count > 2 ? run<4, 2, TILED, true, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s)
                               : run<4, 2, TILED, false, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s);
     } else {
-        if constexpr (TILED)  // (row-major weights run no converter waves)
-            if (sh.cw == 8) return run_xp<4, TILED, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s);
+        if (sh.cw == 8) return run_xp<4, TILED, XOP, EPI, 8>(jobs, x, xa, k, ks, waves, s);
         if constexpr (XOP != kXNone || EPI != kEpiNone) {
             return run_xp<4, TILED, XOP, EPI>(jobs, x, xa, k, ks, waves, s);
         } else {
