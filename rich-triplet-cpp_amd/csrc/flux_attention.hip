@@ -53,12 +53,13 @@
 // wave, 6144 cycles a SIMD; between them come the softmax and the limb splits,
 // about 440 VALU instructions a wave and tile.  Measured at t = 4352, 24 heads
 // of 128: 2070 us with f32 MFMA (71% of that unit's peak, where 1480 us is the
-// least), 1200-1320 us with limbs: MFMA busy 57% at the 1.76 GHz the power
+// least), 1175-1290 us with limbs: MFMA busy 57% at the 1.76 GHz the power
 // limit leaves (2.2 GHz when half idle), which also sets the spread.  Without
 // the limb staging it would be 1075.
-// t = 1280: 230 -> 154 us; t = 2622, 18 x 88: 753 -> 355; t = 477, 13 x 128:
-// 88 -> 61; t = 466, 9 x 64: 38 -> 33; t = 100, 12 x 64: 12.6 -> 12.1.  The
-// normwise error against float64 at t = 4352 fell from 1.6e-6 to 8.7e-7.
+// t = 1280: 230 -> 160 us; t = 2622, 18 x 88: 750 -> 330; t = 477, 13 x 128:
+// 87 -> 61; t = 466, 9 x 64: 39 -> 33; t = 100, 12 x 64: 13.5 -> 12.8 (t = 33,
+// 4 x 32: 5.9 -> 6.5).  The error against float64 at t = 4352 fell from 1.6e-6
+// to 8.5e-7.
 //  * Of the two waves of a SIMD one is in its products (priority 1) while the
 //    other does its softmax and staging, a barrier between phases: 1250 us;
 //    free-running waves 1410.
